@@ -669,7 +669,11 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
     for (int m = 0; m < 4; ++m)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float v = qr[16 * m + i] * c;
+        // v as rounded to f32: otherwise the compiler forms one of the two uses
+        // of h as f16(q c) in a single rounding and the other from v, and where
+        // v lies halfway between two f16 values hi + lo is off by 2^-11
+        float v = qr[16 * m + i] * c;
+        asm volatile("" : "+v"(v));
         const _Float16 h = (_Float16)v;
         qh[m][i] = h;
         ql[m][i] = (_Float16)(v - (float)h);

@@ -269,3 +269,29 @@ def test_batched_prompt_precision_full_size_360m(oracle_lib):
     rel = float(np.abs(lg - lr).max()) / float(np.abs(lr).max())
     print(f"batched prompt precision 360m: {rel:.2e}", flush=True)
     assert rel <= PREFILL_TOL, rel
+
+
+@gpu
+def test_batched_prompt_every_length_vs_oracle(oracle_lib):
+    """The last-token logits of the prompt's first n tokens for every n in
+    2 .. 200, one layer: every query row of the attention kernel is looked at
+    by itself.  The scaled queries are split into two f16 halves; where one
+    lies halfway between two f16 values (one in 2^13 of them) a high half that
+    is rounded twice leaves the split off by 2^-11 of it, which showed as
+    2e-6 to 1e-5 of the logits' scale in one length of forty.  With both
+    halves from one rounding every length is within PREFILL_TOL."""
+    bundle = build("llama", seed=29, n_layers=1, d_model=384, n_heads=6, n_kv_heads=2, max_seq_len=256)
+    g = mllm.PetitGPT(bundle)
+    g.set_prefill(2)
+    ref = oracle_lib.OracleModel(bundle)
+    ids = [int(v) for v in np.random.default_rng(30).integers(0, bundle.cfg.vocab_size, 200)]
+    ref.forward_prompt(ids[:1])
+    rel = {}
+    for n in range(2, 201):
+        lr = ref.forward_decode(ids[n - 1])
+        lg = g.forwardPrompt(ids[:n])
+        rel[n] = float(np.abs(lg - lr).max()) / float(np.abs(lr).max())
+    g.destroy()
+    ref.close()
+    print(f"every length: worst {max(rel.values()):.2e}", flush=True)
+    assert max(rel.values()) <= PREFILL_TOL, {n: r for n, r in rel.items() if r > PREFILL_TOL}
