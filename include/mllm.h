@@ -164,8 +164,12 @@ typedef struct mllm_model mllm_model;
  * and lm_head are all Q4 group-32, at the fused step's shapes, runs the
  * fused decode step (mllm_decode_kernel_name: "k_flow3", "phase kernels",
  * ...); any other runs the kind-generic step ("generic kernels": a few
- * kernels per layer and token, exec modes 1 and 2 only, prompts token by
- * token). */
+ * kernels per layer and token, exec modes 1 and 2 only).  Its prompts of at
+ * least 3 tokens go through every layer in batches on the bf16 matrix cores,
+ * from a copy of the layer matrices as bf16 planes (2, 4 or 6 bytes per
+ * weight: bf16 and per-row Q8, f16, the others); models with more than 4
+ * query heads per KV head or d_ff not a multiple of 64, and a device without
+ * room for the copy, keep the token steps. */
 int mllm_model_create(const mllm_config *cfg, const void *payload, uint64_t payload_nbytes,
                       const mllm_tensor *tensors, int n_tensors, mllm_model **out);
 /* GpuPetitGPT.destroy (webgpu.js:1284-1297); NULL is accepted. */

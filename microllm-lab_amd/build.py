@@ -37,10 +37,11 @@ CONVERT_LIB = os.path.join(PKG, "convert", "libpgwconvert.so")
 CONVERT_BIN = os.path.join(PKG, "convert", "pgw_convert")
 NAPI_OUT = os.path.join(PKG, "js", "mllm_napi.node")
 
-HIP_SOURCES = ["mllm_ops.hip", "mllm_engine.hip", "mllm_prefill.hip", "mllm_generic.hip"]
+HIP_SOURCES = ["mllm_ops.hip", "mllm_engine.hip", "mllm_prefill.hip", "mllm_generic.hip",
+               "mllm_gprompt.hip"]
 # per-source flags: the prefill kernels consume their matrix-core results in
 # VALU epilogues, so the results go to VGPRs (no AGPR-to-VGPR copies)
-EXTRA_FLAGS = {"mllm_prefill.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("mllm_prefill.hip", "mllm_gprompt.hip")}
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("MLLM_OFFLOAD_ARCH", "gfx950")
 HIP_FLAGS = [

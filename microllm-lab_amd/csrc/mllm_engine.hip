@@ -58,6 +58,7 @@
 #include "mllm_device.h"
 #include "mllm_host.h"
 #include "mllm_generic.h"
+#include "mllm_gprompt.h"
 #include "mllm_prefill.h"
 
 namespace mllm {
@@ -2901,6 +2902,9 @@ struct mllm_model {
   GArgs g{};
   std::vector<GLayer> g_layers, g_layers_base;
   int *d_ids = nullptr;              // a call's token ids
+  // their batched prompts (mllm_gprompt.hip): gp.tc = 0 where there are none
+  GpArgs gp{};
+  std::vector<GpLayer> gp_layer;
   GCursor *h_gcur = nullptr;         // pinned: the cursor a call starts from
   hipGraphExec_t g_graph[2] = {};    // one step without / with the lm_head (exec mode 1)
 };
@@ -3318,6 +3322,78 @@ int get_gmat(mllm_model *M, const std::string &n, int rows, int cols, GMat *out)
   return 0;
 }
 
+// Batched prompts of a kind-generic model: the layer matrices as tiled bf16
+// planes (1 to 3 times 2 bytes per weight) and the work buffers.  Shapes that
+// they do not take, and a device without room for them, leave the prompts to
+// the token steps.
+int generic_prompt_create(mllm_model *M) {
+  const GArgs &A = M->g;
+  GpArgs &P = M->gp;
+  P.arch = A.arch;
+  P.L = A.L;
+  P.D = A.D;
+  P.NH = A.NH;
+  P.NKV = A.NKV;
+  P.FF = A.FF;
+  P.max_seq = A.max_seq;
+  P.kv_fp16 = A.kv_fp16;
+  P.rope_dim = A.rope_dim;
+  P.eps = A.eps;
+  P.attn_scale = A.attn_scale;
+  P.emb = A.lm;
+  P.wpe = A.wpe;
+  P.sf = A.sf;
+  P.rope_cos = A.rope_cos;
+  P.rope_sin = A.rope_sin;
+  P.kv = A.kv;
+  if (!gp_supported(P)) return 0;
+  struct Job {
+    const GMat *src;
+    GpMat *dst;
+    int np;
+  };
+  std::vector<Job> jobs;
+  M->gp_layer.assign(A.L, GpLayer{});
+  for (int i = 0; i < A.L; ++i) {
+    const GLayer &w = M->g_layers[i];
+    GpLayer &f = M->gp_layer[i];
+    f.n1 = w.n1;
+    f.n2 = w.n2;
+    f.qkv_b = w.qkv_b;
+    f.proj_b = w.proj_b;
+    f.fc_b = w.fc_b;
+    f.mproj_b = w.mproj_b;
+    // gate and up rows share a launch, so they have the same planes
+    const int up = std::max(gp_planes(w.w1.kind), w.w3.w ? gp_planes(w.w3.kind) : 1);
+    jobs.push_back({&w.qkv, &f.qkv, gp_planes(w.qkv.kind)});
+    jobs.push_back({&w.proj, &f.proj, gp_planes(w.proj.kind)});
+    jobs.push_back({&w.w1, &f.w1, up});
+    if (w.w3.w) jobs.push_back({&w.w3, &f.w3, up});
+    jobs.push_back({&w.w2, &f.w2, gp_planes(w.w2.kind)});
+  }
+  const int tc = std::min(M->cfg.max_seq_len, 2048);
+  const size_t work = gp_buffer_bytes(P, tc);
+  size_t bytes = work;
+  for (const Job &j : jobs) bytes += gp_tiled_bytes(j.src->rows, j.src->cols, j.np);
+  void *buf = nullptr;
+  if (hipMalloc(&buf, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  M->allocs.push_back(buf);
+  M->device_bytes += bytes;
+  if (int rc = gp_init()) return rc;
+  uint8_t *at = static_cast<uint8_t *>(buf) + work;
+  for (const Job &j : jobs) {
+    if (int rc = gp_tile(*j.src, j.np, at, j.dst, M->stream)) return rc;
+    at += gp_tiled_bytes(j.src->rows, j.src->cols, j.np);
+  }
+  MLLM_HIP(hipStreamSynchronize(M->stream));
+  P.layers = M->gp_layer.data();
+  gp_carve(P, buf, tc);
+  return 0;
+}
+
 // The kind-generic model: its matrices as stored, the f32 vectors, the
 // RoPE tables, the KV cache and one token's work rows.
 int generic_create(mllm_model *M) {
@@ -3409,7 +3485,7 @@ int generic_create(mllm_model *M) {
   M->generic = true;
   M->max_pass = MAXT;
   M->exec_mode = 1;
-  return 0;
+  return generic_prompt_create(M);
 }
 
 }  // namespace
@@ -3997,12 +4073,34 @@ static int g_run(mllm_model *M, const int32_t *ids, int n, int pos0, bool rows, 
   return 0;
 }
 
+// A prompt of a kind-generic model through the batched path, in chunks.
+static int g_prompt(mllm_model *M, const int32_t *ids, int n, float *logits, int32_t *argmax) {
+  if (int rc = g_begin(M, nullptr, 0, 0, 0, 0, 0, 0, -1)) return rc;
+  MLLM_HIP(hipEventRecord(M->ev0, M->stream));
+  const float *row = nullptr;
+  for (int p0 = 0; p0 < n; p0 += M->gp.tc) {
+    const int m = std::min(M->gp.tc, n - p0);
+    if (int rc = gp_layers(M->gp, ids + p0, m, p0, p0 + m == n, &row, M->stream)) return rc;
+  }
+  if (int rc = g_head(M->g, row, M->stream)) return rc;
+  MLLM_HIP(hipEventRecord(M->ev1, M->stream));
+  MLLM_HIP(hipStreamSynchronize(M->stream));
+  MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
+  M->last_tokens = n;
+  if (logits) MLLM_HIP(hipMemcpy(logits, M->d_logits, sizeof(float) * (size_t)M->cfg.vocab_size, hipMemcpyDeviceToHost));
+  if (argmax) MLLM_HIP(hipMemcpy(argmax, M->g.res, sizeof(int32_t), hipMemcpyDeviceToHost));
+  return 0;
+}
+
 extern "C" int mllm_forward_prompt(mllm_model *M, const int32_t *ids, int n, float *logits, int32_t *argmax) {
   MLLM_CHECK(M && ids, "null argument");
   MLLM_CHECK(n > 0 && n <= M->cfg.max_seq_len, "prompt length %d out of range", n);
   if (int rc = check_ids(M, ids, n)) return rc;
   if (M->generic) {
-    if (int rc = g_run(M, ids, n, 0, false, logits, argmax)) return rc;
+    // batched from 3 tokens on: two token steps of the 135M shape take less
+    // than the batch's launches
+    const bool batch = M->gp.tc > 0 && n >= 3 && !M->dbg_on;
+    if (int rc = batch ? g_prompt(M, ids, n, logits, argmax) : g_run(M, ids, n, 0, false, logits, argmax)) return rc;
     M->cache_len = n;
     return 0;
   }

@@ -67,6 +67,10 @@ struct GArgs {
 // returns at once once an EOS has been emitted.
 int g_step(const GArgs &A, bool lm, hipStream_t s);
 
+// The end of a step from the residual row x: the final norm, the lm_head
+// (logits row as in g_step) and the argmax.
+int g_head(const GArgs &A, const float *x, hipStream_t s);
+
 // y[rows] = W . x[cols] (model.gemv for any storage).
 int g_gemv(const GMat &W, const float *x, float *y, hipStream_t s);
 

@@ -34,6 +34,7 @@
 #include "mllm_device.h"
 #include "mllm_generic.h"
 #include "mllm_host.h"
+#include "mllm_kinds.h"
 
 namespace mllm {
 namespace {
@@ -47,53 +48,6 @@ enum { GN_NONE = 0, GN_RMS = 1, GN_LN = 2 };
 // Chained calls stop once an EOS was emitted.
 __device__ __forceinline__ bool stopped(const GCursor *c) {
   return c && *reinterpret_cast<const volatile int *>(&c->done) != 0;
-}
-
-__device__ __forceinline__ float f16_bits(uint32_t h) { return __half2float(__ushort_as_half((unsigned short)h)); }
-__device__ __forceinline__ float bf16_bits(uint32_t h) { return __uint_as_float(h << 16); }
-
-// Columns 8c .. 8c+7 of row r as floats (w) and the chunk's scale (Q8
-// group-32 and Q4: the group's; 1 otherwise -- per-row Q8 scales the row's sum).
-__device__ __forceinline__ float load8(const GMat &W, int r, int c, float (&w)[8]) {
-  const size_t e0 = (size_t)r * W.cols + 8 * (size_t)c;
-  switch (W.kind) {
-  case MLLM_F32: {
-    const float4 *p = reinterpret_cast<const float4 *>(static_cast<const float *>(W.w) + e0);
-    const float4 a = p[0], b = p[1];
-    w[0] = a.x, w[1] = a.y, w[2] = a.z, w[3] = a.w, w[4] = b.x, w[5] = b.y, w[6] = b.z, w[7] = b.w;
-    return 1.f;
-  }
-  case MLLM_F16:
-  case MLLM_BF16: {
-    const uint4 u = *reinterpret_cast<const uint4 *>(static_cast<const uint16_t *>(W.w) + e0);
-    const uint32_t p[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      w[2 * k] = W.kind == MLLM_F16 ? f16_bits(p[k] & 0xffffu) : bf16_bits(p[k] & 0xffffu);
-      w[2 * k + 1] = W.kind == MLLM_F16 ? f16_bits(p[k] >> 16) : bf16_bits(p[k] >> 16);
-    }
-    return 1.f;
-  }
-  case MLLM_Q8:
-  case MLLM_Q8G32: {
-    const uint2 u = *reinterpret_cast<const uint2 *>(static_cast<const int8_t *>(W.w) + e0);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      w[k] = (float)(int8_t)(u.x >> (8 * k));
-      w[4 + k] = (float)(int8_t)(u.y >> (8 * k));
-    }
-    return W.kind == MLLM_Q8G32 ? W.s[(size_t)r * (W.cols >> 5) + (c >> 2)] : 1.f;
-  }
-  default: {  // MLLM_Q4: byte k holds element 2k (low nibble) and 2k + 1, stored as q + 8
-    const uint32_t u = *reinterpret_cast<const uint32_t *>(static_cast<const uint8_t *>(W.w) + e0 / 2);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      w[2 * k] = (float)((int)((u >> (8 * k)) & 15u) - 8);
-      w[2 * k + 1] = (float)((int)((u >> (8 * k + 4)) & 15u) - 8);
-    }
-    return W.s[(size_t)r * (W.cols / W.group) + (8 * c) / W.group];
-  }
-  }
 }
 
 __device__ __forceinline__ float dot8(const GMat &W, int r, int c, const float *xs) {
@@ -457,6 +411,18 @@ int g_gemv(const GMat &W, const float *x, float *y, hipStream_t s) {
   return 0;
 }
 
+int g_head(const GArgs &A, const float *x, hipStream_t s) {
+  GemvArgs f = gemv_args(A.lm, x, A.norm_f, A.eps, nullptr, A.logits, A.cur);
+  f.lm = 1;
+  if (A.arch == 1)
+    launch_gemv<G_STORE, GN_LN>(f, s);
+  else
+    launch_gemv<G_STORE, GN_RMS>(f, s);
+  hipLaunchKernelGGL(k_g_argmax, dim3(1), dim3(GAT), sizeof(int) * (34 + (size_t)A.max_seq), s, A);
+  MLLM_HIP(hipGetLastError());
+  return 0;
+}
+
 int g_step(const GArgs &A, bool lm, hipStream_t s) {
   const bool gpt2 = A.arch == 1;
   const GCursor *cur = A.cur;
@@ -484,15 +450,7 @@ int g_step(const GArgs &A, bool lm, hipStream_t s) {
       launch_gemv<G_RESID, GN_NONE>(gemv_args(w.w2, A.h, nullptr, 0.f, w.mproj_b, A.x, cur), s);
     }
   }
-  if (lm) {
-    GemvArgs f = gemv_args(A.lm, A.x, A.norm_f, A.eps, nullptr, A.logits, cur);
-    f.lm = 1;
-    if (gpt2)
-      launch_gemv<G_STORE, GN_LN>(f, s);
-    else
-      launch_gemv<G_STORE, GN_RMS>(f, s);
-    hipLaunchKernelGGL(k_g_argmax, dim3(1), dim3(GAT), sizeof(int) * (34 + (size_t)A.max_seq), s, A);
-  }
+  if (lm) return g_head(A, A.x, s);
   MLLM_HIP(hipGetLastError());
   return 0;
 }

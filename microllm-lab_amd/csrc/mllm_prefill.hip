@@ -49,6 +49,7 @@
 
 #include "mllm_device.h"
 #include "mllm_host.h"
+#include "mllm_planes.h"
 #include "mllm_prefill.h"
 
 namespace mllm {
@@ -835,6 +836,7 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
       l = l + mrg0[(s - 1) * MSET + 33] * a[s];
     }
     float *out = A.att + (size_t)(T0 + j) * A.D + hq * PF_HD + 4 * hh;
+    uint8_t *opx = A.opx ? A.opx + ((size_t)((T0 >> 5) * (A.D >> 5)) + 2 * hq) * BPX + j * 16 + 8 * hh : nullptr;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       float r[8];
@@ -849,8 +851,22 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
         r[e] = r0 / l;
         r[4 + e] = r1 / l;
       }
-      *reinterpret_cast<float4 *>(out + 8 * g) = make_float4(r[0], r[1], r[2], r[3]);
-      *reinterpret_cast<float4 *>(out + 32 + 8 * g) = make_float4(r[4], r[5], r[6], r[7]);
+      if (opx) {
+        // dimensions 8g + 4hh .. +3 of the head's first and second group of 32
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          uint32_t p0[4], p1[4], p2[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) bf16_split3(r[4 * u + e], p0[e], p1[e], p2[e]);
+          uint8_t *o = opx + u * BPX + (g >> 1) * 1024 + (g & 1) * 512;
+          *reinterpret_cast<uint2 *>(o) = make_uint2(p0[0] | p0[1] << 16, p0[2] | p0[3] << 16);
+          *reinterpret_cast<uint2 *>(o + 2048) = make_uint2(p1[0] | p1[1] << 16, p1[2] | p1[3] << 16);
+          *reinterpret_cast<uint2 *>(o + 4096) = make_uint2(p2[0] | p2[1] << 16, p2[2] | p2[3] << 16);
+        }
+      } else {
+        *reinterpret_cast<float4 *>(out + 8 * g) = make_float4(r[0], r[1], r[2], r[3]);
+        *reinterpret_cast<float4 *>(out + 32 + 8 * g) = make_float4(r[4], r[5], r[6], r[7]);
+      }
     }
   }
 }
@@ -994,6 +1010,16 @@ void pf_carve(PfArgs &A, void *base, int tc) {
   A.px = p;
 }
 
+void pf_attention(const PfArgs &A, int li, int n, int pos0, int tt0, hipStream_t s) {
+  const int nqt = (n + QTL - 1) / QTL, rep = A.NH / A.NKV;
+  if (A.kv_fp16 && rep <= 3)
+    hipLaunchKernelGGL((k_pf_attn<false, 4>), dim3(nqt - tt0, A.NKV), dim3(256 * rep), 0, s, A, li, n, pos0, tt0);
+  else if (A.kv_fp16)
+    hipLaunchKernelGGL((k_pf_attn<false, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
+  else
+    hipLaunchKernelGGL((k_pf_attn<true, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
+}
+
 int pf_layers(const PfArgs &A, const int32_t *ids, int n, int pos0, bool last, hipStream_t s) {
   if (n <= 0) return 0;
   MLLM_CHECK(n <= A.tc && pos0 >= 0 && pos0 + n <= A.max_seq, "prefill chunk of %d tokens at %d out of range", n,
@@ -1003,7 +1029,7 @@ int pf_layers(const PfArgs &A, const int32_t *ids, int n, int pos0, bool last, h
   MLLM_HIP(hipMemcpyAsync(A.ids, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, s));
   const bool gpt2 = A.arch == 1;
   hipLaunchKernelGGL(k_pf_embed, dim3(n), dim3(WG), 0, s, A, n, pos0);
-  const int nqt = (n + QTL - 1) / QTL, rep = A.NH / A.NKV;
+  const int nqt = (n + QTL - 1) / QTL;
   for (int li = 0; li < A.L; ++li) {
     const PfLayer &W = A.layers[li];
     if (gpt2)
@@ -1019,12 +1045,7 @@ int pf_layers(const PfArgs &A, const int32_t *ids, int n, int pos0, bool last, h
     const bool final_layer = li == A.L - 1;
     if (final_layer && !last) break;
     const int tt0 = final_layer ? nqt - 1 : 0, t0 = tt0 * QTL;
-    if (A.kv_fp16 && rep <= 3)
-      hipLaunchKernelGGL((k_pf_attn<false, 4>), dim3(nqt - tt0, A.NKV), dim3(256 * rep), 0, s, A, li, n, pos0, tt0);
-    else if (A.kv_fp16)
-      hipLaunchKernelGGL((k_pf_attn<false, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
-    else
-      hipLaunchKernelGGL((k_pf_attn<true, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
+    pf_attention(A, li, n, pos0, tt0, s);
     launch_quant<NORM_NONE>(A, A.att, A.D, nullptr, t0, n, s);
     PfGemm O = gemm_same(W.proj, n, gpt2 ? W.proj_b : nullptr, A.x, A.D);
     O.tt0 = tt0;

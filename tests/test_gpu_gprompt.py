@@ -1,0 +1,85 @@
+"""Batched prompts of the kind-generic models (mllm_gprompt.hip; forwardPrompt,
+infer.js:553-577) against the oracle, which accumulates in float64: every
+storage at lengths around the 32-token tile, the workgroup order by XCD (a
+tile count that divides by eight), a chunk boundary, partial rotary, four
+query heads per KV head, gate and up rows in different storages.
+
+Bar: the last-token logits, and those of decode steps that read the cache,
+within TOL of the oracle relative to their scale: the GEMMs' operands are
+exact (Q8 group-32 and Q4 weights rounded once to float32), so what is left
+are float32 roundings, 2e-7 to 5e-7 measured, as in the token steps.
+"""
+import numpy as np
+import pytest
+
+import mllm
+from mllm import pgw
+
+gpu = pytest.mark.gpu
+TOL = 2e-6
+TOL_F16KV = 5e-3  # K or V elements may round to neighbouring f16 values
+
+
+def build(arch="llama", seed=1, std=0.02, **kw):
+    model = {k: kw.pop(k) for k in ("kind", "group", "storages", "bias_std") if k in kw}
+    return pgw.parse_pgw(pgw.make_model(pgw.small_config(arch, **kw), seed=seed, std=std, **model))
+
+
+def worst(oracle_lib, bundle, n, kv_fp16=False):
+    g = mllm.PetitGPT(bundle, kv_fp16=kv_fp16)
+    assert g.decodeKernel == "generic kernels"
+    ref = oracle_lib.OracleModel(bundle)
+    ids = [int(v) for v in np.random.default_rng(n).integers(0, bundle.cfg.vocab_size, n + 2)]
+    rows = [(g.forwardPrompt(ids[:n]).copy(), ref.forward_prompt(ids[:n]))]
+    rows += [(g.forwardDecode(t).copy(), ref.forward_decode(t)) for t in ids[n:]]
+    assert g.cacheLen == n + 2
+    g.destroy()
+    ref.close()
+    return max(float(np.abs(a - b).max()) / float(np.abs(b).max()) for a, b in rows)
+
+
+@gpu
+@pytest.mark.parametrize("arch", ["llama", "gpt2"])
+@pytest.mark.parametrize("kind,group", [("f32", 32), ("f16", 32), ("bf16", 32), ("q8", 32), ("q8g32", 32), ("q4", 64),
+                                        ("q4", 8)])
+@pytest.mark.parametrize("n", [3, 32, 33, 100])
+def test_kind_prompt_vs_oracle(oracle_lib, arch, kind, group, n):
+    extra = {"bias_std": 0.02} if arch == "gpt2" else {}
+    bundle = build(arch, seed=41, kind=kind, group=group, d_model=192, n_heads=3, d_ff=320, max_seq_len=160,
+                   n_kv_heads=3 if arch == "gpt2" else 1, **extra)
+    print(f"prompt {arch} {kind}/{group} n={n}", flush=True)
+    assert worst(oracle_lib, bundle, n) <= TOL
+
+
+@gpu
+@pytest.mark.parametrize("n", [255, 256, 300, 512])
+def test_tile_placement_vs_oracle(oracle_lib, n):
+    """8 and 16 tiles (each tile's workgroups on one XCD), 10 (plain order)."""
+    bundle = build(seed=42, kind="bf16", d_model=256, n_heads=4, n_kv_heads=1, max_seq_len=640)
+    print(f"placement n={n}", flush=True)
+    assert worst(oracle_lib, bundle, n) <= TOL
+
+
+@gpu
+@pytest.mark.parametrize("n", [2048, 2049, 2085])
+def test_chunk_boundary_vs_oracle(oracle_lib, n):
+    """More tokens than a chunk holds: the second chunk reads the first's keys."""
+    bundle = build(seed=43, kind="q8", n_layers=1, max_seq_len=2100)
+    print(f"chunk n={n}", flush=True)
+    assert worst(oracle_lib, bundle, n) <= TOL
+
+
+@gpu
+@pytest.mark.parametrize("case", ["partial rotary", "mixed gate/up", "f16 cache", "q4 large d_ff"])
+def test_prompt_options_vs_oracle(oracle_lib, case):
+    print(case, flush=True)
+    if case == "partial rotary":
+        assert worst(oracle_lib, build(seed=44, kind="f16", rope_pct=0.5), 50) <= TOL
+    elif case == "mixed gate/up":
+        for a, b in (("q8", "f32"), ("f16", "bf16"), ("q4", "q8")):
+            st = {"blocks.0.mlp.w1": a, "blocks.0.mlp.w3": b, "blocks.1.attn.qkv": "f16"}
+            assert worst(oracle_lib, build(seed=45, kind="bf16", storages=st), 40) <= TOL
+    elif case == "f16 cache":
+        assert worst(oracle_lib, build(seed=46, kind="f32", n_layers=1), 60, kv_fp16=True) <= TOL_F16KV
+    else:  # Q4 group-32 beyond the fused step's limits
+        assert worst(oracle_lib, build(seed=47, kind="q4", d_ff=4160, n_layers=1), 45) <= TOL
