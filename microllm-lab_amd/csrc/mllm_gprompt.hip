@@ -24,10 +24,18 @@
 // form, so its rows are normalised by a kernel of their own.
 //
 // What bounds it: at a few hundred tokens a launch has fewer wave tiles than
-// the chip has SIMDs, and its time is the latency of its loads.  A wave tile is
-// 64 rows x 32 tokens; a workgroup is 1 to 8 waves that take slices of the
-// columns (added in order through LDS), so that about 1024 waves share the
-// loads of a launch.
+// the chip has SIMDs, and its time is latency: 2.5-3 us until the first
+// operands arrive (they come from HBM or another XCD's L2), as much again for
+// each further round of loads, about 1 us for a cold instruction cache.  So a
+// wave tile is 64 rows x 32 tokens; a workgroup is 1 to 8 waves that take
+// slices of the columns (added in order through LDS), about 1024 waves a
+// launch; a wave loads 5 half-groups (of 16 columns) ahead; what the epilogue
+// reads is loaded first; the XCDs are laid out so that their L2s fetch least.
+// Measured at 200 tokens of the 135M shape in f16, us a launch: QKV 14.0 ->
+// 8.7 (whole groups ahead, read past the slice's end; epilogue loads after the
+// products, eight values a thread), O and down 13.3 -> 11.6, gate/up 14.0 ->
+// 12.3; the prompt 2.27 -> 2.03 ms.  Weights loaded with the non-temporal
+// policy were slower (2.40 ms): other token tiles read them again.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 #include <math.h>
@@ -52,7 +60,6 @@ enum { GP_QKV = 0, GP_RESID = 1, GP_SWIGLU = 2, GP_GELU = 3 };
 constexpr int GPHD = 64;
 constexpr int GPW = 8;               // waves (column slices) of a GEMM workgroup at most
 constexpr int GPT = 32 * 68;         // floats of one slice's tile in LDS: 32 tokens x 64 rows (+ 4)
-constexpr int GPAD = 3;              // groups read past the end of an operand (never used)
 
 struct GpGemm {
   const uint8_t *w0, *w1;   // tiled rows of sub-tile 0 and 1 (32 rows each)
@@ -60,6 +67,8 @@ struct GpGemm {
   int off1;                 // row tile of sub-tile 1 minus that of sub-tile 0
   int rstep;                // row tiles of the matrix per workgroup (2; 1 where w1 is another matrix)
   int ng;                   // groups per row
+  int rtiles, ttiles;       // row tiles of rstep, token tiles
+  int xt, nbx;              // token groups of XCDs; row tiles per XCD
   int n, tt0, li, pos0;     // tokens, first token tile, layer, first position
   const uint8_t *px;        // the input's planes
   uint8_t *po;              // the output's planes, or null
@@ -69,9 +78,10 @@ struct GpGemm {
   int rms;                  // the input is x g: scale by 1 / sqrt(mean x^2 + eps)
 };
 
+// A half (16 columns) of a group: the token tile's planes, two row tiles' planes.
 template <int NP>
 struct GpLd {
-  v8b x[3][2], w[2][NP][2];
+  v8b x[3], w[2][NP];
 };
 
 __device__ __forceinline__ v8b ld_op(const uint8_t *p) {
@@ -82,78 +92,126 @@ __device__ __forceinline__ v16f mfma(v8b a, v8b b, v16f c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
 }
 
-// One group of one sub-tile: hi += w0 x0, lo += the corrections.
+// One sub-tile: hi += w0 x0, lo += the corrections.
 template <int NP>
-__device__ __forceinline__ void gp_group(const v8b (&x)[3][2], const v8b (&w)[NP][2], v16f &hi, v16f &lo) {
-#pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    hi = mfma(w[0][m], x[0][m], hi);
-    lo = mfma(w[0][m], x[1][m], lo);
-    lo = mfma(w[0][m], x[2][m], lo);
-    if constexpr (NP > 1) {
-      lo = mfma(w[1][m], x[0][m], lo);
-      lo = mfma(w[1][m], x[1][m], lo);
-    }
-    if constexpr (NP > 2) lo = mfma(w[2][m], x[0][m], lo);
+__device__ __forceinline__ void gp_half(const v8b (&x)[3], const v8b (&w)[NP], v16f &hi, v16f &lo) {
+  hi = mfma(w[0], x[0], hi);
+  lo = mfma(w[0], x[1], lo);
+  lo = mfma(w[0], x[2], lo);
+  if constexpr (NP > 1) {
+    lo = mfma(w[1], x[0], lo);
+    lo = mfma(w[1], x[1], lo);
   }
+  if constexpr (NP > 2) lo = mfma(w[2], x[0], lo);
 }
 
-// Dynamic LDS: blockDim / 64 tiles of GPT floats, then 32 floats.
+// What an epilogue item (four rows of one token) reads from memory.  A thread
+// of an eight-slice workgroup has one item and loads it before its operands:
+// loaded after the products it would cost the launch a second memory latency.
+struct GpItem {
+  float4 s0, bias;  // the rows' scales and biases
+  float4 a, b;      // RESID: residual, next gains; QKV: cos, sin; SWIGLU: b = the up rows' scales
+};
+
+__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
+__device__ __forceinline__ float el(const float4 &v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; }
+
+template <int EPI>
+__device__ __forceinline__ GpItem gp_item(const GpArgs &A, const GpGemm &G, int rt, int rd, int t, int c) {
+  GpItem I;
+  const int row = 32 * rt + 4 * c;
+  I.s0 = I.bias = I.a = I.b = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (G.s0) I.s0 = ld4(G.s0 + row);
+  if (EPI == GP_SWIGLU && G.s1) I.b = ld4(G.s1 + row);
+  if (G.bias) I.bias = ld4(G.bias + row);
+  t = min(t, G.n - 1);
+  if (EPI == GP_RESID) {
+    I.a = ld4(A.x + (size_t)t * A.D + row);
+    if (G.gain) I.b = ld4(G.gain + row);
+  }
+  if (EPI == GP_QKV && 4 * c < rd) {
+    const size_t at = (size_t)(G.pos0 + t) * rd;
+    float cs[4], sn[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      cs[e] = A.rope_cos[at + min(4 * c + e, rd - 1)];
+      sn[e] = A.rope_sin[at + min(4 * c + e, rd - 1)];
+    }
+    I.a = make_float4(cs[0], cs[1], cs[2], cs[3]);
+    I.b = make_float4(sn[0], sn[1], sn[2], sn[3]);
+  }
+  return I;
+}
+
+// Dynamic LDS: blockDim / 64 tiles of GPT floats, then 32 norm scales.
 template <int EPI, int NP>
 __global__ __launch_bounds__(64 * GPW) void k_gp_gemm(GpArgs A, GpGemm G) {
   extern __shared__ __attribute__((aligned(16))) float buf[];
   const int KS = blockDim.x >> 6, ks = tid() >> 6, lane = tid() & 63, j = lane & 31, hh = lane >> 5;
-  // the workgroups of one token tile on one XCD, as in mllm_prefill.hip
-  int bx = blockIdx.x, by = blockIdx.y;
-  if (gridDim.y % 8 == 0) {
-    const int b = bx + (int)gridDim.x * by, k = b >> 3;
-    by = (b & 7) + 8 * (k / (int)gridDim.x);
-    bx = k % (int)gridDim.x;
-  }
+  // workgroup b runs on XCD b % 8, each with an L2 of its own: the XCDs are a
+  // grid of G.xt token groups x 8 / G.xt row groups (launch_gemm)
+  const int xr = 8 / G.xt, xcd = blockIdx.x & 7, kb = blockIdx.x >> 3;
+  const int bx = xcd % xr + xr * (kb % G.nbx), by = xcd / xr + G.xt * (kb / G.nbx);
+  if (bx >= G.rtiles || by >= G.ttiles) return;
   const int T0 = (G.tt0 + by) * 32, rt = bx * G.rstep;
-  const int ng = G.ng, gb = ng * ks / KS, ge = ng * (ks + 1) / KS;
+  const int ng = G.ng, hb = 2 * ng * ks / KS, he = 2 * ng * (ks + 1) / KS;  // this wave's halves
   const uint8_t *wa = G.w0 + (size_t)rt * ng * NP * 2048 + 16 * lane;
   const uint8_t *wb = G.w1 + (size_t)(rt + G.off1) * ng * NP * 2048 + 16 * lane;
   const uint8_t *xa = G.px + (size_t)(G.tt0 + by) * ng * BPX + 16 * lane;
-  auto load = [&](int g) {
+  auto load = [&](int h) {
     GpLd<NP> L;
+    const int g = h >> 1, m = h & 1;
 #pragma unroll
-    for (int p = 0; p < 3; ++p)
+    for (int p = 0; p < 3; ++p) L.x[p] = ld_op(xa + (size_t)g * BPX + (2 * p + m) * 1024);
 #pragma unroll
-      for (int m = 0; m < 2; ++m) L.x[p][m] = ld_op(xa + (size_t)g * BPX + (2 * p + m) * 1024);
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-      for (int m = 0; m < 2; ++m) {
-        L.w[0][p][m] = ld_op(wa + ((size_t)g * NP + p) * 2048 + m * 1024);
-        L.w[1][p][m] = ld_op(wb + ((size_t)g * NP + p) * 2048 + m * 1024);
-      }
+    for (int p = 0; p < NP; ++p) {
+      L.w[0][p] = ld_op(wa + ((size_t)g * NP + p) * 2048 + m * 1024);
+      L.w[1][p] = ld_op(wb + ((size_t)g * NP + p) * 2048 + m * 1024);
+    }
     return L;
   };
-  constexpr int RD = NP == 1 ? 3 : 2;  // groups of loads in flight (the registers they take)
-  static_assert(RD <= GPAD, "operands are padded for the read-ahead");
+  // first the epilogue's loads and the residual's sums of squares (eight lanes
+  // a token), then the operands': loads complete in order
+  constexpr int CH = EPI == GP_SWIGLU ? 8 : 16;
+  const int rd = EPI == GP_QKV && A.arch == 0 && (rt >> 1) < A.NH + A.NKV ? A.rope_dim : 0;
+  const GpItem first = gp_item<EPI>(A, G, rt, rd, T0 + (int)tid() / CH, tid() % CH);
+  const int nb = A.D >> 6;
+  float s0 = 0.f, s1 = 0.f;
+  if (G.rms && tid() < 256) {
+    const float *sp = A.ss + (size_t)(T0 + (tid() >> 3)) * nb;
+    const int b = tid() & 7;
+    if (b < nb) s0 = sp[b];
+    if (b + 8 < nb) s1 = sp[b + 8];
+  }
+  constexpr int RD = NP == 1 ? 7 : NP == 2 ? 5 : 4;  // halves of loads in flight: as many as the registers hold
   GpLd<NP> ring[RD];
 #pragma unroll
-  for (int i = 0; i < RD; ++i) ring[i] = load(gb + i);
+  for (int i = 0; i < RD; ++i) ring[i] = load(min(hb + i, he - 1));
   float *rs = buf + KS * GPT;
-  if (G.rms && tid() < 32) {  // the tokens' norm scales
-    const int nb = A.D >> 6;
-    const float *sp = A.ss + (size_t)(T0 + tid()) * nb;
-    float s = 0.f;
-    for (int b = 0; b < nb; ++b) s += sp[b];
-    rs[tid()] = 1.0f / sqrtf(s / (float)A.D + A.eps);
+  if (G.rms) {
+    for (int i = tid(); i < 256; i += blockDim.x) {
+      const float *sp = A.ss + (size_t)(T0 + (i >> 3)) * nb;
+      float s = 0.f;
+      if (i == (int)tid()) {
+        s = s0 + s1;
+        for (int b = (i & 7) + 16; b < nb; b += 8) s += sp[b];
+      } else {
+        for (int b = i & 7; b < nb; b += 8) s += sp[b];
+      }
+      s = sum8f(s);
+      if ((i & 7) == 0) rs[i >> 3] = 1.0f / sqrtf(s / (float)A.D + A.eps);
+    }
   }
   v16f h0, h1, l0, l1;
 #pragma unroll
   for (int v = 0; v < 16; ++v) h0[v] = h1[v] = l0[v] = l1[v] = 0.f;
-  for (int g0 = gb; g0 < ge; g0 += RD)
+  for (int h = hb; h < he; h += RD)
 #pragma unroll
     for (int i = 0; i < RD; ++i) {
-      if (g0 + i >= ge) break;
-      const GpLd<NP> cur = ring[i];
-      ring[i] = load(g0 + i + RD);
-      gp_group<NP>(cur.x, cur.w[0], h0, l0);
-      gp_group<NP>(cur.x, cur.w[1], h1, l1);
+      if (h + i >= he) break;
+      gp_half<NP>(ring[i].x, ring[i].w[0], h0, l0);
+      gp_half<NP>(ring[i].x, ring[i].w[1], h1, l1);
+      if (h + i + RD < he) ring[i] = load(h + i + RD);
     }
   // value v of lane (j, hh): token j, row 8 (v / 4) + 4 hh + v % 4
   float *mine = buf + ks * GPT + j * 68 + 4 * hh;
@@ -168,112 +226,102 @@ __global__ __launch_bounds__(64 * GPW) void k_gp_gemm(GpArgs A, GpGemm G) {
   if (KS > 1) {
     for (int i = tid(); i < 512; i += blockDim.x) {
       float *p = buf + (i >> 4) * 68 + 4 * (i & 15);
-      float4 s = *reinterpret_cast<const float4 *>(p);
-      for (int k = 1; k < KS; ++k) {
-        const float4 o = *reinterpret_cast<const float4 *>(p + k * GPT);
-        s = make_float4(s.x + o.x, s.y + o.y, s.z + o.z, s.w + o.w);
-      }
+      float4 o[GPW];
+#pragma unroll
+      for (int k = 0; k < GPW; ++k) o[k] = *reinterpret_cast<const float4 *>(p + (k < KS ? k : 0) * GPT);
+      float4 s = o[0];
+#pragma unroll
+      for (int k = 1; k < GPW; ++k)
+        if (k < KS) s = make_float4(s.x + o[k].x, s.y + o[k].y, s.z + o[k].z, s.w + o[k].w);
       *reinterpret_cast<float4 *>(p) = s;
     }
     __syncthreads();
   }
-  // epilogue: item = (token jt, rows 8c .. 8c+7 of the tile)
-  constexpr int CH = EPI == GP_SWIGLU ? 4 : 8;
+  // epilogue: item = (token jt, rows 4c .. 4c+3 of the tile).  Four values a
+  // thread keep the code short: a launch runs it once, from a cold
+  // instruction cache.
   for (int it = tid(); it < 32 * CH; it += blockDim.x) {
     const int jt = it / CH, c = it % CH, t = T0 + jt;
     const bool in = t < G.n;
     const float *row = buf + jt * 68;
     const float r = G.rms ? rs[jt] : 1.f;
+    const GpItem I = it == (int)tid() ? first : gp_item<EPI>(A, G, rt, rd, t, c);
+    // output e of the item
+    auto at = [&](int e) {
+      float v = row[4 * c + e] * r;
+      if (G.s0) v *= el(I.s0, e);
+      return G.bias ? v + el(I.bias, e) : v;
+    };
+    float y[4];
     if (EPI == GP_QKV) {
       if (!in) continue;
-      const int head = rt >> 1, pos = G.pos0 + t;
-      const bool is_q = head < A.NH, is_k = !is_q && head < A.NH + A.NKV;
-      const int rd = A.rope_dim, half = rd >> 1;
-      const bool rope = A.arch == 0 && (is_q || is_k);
-      auto at = [&](int d) {
-        const float v = row[d] * r;
-        return G.s0 ? v * G.s0[head * GPHD + d] : v;
-      };
-      float y[8];
+      const int head = rt >> 1, pos = G.pos0 + t, half = rd >> 1;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int d = 8 * c + e;
-        float v = at(d);
-        if (G.bias) v += G.bias[head * GPHD + d];
-        if (rope && d < rd) {
-          const float cs = A.rope_cos[(size_t)pos * rd + d], sn = A.rope_sin[(size_t)pos * rd + d];
-          v = __builtin_fmaf(v, cs, (d < half ? -at(d + half) : at(d - half)) * sn);
+      for (int e = 0; e < 4; ++e) {
+        const int d = 4 * c + e;
+        y[e] = at(e);
+        if (d < rd) {  // rotate-half RoPE on the first rd components (infer.js:208-225)
+          const int m = d < half ? d + half : d - half;
+          float o = row[m] * r;
+          if (G.s0) o *= G.s0[32 * rt + m];
+          y[e] = __builtin_fmaf(y[e], el(I.a, e), (d < half ? -o : o) * el(I.b, e));
         }
-        y[e] = v;
       }
-      if (is_q) {
-        float4 *o = reinterpret_cast<float4 *>(A.q + (size_t)t * A.D + head * GPHD + 8 * c);
-        o[0] = make_float4(y[0], y[1], y[2], y[3]);
-        o[1] = make_float4(y[4], y[5], y[6], y[7]);
+      if (head < A.NH) {
+        *reinterpret_cast<float4 *>(A.q + (size_t)t * A.D + head * GPHD + 4 * c) = make_float4(y[0], y[1], y[2], y[3]);
       } else {
+        const bool is_k = head < A.NH + A.NKV;
         const int kvh = is_k ? head - A.NH : head - A.NH - A.NKV;
-        const size_t k = ((((size_t)G.li * 2 + (is_k ? 0 : 1)) * A.NKV + kvh) * A.max_seq + pos) * GPHD + 8 * c;
+        const size_t k = ((((size_t)G.li * 2 + (is_k ? 0 : 1)) * A.NKV + kvh) * A.max_seq + pos) * GPHD + 4 * c;
         if (A.kv_fp16) {
-          uint32_t w[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            w[e] = (uint32_t)__half_as_ushort(__float2half_rn(y[2 * e])) |
-                   (uint32_t)__half_as_ushort(__float2half_rn(y[2 * e + 1])) << 16;
-          *reinterpret_cast<uint4 *>(reinterpret_cast<__half *>(A.kv) + k) = make_uint4(w[0], w[1], w[2], w[3]);
+          const __half2 a = __floats2half2_rn(y[0], y[1]), b = __floats2half2_rn(y[2], y[3]);
+          *reinterpret_cast<uint2 *>(reinterpret_cast<__half *>(A.kv) + k) =
+              make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));
         } else {
-          float4 *o = reinterpret_cast<float4 *>(reinterpret_cast<float *>(A.kv) + k);
-          o[0] = make_float4(y[0], y[1], y[2], y[3]);
-          o[1] = make_float4(y[4], y[5], y[6], y[7]);
+          *reinterpret_cast<float4 *>(reinterpret_cast<float *>(A.kv) + k) = make_float4(y[0], y[1], y[2], y[3]);
         }
       }
     } else if (EPI == GP_RESID) {
-      const int d0 = 32 * rt + 8 * c;
-      float4 *xp = reinterpret_cast<float4 *>(A.x + (size_t)min(t, G.n - 1) * A.D + d0);
-      const float4 xa4 = xp[0], xb4 = xp[1];
-      float y[8] = {xa4.x, xa4.y, xa4.z, xa4.w, xb4.x, xb4.y, xb4.z, xb4.w}, sq = 0.f;
+      float sq = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float v = row[8 * c + e];
-        if (G.s0) v *= G.s0[d0 + e];
-        if (G.bias) v += G.bias[d0 + e];
-        y[e] += v;
+      for (int e = 0; e < 4; ++e) {
+        y[e] = el(I.a, e) + at(e);
         sq += y[e] * y[e];
       }
-      sq = sum8f(sq);  // the token's 64 columns of this tile
+      sq = row16_sum(sq);  // the token's 64 columns of this tile
       if (!in) continue;
-      xp[0] = make_float4(y[0], y[1], y[2], y[3]);
-      xp[1] = make_float4(y[4], y[5], y[6], y[7]);
+      *reinterpret_cast<float4 *>(A.x + (size_t)t * A.D + 32 * rt + 4 * c) = make_float4(y[0], y[1], y[2], y[3]);
       if (G.gain) {
         if (c == 0) A.ss[(size_t)t * (A.D >> 6) + (rt >> 1)] = sq;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) y[e] *= G.gain[d0 + e];
-        planes_store8(G.po + ((size_t)(T0 >> 5) * G.ldp + rt) * BPX, jt, c, y);
+        for (int e = 0; e < 4; ++e) y[e] *= el(I.b, e);
+        planes_store4(G.po + ((size_t)(T0 >> 5) * G.ldp + rt) * BPX, jt, c, y);
       }
-    } else if (EPI == GP_SWIGLU) {
-      if (!in) continue;
-      const int u0 = 32 * rt + 8 * c;
-      float y[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float a = row[8 * c + e] * r, b = row[32 + 8 * c + e] * r;
-        if (G.s0) a *= G.s0[u0 + e];
-        if (G.s1) b *= G.s1[u0 + e];
-        y[e] = (a / (1.0f + expf(-a))) * b;  // infer.js:175-181
-      }
-      planes_store8(G.po + ((size_t)(T0 >> 5) * G.ldp + rt) * BPX, jt, c, y);
     } else {
       if (!in) continue;
-      const int u0 = 32 * rt + 8 * c;
-      float y[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        float v = row[8 * c + e];
-        if (G.s0) v *= G.s0[u0 + e];
-        if (G.bias) v += G.bias[u0 + e];
-        y[e] = 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));  // infer.js:166-172
+      for (int e = 0; e < 4; ++e) {
+        if (EPI == GP_SWIGLU) {
+          const float a = at(e);
+          float b = row[32 + 4 * c + e] * r;
+          if (G.s1) b *= el(I.b, e);
+          y[e] = (a / (1.0f + expf(-a))) * b;  // infer.js:175-181
+        } else {
+          const float v = at(e);
+          y[e] = 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));  // infer.js:166-172
+        }
       }
-      planes_store8(G.po + ((size_t)(T0 >> 5) * G.ldp + rt) * BPX, jt, c, y);
+      planes_store4(G.po + ((size_t)(T0 >> 5) * G.ldp + rt) * BPX, jt, c, y);
     }
+  }
+}
+
+// Columns 8c .. 8c+7 of a token.
+__device__ __forceinline__ void planes_put8(uint8_t *tile, int j, int c, const float (&v)[8]) {
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const float u[4] = {v[4 * h], v[4 * h + 1], v[4 * h + 2], v[4 * h + 3]};
+    planes_store4(tile, j, 2 * c + h, u);
   }
 }
 
@@ -307,7 +355,7 @@ __global__ __launch_bounds__(WG) void k_gp_embed(GpArgs A, const float *gain, in
       if ((c & 7) == 0) A.ss[(size_t)t * (D >> 6) + (c >> 3)] = sq;
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] *= gain[8 * c + e];
-      planes_store8(A.pxa + (size_t)(t >> 5) * (D >> 5) * BPX, t & 31, c, v);
+      planes_put8(A.pxa + (size_t)(t >> 5) * (D >> 5) * BPX, t & 31, c, v);
     }
   }
 }
@@ -331,7 +379,7 @@ __global__ __launch_bounds__(WG) void k_gp_ln(GpArgs A, const float *g, int t0, 
     float v[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] = (x[8 * c + e] - mean) * r * g[8 * c + e] + g[D + 8 * c + e];
-    planes_store8(A.pxa + (size_t)(t >> 5) * (D >> 5) * BPX, t & 31, c, v);
+    planes_put8(A.pxa + (size_t)(t >> 5) * (D >> 5) * BPX, t & 31, c, v);
   }
 }
 
@@ -345,14 +393,13 @@ __global__ __launch_bounds__(WG) void k_gp_tile(GMat W, int np, uint8_t *dst) {
     const int g = (int)(tg % ng), r = (int)(tg / ng) * 32 + (l & 31);
     float v[8];
     const float sc = load8(W, r, 4 * g + 2 * (l >> 6) + ((l >> 5) & 1), v);
-    uint32_t p[3][8];
+    uint32_t p[4][3];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) bf16_split3(v[e] * sc, p[0][e], p[1][e], p[2][e]);
+    for (int e = 0; e < 4; ++e) bf16_split2(v[2 * e] * sc, v[2 * e + 1] * sc, p[e]);
 #pragma unroll
     for (int k = 0; k < 3; ++k)
       if (k < np)
-        *reinterpret_cast<uint4 *>(dst + (tg * np + k) * 2048 + 16 * l) =
-            make_uint4(p[k][0] | p[k][1] << 16, p[k][2] | p[k][3] << 16, p[k][4] | p[k][5] << 16, p[k][6] | p[k][7] << 16);
+        *reinterpret_cast<uint4 *>(dst + (tg * np + k) * 2048 + 16 * l) = make_uint4(p[0][k], p[1][k], p[2][k], p[3][k]);
   }
 }
 
@@ -368,11 +415,21 @@ size_t gp_lds(int ks) { return sizeof(float) * ((size_t)ks * GPT + 32); }
 
 // Column slices per tile: doubled while the launch has fewer than 1024 waves
 // and every slice keeps two groups.
+// XCDs: with xt token groups and 8 / xt row groups each XCD's L2 fetches a part
+// of the weights and a part of the planes, xt times the weights' bytes plus
+// 8 / xt times the planes' in all; the split that fetches least.
 void launch_gemm(int epi, const GpArgs &A, const GpMat &W, GpGemm G, hipStream_t s) {
-  const int tiles = W.rows / (32 * G.rstep), tt = (G.n + 31) / 32 - G.tt0;
+  G.rtiles = W.rows / (32 * G.rstep);
+  G.ttiles = (G.n + 31) / 32 - G.tt0;
   int ks = 1;
-  while (ks < GPW && tiles * tt * ks < 1024 && G.ng / (2 * ks) >= 2) ks *= 2;
-  hipLaunchKernelGGL(kGpKernels[epi][W.np - 1], dim3(tiles, tt), dim3(64 * ks), gp_lds(ks), s, A, G);
+  while (ks < GPW && G.rtiles * G.ttiles * ks < 1024 && G.ng / (2 * ks) >= 2) ks *= 2;
+  const long wb = (long)G.rtiles * 64 * W.np * 2, xb = (long)G.ttiles * 32 * 6;  // bytes per column
+  G.xt = 1;
+  for (int xt = 2; xt <= 8; xt *= 2)
+    if (xt * wb + 8 / xt * xb < G.xt * wb + 8 / G.xt * xb) G.xt = xt;
+  const int xr = 8 / G.xt, nby = (G.ttiles + G.xt - 1) / G.xt;
+  G.nbx = (G.rtiles + xr - 1) / xr;
+  hipLaunchKernelGGL(kGpKernels[epi][W.np - 1], dim3(8 * G.nbx * nby), dim3(64 * ks), gp_lds(ks), s, A, G);
 }
 
 GpGemm gemm_of(const GpMat &W, int n, int tt0, const uint8_t *px) {
@@ -393,7 +450,7 @@ GpGemm gemm_of(const GpMat &W, int n, int tt0, const uint8_t *px) {
 int gp_planes(int kind) { return kind == MLLM_BF16 || kind == MLLM_Q8 ? 1 : kind == MLLM_F16 ? 2 : 3; }
 
 size_t gp_tiled_bytes(int rows, int cols, int np) {
-  return (size_t)(rows >> 5) * (cols >> 5) * np * 2048 + (size_t)GPAD * np * 2048;
+  return (size_t)(rows >> 5) * (cols >> 5) * np * 2048;
 }
 
 int gp_tile(const GMat &W, int np, void *dst, GpMat *out, hipStream_t s) {
@@ -412,7 +469,7 @@ bool gp_supported(const GpArgs &A) {
 
 namespace {
 size_t al256(size_t b) { return (b + 255) & ~(size_t)255; }
-size_t px_bytes(int tc, int cols) { return al256(((size_t)((tc + 31) / 32) * (cols >> 5) + GPAD) * BPX); }
+size_t px_bytes(int tc, int cols) { return al256((size_t)((tc + 31) / 32) * (cols >> 5) * BPX); }
 }  // namespace
 
 size_t gp_buffer_bytes(const GpArgs &A, int tc) {

@@ -21,33 +21,34 @@ namespace mllm {
 
 constexpr int BPX = 6 * 1024;  // bytes per (32-token tile, group of 32 columns): 3 planes x 2 halves x 64 lanes x 16
 
-// Bits of the nearest bf16 (ties to even); a finite value past bf16's largest
-// is cut instead, so that the planes of a finite value stay finite.
-__device__ __forceinline__ uint32_t bf16_rne(float x) {
-  const uint32_t u = __float_as_uint(x);
-  const uint32_t r = (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-  return (r & 0x7f80u) == 0x7f80u ? u >> 16 : r;
+typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+typedef float v2fl __attribute__((ext_vector_type(2)));
+
+// The planes of two values, packed (the first in the low half).  The first
+// plane is taken from the value cut to bf16's largest, so that a finite value
+// past it keeps finite planes.
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2fl){a, b}, v2bf));  // nearest even
 }
-__device__ __forceinline__ void bf16_split3(float x, uint32_t &p0, uint32_t &p1, uint32_t &p2) {
-  p0 = bf16_rne(x);
-  // an infinity or NaN is all in the first plane
-  const float r1 = (p0 & 0x7f80u) == 0x7f80u ? 0.f : x - __uint_as_float(p0 << 16);
-  p1 = bf16_rne(r1);
-  p2 = bf16_rne(r1 - __uint_as_float(p1 << 16));
+__device__ __forceinline__ void bf16_split2(float a, float b, uint32_t (&p)[3]) {
+  constexpr float M = 3.3895313892515355e38f;
+  p[0] = bf16_pair(__builtin_amdgcn_fmed3f(a, -M, M), __builtin_amdgcn_fmed3f(b, -M, M));
+  a -= __uint_as_float(p[0] << 16);
+  b -= __uint_as_float(p[0] & 0xffff0000u);
+  p[1] = bf16_pair(a, b);
+  a -= __uint_as_float(p[1] << 16);
+  b -= __uint_as_float(p[1] & 0xffff0000u);
+  p[2] = bf16_pair(a, b);
 }
 
-// Columns 8c .. 8c+7 (v) of token j of tile base `tile` (its group 0).
-__device__ __forceinline__ void planes_store8(uint8_t *tile, int j, int c, const float (&v)[8]) {
-  uint32_t p0[8], p1[8], p2[8];
+// Columns 4c .. 4c+3 (v) of token j of a tile (its group 0 at `tile`).
+__device__ __forceinline__ void planes_store4(uint8_t *tile, int j, int c, const float (&v)[4]) {
+  uint32_t a[3], b[3];
+  bf16_split2(v[0], v[1], a);
+  bf16_split2(v[2], v[3], b);
+  uint8_t *o = tile + (size_t)(c >> 3) * BPX + ((c >> 1) & 3) * 512 + j * 16 + (c & 1) * 8;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) bf16_split3(v[e], p0[e], p1[e], p2[e]);
-  uint8_t *o = tile + (size_t)(c >> 2) * BPX + ((c >> 1) & 1) * 1024 + (c & 1) * 512 + j * 16;
-  *reinterpret_cast<uint4 *>(o) =
-      make_uint4(p0[0] | p0[1] << 16, p0[2] | p0[3] << 16, p0[4] | p0[5] << 16, p0[6] | p0[7] << 16);
-  *reinterpret_cast<uint4 *>(o + 2048) =
-      make_uint4(p1[0] | p1[1] << 16, p1[2] | p1[3] << 16, p1[4] | p1[5] << 16, p1[6] | p1[7] << 16);
-  *reinterpret_cast<uint4 *>(o + 4096) =
-      make_uint4(p2[0] | p2[1] << 16, p2[2] | p2[3] << 16, p2[4] | p2[5] << 16, p2[6] | p2[7] << 16);
+  for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2 *>(o + 2048 * p) = make_uint2(a[p], b[p]);
 }
 
 }  // namespace mllm

@@ -638,7 +638,7 @@ constexpr int SCH = 4;   // staged 8-value chunks per thread and super-block (32
 // others one); NSET = 4 with rep 3 puts three waves on every SIMD and takes
 // twice the keys per staging round.  (NSET = 4 needs rep <= 3 and the f16
 // cache: 4 rep waves of an f32 cache's registers would not fit.)
-template <bool SPLIT_KV, int NSET>
+template <bool SPLIT_KV, int NSET, bool OPX>
 __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int li, int n, int pos0, int tt0) {
   constexpr int KSB = 32 * NSET;    // keys per super-block
   constexpr int VROW = KSB + 4;     // halves per staged value column (KSB keys + pad)
@@ -674,7 +674,7 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
         // of h as f16(q c) in a single rounding and the other from v, and where
         // v lies halfway between two f16 values hi + lo is off by 2^-11
         float v = qr[16 * m + i] * c;
-        asm volatile("" : "+v"(v));
+        asm("" : "+v"(v));
         const _Float16 h = (_Float16)v;
         qh[m][i] = h;
         ql[m][i] = (_Float16)(v - (float)h);
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
       l = l + mrg0[(s - 1) * MSET + 33] * a[s];
     }
     float *out = A.att + (size_t)(T0 + j) * A.D + hq * PF_HD + 4 * hh;
-    uint8_t *opx = A.opx ? A.opx + ((size_t)((T0 >> 5) * (A.D >> 5)) + 2 * hq) * BPX + j * 16 + 8 * hh : nullptr;
+    uint8_t *opx = OPX ? A.opx + ((size_t)(T0 >> 5) * (A.D >> 5) + 2 * hq) * BPX : nullptr;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       float r[8];
@@ -851,18 +851,11 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
         r[e] = r0 / l;
         r[4 + e] = r1 / l;
       }
-      if (opx) {
+      if (OPX) {
         // dimensions 8g + 4hh .. +3 of the head's first and second group of 32
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          uint32_t p0[4], p1[4], p2[4];
-#pragma unroll
-          for (int e = 0; e < 4; ++e) bf16_split3(r[4 * u + e], p0[e], p1[e], p2[e]);
-          uint8_t *o = opx + u * BPX + (g >> 1) * 1024 + (g & 1) * 512;
-          *reinterpret_cast<uint2 *>(o) = make_uint2(p0[0] | p0[1] << 16, p0[2] | p0[3] << 16);
-          *reinterpret_cast<uint2 *>(o + 2048) = make_uint2(p1[0] | p1[1] << 16, p1[2] | p1[3] << 16);
-          *reinterpret_cast<uint2 *>(o + 4096) = make_uint2(p2[0] | p2[1] << 16, p2[2] | p2[3] << 16);
-        }
+        const float u0[4] = {r[0], r[1], r[2], r[3]}, u1[4] = {r[4], r[5], r[6], r[7]};
+        planes_store4(opx, j, 2 * g + hh, u0);
+        planes_store4(opx + BPX, j, 2 * g + hh, u1);
       } else {
         *reinterpret_cast<float4 *>(out + 8 * g) = make_float4(r[0], r[1], r[2], r[3]);
         *reinterpret_cast<float4 *>(out + 32 + 8 * g) = make_float4(r[4], r[5], r[6], r[7]);
@@ -1010,14 +1003,22 @@ void pf_carve(PfArgs &A, void *base, int tc) {
   A.px = p;
 }
 
-void pf_attention(const PfArgs &A, int li, int n, int pos0, int tt0, hipStream_t s) {
+template <bool OPX>
+static void launch_attention(const PfArgs &A, int li, int n, int pos0, int tt0, hipStream_t s) {
   const int nqt = (n + QTL - 1) / QTL, rep = A.NH / A.NKV;
   if (A.kv_fp16 && rep <= 3)
-    hipLaunchKernelGGL((k_pf_attn<false, 4>), dim3(nqt - tt0, A.NKV), dim3(256 * rep), 0, s, A, li, n, pos0, tt0);
+    hipLaunchKernelGGL((k_pf_attn<false, 4, OPX>), dim3(nqt - tt0, A.NKV), dim3(256 * rep), 0, s, A, li, n, pos0, tt0);
   else if (A.kv_fp16)
-    hipLaunchKernelGGL((k_pf_attn<false, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
+    hipLaunchKernelGGL((k_pf_attn<false, 2, OPX>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
   else
-    hipLaunchKernelGGL((k_pf_attn<true, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
+    hipLaunchKernelGGL((k_pf_attn<true, 2, OPX>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
+}
+
+void pf_attention(const PfArgs &A, int li, int n, int pos0, int tt0, hipStream_t s) {
+  if (A.opx)
+    launch_attention<true>(A, li, n, pos0, tt0, s);
+  else
+    launch_attention<false>(A, li, n, pos0, tt0, s);
 }
 
 int pf_layers(const PfArgs &A, const int32_t *ids, int n, int pos0, bool last, hipStream_t s) {
