@@ -283,9 +283,28 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (readlane_f(v, 0) + readlane_f(v, 16)) + (readlane_f(v, 32) + readlane_f(v, 48));
 }
 
+// Sum over lpr (a power of two <= 64) neighbouring lanes; whole lpr-lane
+// segments are active.
+__device__ __forceinline__ float seg_sum(float a, int lpr) {
+  if (lpr > 1) a += dpp_f<0xB1>(a);    // lane ^ 1
+  if (lpr > 2) a += dpp_f<0x4E>(a);    // lane ^ 2
+  if (lpr > 4) a += dpp_f<0x141>(a);   // mirror within 8
+  if (lpr > 8) a += dpp_f<0x140>(a);   // mirror within 16
+  if (lpr > 16) a += __shfl_xor(a, 16);
+  if (lpr > 32) a += __shfl_xor(a, 32);
+  return a;
+}
+
 __device__ __forceinline__ float wave_max(float v) {
   v = row16_max(v);
   return fmaxf(fmaxf(readlane_f(v, 0), readlane_f(v, 16)), fmaxf(readlane_f(v, 32), readlane_f(v, 48)));
+}
+
+// Four floats at any 4-byte boundary (the f32 tensors of a payload).
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 ld4u(const float *p) {
+  const v4f_u v = *reinterpret_cast<const v4f_u *>(p);
+  return make_float4(v.x, v.y, v.z, v.w);
 }
 
 // Pairwise tree over N = 2^k values: (tree(lower half) + tree(upper half)).

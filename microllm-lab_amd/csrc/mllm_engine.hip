@@ -3466,7 +3466,8 @@ int generic_create(mllm_model *M) {
   int rc = dev_alloc(M, &A.kv, kv_bytes);
   if (!rc) rc = dev_alloc(M, (void **)&A.x, sizeof(float) * D);
   if (!rc) rc = dev_alloc(M, (void **)&A.qkv, sizeof(float) * (D + 2 * kvd));
-  if (!rc) rc = dev_alloc(M, (void **)&A.att, sizeof(float) * D);
+  if (!rc)
+    rc = dev_alloc(M, (void **)&A.attp, sizeof(float) * NH * ((c.max_seq_len + kGenericSplit - 1) / kGenericSplit) * kGenericPart);
   if (!rc) rc = dev_alloc(M, (void **)&A.h, sizeof(float) * FF);
   if (!rc) rc = dev_alloc(M, (void **)&M->d_logits, sizeof(float) * MAXT * (size_t)V);
   if (!rc) rc = dev_alloc(M, (void **)&A.res, sizeof(int) * MAXT);

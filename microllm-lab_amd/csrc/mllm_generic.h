@@ -44,6 +44,9 @@ struct GCursor {
   int done, emitted;     // chained calls: an EOS was emitted; ids emitted so far
 };
 
+// Positions per attention workgroup, and the floats of its partial.
+constexpr int kGenericSplit = 256, kGenericPart = 68;
+
 struct GArgs {
   int arch, L, D, NH, NKV, FF, V, max_seq, kv_fp16;
   int rope_dim;          // rotated components per head (llama; infer.js:185-206)
@@ -52,7 +55,8 @@ struct GArgs {
   GMat lm;               // tied lm_head (and the embedding rows)
   const float *norm_f, *wpe, *sf, *rope_cos, *rope_sin;
   void *kv;                  // [L][2][NKV][max_seq][64], f32 or f16 (the engine's cache)
-  float *x, *qkv, *att, *h;  // one token's rows: [D], [D + 2 NKV 64], [D], [FF]
+  float *x, *qkv, *h;        // one token's rows: [D], [D + 2 NKV 64], [FF]
+  float *attp;               // [NH][splits of max_seq][kGenericPart] attention partials
   float *logits;             // [rows][V]
   int *res;                  // argmax per logits row
   GCursor *cur;

@@ -8,16 +8,17 @@
 //   k_g_embed    the token's row of the tied lm_head in its storage
 //                (infer.js:360-420: quantised rows de-scaled by gpt2's
 //                scale_factors) + gpt2's learned position
-//   k_g_gemv     norm (RMSNorm / LayerNorm) of the input row as a prologue,
-//                then one wave per weight row: 8-column chunks of any
-//                storage kind dotted with the staged row, the wave's sum,
-//                and an epilogue: store (+ bias), residual add (+ bias),
-//                SwiGLU over the w1 / w3 rows, or bias + GELU-tanh
-//   k_g_attn     one workgroup per query head: rotate-half RoPE of its q
-//                and of its KV group's new k (infer.js:208-225) in LDS, the
-//                group's first head writes k / v to the KV cache (the
-//                engine's layout); scores over the cache, the softmax of
-//                infer.js:227-238, P.V (infer.js:466-495)
+//   k_g_gemv     a weight row per segment of lanes, its input row -- with
+//                the norm (RMSNorm / LayerNorm) or, for O, the merge of the
+//                attention's splits -- in registers; epilogue: store (+ bias),
+//                residual add (+ bias), SwiGLU over the w1 / w3 rows, or bias
+//                + GELU-tanh
+//   k_g_attn     a workgroup per query head and 256 positions: rotate-half
+//                RoPE of its q and of its KV group's new k (infer.js:208-225);
+//                the group's first head writes k / v to the KV cache (the
+//                engine's layout); scores, softmax statistics
+//                (infer.js:227-238) and P.V (infer.js:466-495) of its
+//                positions
 //   k_g_argmax   first maximum (infer.js:240-250), or argmaxGpt2
 //                (infer.js:252-287) in gpt2 chains
 // These matrices are read once per token, as by the Q4 engine, at the
@@ -43,99 +44,373 @@ constexpr int GHD = 64;   // head dimension
 constexpr int GT = 256;   // threads per workgroup
 constexpr int GAT = 1024;  // threads of the argmax workgroup
 enum { G_STORE = 0, G_RESID = 1, G_SWIGLU = 2, G_GELU = 3 };
-enum { GN_NONE = 0, GN_RMS = 1, GN_LN = 2 };
+enum { GN_NONE = 0, GN_RMS = 1, GN_LN = 2, GN_SPLITS = 3 };
+constexpr int GSPLIT = kGenericSplit;  // positions per attention workgroup
+constexpr int GAW = 8, GAK = GSPLIT / GAW;  // its waves, the positions of each
+constexpr int GAPS = kGenericPart;     // floats of its partial: max, sum, 2 pad, 64 outputs
 
 // Chained calls stop once an EOS was emitted.
 __device__ __forceinline__ bool stopped(const GCursor *c) {
   return c && *reinterpret_cast<const volatile int *>(&c->done) != 0;
 }
 
-__device__ __forceinline__ float dot8(const GMat &W, int r, int c, const float *xs) {
-  float w[8];
-  const float sc = load8(W, r, c, w);
-  const float4 xa = *reinterpret_cast<const float4 *>(xs + 8 * c), xb = *reinterpret_cast<const float4 *>(xs + 8 * c + 4);
-  float d = w[0] * xa.x;
-  d = __builtin_fmaf(w[1], xa.y, d);
-  d = __builtin_fmaf(w[2], xa.z, d);
-  d = __builtin_fmaf(w[3], xa.w, d);
-  d = __builtin_fmaf(w[4], xb.x, d);
-  d = __builtin_fmaf(w[5], xb.y, d);
-  d = __builtin_fmaf(w[6], xb.z, d);
-  d = __builtin_fmaf(w[7], xb.w, d);
-  return d * sc;
+// ---------------------------------------------------------------- GEMV
+// A row of the matrix is on a segment of L lanes (a power of two): lane l
+// takes the 8-column chunks l, l + L, ... (at most CB of them where L = 64
+// allows it), keeps their inputs in registers and dots them in order; a DPP /
+// swizzle tree over the segment ends the row.  L follows from the column count
+// and the storage alone, so a row's bits do not depend on the launch.
+//
+// Every segment reads the whole input row, so the RMS norm's mean square and
+// the LayerNorm's moments are the same tree: no LDS and no barrier, and every
+// load of the kernel -- weights, inputs, gains, what the epilogue needs -- is
+// on its way at once.  These launches are bound by that one latency (a layer's
+// matrices are 0.2 to 3 MB), where the former form (inputs staged in LDS, two
+// to three block reductions, then the weights) paid it two to three times:
+// per-row Q8 at the 135M shape, us a launch, QKV 5.1 -> 4.4, O 5.1 -> 4.0 (it
+// merges the attention's splits, too), gate/up 6.3 -> 4.7, down 5.1 -> 3.8,
+// lm_head 21 -> 12.5.
+constexpr int G_MIXED = -1;  // W and W3 of different storages
+template <int KIND>
+__host__ __device__ constexpr int g_cb() {
+  return KIND == MLLM_F32 || KIND == G_MIXED ? 4 : 8;
+}
+
+// A chunk as loaded and its scale.
+template <int KIND>
+struct Raw {
+  uint32_t d[KIND == MLLM_F32 || KIND == G_MIXED ? 8 : KIND == MLLM_F16 || KIND == MLLM_BF16 ? 4 : KIND == MLLM_Q4 ? 1 : 2];
+  float sc;
+};
+
+template <int KIND>
+__device__ __forceinline__ Raw<KIND> raw_load(const GMat &W, int r, int c) {
+  Raw<KIND> R;
+  R.sc = 1.f;
+  if constexpr (KIND == G_MIXED) {
+    float w[8];
+    R.sc = load8(W, r, c, w);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) R.d[e] = __float_as_uint(w[e]);
+  } else {
+    const size_t e0 = (size_t)r * W.cols + 8 * (size_t)c;
+    const uint8_t *p = static_cast<const uint8_t *>(W.w);
+    if constexpr (KIND == MLLM_F32) {
+      const uint4 a = *reinterpret_cast<const uint4 *>(p + 4 * e0), b = *reinterpret_cast<const uint4 *>(p + 4 * e0 + 16);
+      R.d[0] = a.x, R.d[1] = a.y, R.d[2] = a.z, R.d[3] = a.w, R.d[4] = b.x, R.d[5] = b.y, R.d[6] = b.z, R.d[7] = b.w;
+    } else if constexpr (KIND == MLLM_F16 || KIND == MLLM_BF16) {
+      const uint4 a = *reinterpret_cast<const uint4 *>(p + 2 * e0);
+      R.d[0] = a.x, R.d[1] = a.y, R.d[2] = a.z, R.d[3] = a.w;
+    } else if constexpr (KIND == MLLM_Q4) {
+      R.d[0] = *reinterpret_cast<const uint32_t *>(p + e0 / 2);
+      R.sc = W.s[(size_t)r * (W.cols / W.group) + (8 * c) / W.group];
+    } else {
+      const uint2 a = *reinterpret_cast<const uint2 *>(p + e0);
+      R.d[0] = a.x, R.d[1] = a.y;
+      if (KIND == MLLM_Q8G32) R.sc = W.s[(size_t)r * (W.cols >> 5) + (c >> 2)];
+    }
+  }
+  return R;
+}
+
+template <int KIND>
+__device__ __forceinline__ float raw_at(const Raw<KIND> &R, int e) {
+  if constexpr (KIND == MLLM_F32 || KIND == G_MIXED) return __uint_as_float(R.d[e]);
+  if constexpr (KIND == MLLM_F16) return f16_bits(e & 1 ? R.d[e >> 1] >> 16 : R.d[e >> 1] & 0xffffu);
+  if constexpr (KIND == MLLM_BF16) return __uint_as_float(e & 1 ? R.d[e >> 1] & 0xffff0000u : R.d[e >> 1] << 16);
+  if constexpr (KIND == MLLM_Q4) return (float)((int)((R.d[0] >> (4 * e)) & 15u) - 8);  // byte k: elements 2k, 2k + 1
+  return (float)(int8_t)(R.d[e >> 2] >> (8 * (e & 3)));
+}
+
+template <int KIND>
+__device__ __forceinline__ float raw_dot(const Raw<KIND> &R, const float (&x)[8], float acc) {
+  float d = raw_at<KIND>(R, 0) * x[0];
+#pragma unroll
+  for (int e = 1; e < 8; ++e) d = __builtin_fmaf(raw_at<KIND>(R, e), x[e], d);
+  if constexpr (KIND == MLLM_Q4 || KIND == MLLM_Q8G32 || KIND == G_MIXED) return __builtin_fmaf(d, R.sc, acc);
+  return acc + d;
 }
 
 struct GemvArgs {
   GMat W, W3;          // W3: the up rows of G_SWIGLU
-  const float *x;      // input row [W.cols]
+  const float *x;      // input row [W.cols] (GN_SPLITS: the attention's partials)
   const float *gains;  // norm gains (LayerNorm: gamma || beta) or null
   float eps;           // RMSNorm eps (LayerNorm: 1e-5, infer.js:145)
   const float *bias;   // per output row, or null
   float *y;            // output row [W.rows]; G_RESID adds to it
-  int rpw;             // rows per wave
+  int L;               // lanes per row
+  int rp;              // row groups (64 / L rows) per wave
   const GCursor *cur;
   int lm;              // 1: y is the logits, row cur->i when cur->rows (verify)
+  int nsplit_max;      // GN_SPLITS: partials per head in x
 };
 
-// Dynamic LDS: W.cols + 4 floats.
-template <int EPI, int NORM>
-__global__ __launch_bounds__(GT) void k_g_gemv(GemvArgs a) {
-  extern __shared__ __attribute__((aligned(16))) float xs[];
-  if (stopped(a.cur)) return;
-  const int K = a.W.cols;
-  float *y = a.y + (a.lm && a.cur->rows ? (size_t)a.cur->i * a.W.rows : 0);
-  float *red = xs + K;
-  if (NORM == GN_NONE) {
-    for (int i = tid(); i < K; i += GT) xs[i] = a.x[i];
-  } else {
-    // infer.js:133-164 (sums in a fixed order: per thread, then the block tree)
-    float s1 = 0.f;
-    for (int i = tid(); i < K; i += GT) {
-      const float v = a.x[i];
-      s1 += NORM == GN_RMS ? v * v : v;
-    }
-    s1 = block_sum<GT>(s1, red);
-    if (NORM == GN_RMS) {
-      const float r = 1.0f / sqrtf(s1 / (float)K + a.eps);
-      for (int i = tid(); i < K; i += GT) xs[i] = a.x[i] * r * a.gains[i];
-    } else {
-      const float mean = s1 / (float)K;
-      float s2 = 0.f;
-      for (int i = tid(); i < K; i += GT) {
-        const float d = a.x[i] - mean;
-        s2 += d * d;
+// The attention's output row from its splits' partials (infer.js:466-495) into
+// LDS: a thread per four components, its splits' loads four at a time.
+__device__ __forceinline__ void merge_splits(const GemvArgs &a, int ns, float *sx) {
+  for (int i = tid(); i < (a.W.cols >> 2); i += GT) {
+    const float *p = a.x + (size_t)(i >> 4) * a.nsplit_max * GAPS;
+    float mx = -INFINITY, l = 0.f;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int s0 = 0; s0 < ns; s0 += 4) {
+      float m[4], ls[4];
+      float4 u[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float *q = p + min(s0 + k, ns - 1) * GAPS;
+        const float2 ml = *reinterpret_cast<const float2 *>(q);
+        m[k] = s0 + k < ns ? ml.x : -INFINITY;
+        ls[k] = ml.y;
+        u[k] = *reinterpret_cast<const float4 *>(q + 4 + 4 * (i & 15));
       }
-      s2 = block_sum<GT>(s2, red);
-      const float r = 1.0f / sqrtf(s2 / (float)K + 1e-5f);
-      for (int i = tid(); i < K; i += GT) xs[i] = (a.x[i] - mean) * r * a.gains[i] + a.gains[K + i];
+      const float mn = fmaxf(mx, fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
+      const float f0 = expf(mx - mn);  // 0 at first
+      l *= f0, o.x *= f0, o.y *= f0, o.z *= f0, o.w *= f0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float f = expf(m[k] - mn);
+        l = __builtin_fmaf(ls[k], f, l);
+        o.x = __builtin_fmaf(u[k].x, f, o.x), o.y = __builtin_fmaf(u[k].y, f, o.y);
+        o.z = __builtin_fmaf(u[k].z, f, o.z), o.w = __builtin_fmaf(u[k].w, f, o.w);
+      }
+      mx = mn;
+    }
+    const float inv = 1.0f / l;
+    *reinterpret_cast<float4 *>(sx + 4 * i) = make_float4(o.x * inv, o.y * inv, o.z * inv, o.w * inv);
+  }
+}
+
+__device__ __forceinline__ void vec8(const float *p, int c, float (&v)[8]) {
+  const float4 u0 = ld4u(p + 8 * c), u1 = ld4u(p + 8 * c + 4);
+  v[0] = u0.x, v[1] = u0.y, v[2] = u0.z, v[3] = u0.w, v[4] = u1.x, v[5] = u1.y, v[6] = u1.z, v[7] = u1.w;
+}
+
+__device__ __forceinline__ void in8(const float *x, int c, float (&v)[8]) {  // 16-byte aligned
+  const float4 u0 = *reinterpret_cast<const float4 *>(x + 8 * c), u1 = *reinterpret_cast<const float4 *>(x + 8 * c + 4);
+  v[0] = u0.x, v[1] = u0.y, v[2] = u0.z, v[3] = u0.w, v[4] = u1.x, v[5] = u1.y, v[6] = u1.z, v[7] = u1.w;
+}
+
+// What a row's end reads besides the sums, loaded with the weights.
+struct RowEnd {
+  float s, s3, bias, y;
+};
+template <int EPI>
+__device__ __forceinline__ RowEnd row_end(const GemvArgs &a, const float *y, int r) {
+  RowEnd E{1.f, 1.f, 0.f, 0.f};
+  if (a.W.kind == MLLM_Q8) E.s = a.W.s[r];
+  if (EPI == G_SWIGLU && a.W3.kind == MLLM_Q8) E.s3 = a.W3.s[r];
+  if (EPI != G_SWIGLU && a.bias) E.bias = a.bias[r];
+  if (EPI == G_RESID) E.y = y[r];
+  return E;
+}
+template <int EPI>
+__device__ __forceinline__ float row_out(const GemvArgs &a, const RowEnd &E, float acc, float acc3) {
+  if (a.W.kind == MLLM_Q8) acc *= E.s;
+  if (EPI == G_SWIGLU) {
+    if (a.W3.kind == MLLM_Q8) acc3 *= E.s3;
+    return (acc / (1.0f + expf(-acc))) * acc3;  // infer.js:175-181
+  }
+  if (a.bias) acc += E.bias;
+  if (EPI == G_RESID) return E.y + acc;
+  if (EPI == G_GELU) return 0.5f * acc * (1.0f + tanhf(0.7978845608028654f * (acc + 0.044715f * acc * acc * acc)));  // infer.js:166-172
+  return acc;
+}
+
+// Loads above are issued before what is below: without it the compiler moves
+// the weights' loads under the branches that follow.
+__device__ __forceinline__ void loads_first() { asm volatile("" ::: "memory"); }
+
+// GN_SPLITS: W.cols floats of dynamic LDS.
+template <int KIND, int EPI, int NORM>
+__global__ __launch_bounds__(GT) void k_g_gemv(GemvArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float sx[];
+  constexpr int CB = g_cb<KIND>();
+  const int K = a.W.cols, nc = K >> 3, L = a.L, nch = (nc + L - 1) / L, rows = a.W.rows;
+  const int lane = tid() & 63, l = lane & (L - 1), seg = lane / L, rpw = 64 / L;
+  const int g0 = ((int)blockIdx.x * (GT / 64) + (tid() >> 6)) * a.rp;
+  auto chunk = [&](int k) { return min(l + k * L, nc - 1); };  // past the row: a valid chunk, its input taken as 0
+  auto row_of = [&](int g) { return min(g * rpw + seg, rows - 1); };
+  const GCursor *cur = a.cur;
+  if (nch <= CB) {
+    // every load of the first rows and of the input row, then the rest
+    Raw<KIND> w[CB], w3[EPI == G_SWIGLU ? CB : 1];
+    auto load = [&](int g) {
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) {
+          w[k] = raw_load<KIND>(a.W, row_of(g), chunk(k));
+          if (EPI == G_SWIGLU) w3[k] = raw_load<KIND>(a.W3, row_of(g), chunk(k));
+        }
+    };
+    float x[CB][8], gv[NORM == GN_RMS || NORM == GN_LN ? CB : 1][8], scale = 1.f;
+    if (NORM != GN_SPLITS) {
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) in8(a.x, chunk(k), x[k]);
+    }
+    load(g0);
+    if (NORM == GN_RMS || NORM == GN_LN) {
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) vec8(a.gains, chunk(k), gv[k]);
+    }
+    float *y = a.y;
+    RowEnd E = row_end<EPI>(a, y, row_of(g0));
+    loads_first();
+    if (cur) {
+      if (stopped(cur)) return;
+      if (a.lm && cur->rows) y += (size_t)cur->i * rows;
+    }
+    if (NORM == GN_SPLITS) {
+      merge_splits(a, cur->pos / GSPLIT + 1, sx);
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) in8(sx, chunk(k), x[k]);
+    }
+    if (g0 * rpw >= rows) return;  // uniform in the wave
+    if (NORM == GN_RMS) {
+      float ss = 0.f;
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) {
+          float s = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            s = __builtin_fmaf(x[k][e], x[k][e], s);
+            x[k][e] *= gv[k][e];
+          }
+          ss += l + k * L < nc ? s : 0.f;
+        }
+      scale = 1.0f / sqrtf(seg_sum(ss, L) / (float)K + a.eps);
+    } else if (NORM == GN_LN) {
+      float bv[CB][8], s = 0.f;
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) vec8(a.gains + K, chunk(k), bv[k]);
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) {
+          float t = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t += x[k][e];
+          s += l + k * L < nc ? t : 0.f;
+        }
+      const float mean = seg_sum(s, L) / (float)K;
+      s = 0.f;
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) {
+          float t = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            x[k][e] -= mean;
+            t = __builtin_fmaf(x[k][e], x[k][e], t);
+          }
+          s += l + k * L < nc ? t : 0.f;
+        }
+      const float r = 1.0f / sqrtf(seg_sum(s, L) / (float)K + 1e-5f);
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) x[k][e] = __builtin_fmaf(x[k][e] * r, gv[k][e], bv[k][e]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < CB; ++k)
+      if (k < nch && l + k * L >= nc) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[k][e] = 0.f;
+      }
+    for (int i = 0; i < a.rp; ++i) {
+      const int g = g0 + i;
+      if (g * rpw >= rows) break;
+      float acc = 0.f, acc3 = 0.f;
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k < nch) {
+          acc = raw_dot<KIND>(w[k], x[k], acc);
+          if (EPI == G_SWIGLU) acc3 = raw_dot<KIND>(w3[k], x[k], acc3);
+        }
+      const RowEnd E0 = E;
+      if (i + 1 < a.rp) {  // the next rows' weights while this sum ends
+        load(g + 1);
+        E = row_end<EPI>(a, y, row_of(g + 1));
+      }
+      acc = seg_sum(acc, L) * scale;
+      if (EPI == G_SWIGLU) acc3 = seg_sum(acc3, L) * scale;
+      const int r = g * rpw + seg;
+      const float o = row_out<EPI>(a, E0, acc, acc3);
+      if (l == 0 && r < rows) y[r] = o;
+    }
+    return;
+  }
+  // rows past the registers (L = 64): the moments first, then CB chunks at a time
+  if (cur && stopped(cur)) return;
+  float *y = a.y + (a.lm && cur->rows ? (size_t)cur->i * rows : 0);
+  if (NORM == GN_SPLITS) {
+    merge_splits(a, cur->pos / GSPLIT + 1, sx);
+    __syncthreads();
+  }
+  const float *x = NORM == GN_SPLITS ? sx : a.x;
+  float scale = 1.f, mean = 0.f;
+  if (NORM == GN_RMS || NORM == GN_LN) {
+    float s = 0.f;
+    for (int k = 0; k < nch; ++k) {
+      float v[8], t = 0.f;
+      in8(x, chunk(k), v);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) t = NORM == GN_RMS ? __builtin_fmaf(v[e], v[e], t) : t + v[e];
+      s += l + k * L < nc ? t : 0.f;
+    }
+    s = seg_sum(s, L) / (float)K;
+    if (NORM == GN_RMS) {
+      scale = 1.0f / sqrtf(s + a.eps);
+    } else {
+      mean = s;
+      s = 0.f;
+      for (int k = 0; k < nch; ++k) {
+        float v[8], t = 0.f;
+        in8(x, chunk(k), v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) t = __builtin_fmaf(v[e] - mean, v[e] - mean, t);
+        s += l + k * L < nc ? t : 0.f;
+      }
+      scale = 1.0f / sqrtf(seg_sum(s, L) / (float)K + 1e-5f);
     }
   }
-  __syncthreads();
-  const int lane = tid() & 63, wv = tid() >> 6, nc = K >> 3;
-  const int r0 = (blockIdx.x * (GT / 64) + wv) * a.rpw;
-  for (int k = 0; k < a.rpw; ++k) {
-    const int r = r0 + k;
-    if (r >= a.W.rows) break;  // uniform in the wave
+  for (int i = 0; i < a.rp && (g0 + i) * rpw < rows; ++i) {
+    const int r = row_of(g0 + i);
+    const RowEnd E = row_end<EPI>(a, y, r);
     float acc = 0.f, acc3 = 0.f;
-    for (int c = lane; c < nc; c += 64) {
-      acc += dot8(a.W, r, c, xs);
-      if (EPI == G_SWIGLU) acc3 += dot8(a.W3, r, c, xs);
-    }
-    acc = wave_sum(acc);
-    if (EPI == G_SWIGLU) acc3 = wave_sum(acc3);
-    if (lane != 0) continue;
-    if (a.W.kind == MLLM_Q8) acc *= a.W.s[r];
-    if (EPI == G_SWIGLU && a.W3.kind == MLLM_Q8) acc3 *= a.W3.s[r];
-    if (EPI == G_STORE) {
-      y[r] = a.bias ? acc + a.bias[r] : acc;
-    } else if (EPI == G_RESID) {
-      y[r] = y[r] + (a.bias ? acc + a.bias[r] : acc);
-    } else if (EPI == G_SWIGLU) {
-      y[r] = (acc / (1.0f + expf(-acc))) * acc3;  // infer.js:175-181
-    } else {
-      const float v = a.bias ? acc + a.bias[r] : acc;  // infer.js:166-172
-      y[r] = 0.5f * v * (1.0f + tanhf(0.7978845608028654f * (v + 0.044715f * v * v * v)));
-    }
+    for (int k0 = 0; k0 < nch; k0 += CB)
+#pragma unroll
+      for (int k = 0; k < CB; ++k)
+        if (k0 + k < nch) {
+          const int c = chunk(k0 + k);
+          const Raw<KIND> w = raw_load<KIND>(a.W, r, c);
+          float v[8];
+          in8(x, c, v);
+          if (NORM == GN_RMS || NORM == GN_LN) {
+            float gv[8], bv[8];
+            vec8(a.gains, c, gv);
+            if (NORM == GN_LN) vec8(a.gains + K, c, bv);
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+              v[e] = NORM == GN_LN ? __builtin_fmaf((v[e] - mean) * scale, gv[e], bv[e]) : v[e] * scale * gv[e];
+          }
+          if (l + (k0 + k) * L >= nc) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = 0.f;
+          }
+          acc = raw_dot<KIND>(w, v, acc);
+          if (EPI == G_SWIGLU) acc3 = raw_dot<KIND>(raw_load<KIND>(a.W3, r, c), v, acc3);
+        }
+    acc = seg_sum(acc, L);
+    if (EPI == G_SWIGLU) acc3 = seg_sum(acc3, L);
+    const float o = row_out<EPI>(a, E, acc, acc3);
+    if (l == 0 && (g0 + i) * rpw + seg < rows) y[r] = o;
   }
 }
 
@@ -177,29 +452,6 @@ __global__ __launch_bounds__(GT) void k_g_embed(GArgs A) {
   }
 }
 
-__device__ __forceinline__ void kv_row(const GArgs &A, size_t off, float (&r)[GHD]) {
-  if (A.kv_fp16) {
-    const uint4 *p = reinterpret_cast<const uint4 *>(reinterpret_cast<const __half *>(A.kv) + off);
-#pragma unroll
-    for (int k = 0; k < GHD / 8; ++k) {
-      const uint4 u = p[k];
-      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        r[8 * k + 2 * e] = f16_bits(w[e] & 0xffffu);
-        r[8 * k + 2 * e + 1] = f16_bits(w[e] >> 16);
-      }
-    }
-  } else {
-    const float4 *p = reinterpret_cast<const float4 *>(reinterpret_cast<const float *>(A.kv) + off);
-#pragma unroll
-    for (int k = 0; k < GHD / 4; ++k) {
-      const float4 u = p[k];
-      r[4 * k] = u.x, r[4 * k + 1] = u.y, r[4 * k + 2] = u.z, r[4 * k + 3] = u.w;
-    }
-  }
-}
-
 // One head's rotated component d (rotate-half on the first rope_dim
 // components: out[d] = x[d] cos[d] + rot[d] sin[d], rot = (-x[half .. rd),
 // x[0 .. half))).
@@ -210,76 +462,140 @@ __device__ __forceinline__ float rope_at(const GArgs &A, const float *hd, int d,
   return d < half ? hd[d] * c + (-hd[d + half]) * sn : hd[d] * c + hd[d - half] * sn;
 }
 
-// Dynamic LDS: 3 x 64 (q, the new k and v) + max_seq (weights) + 256 (P.V
-// partials) + 4 floats.  The new position's k and v are used from LDS (as
-// the cache holds them: f16-rounded for an f16 cache), so the heads of a
-// group do not wait for the one that writes them to the cache.
-__global__ __launch_bounds__(GT) void k_g_attn(GArgs A, int li) {
-  extern __shared__ __attribute__((aligned(16))) float sa[];
-  if (stopped(A.cur)) return;
-  const int pos = A.cur->pos, rep = A.NH / A.NKV;
-  const int h = blockIdx.x, kvh = h / rep, n = pos + 1;
-  float *qs = sa, *kn = sa + GHD, *vn = kn + GHD, *p = vn + GHD;
-  float *part = p + ((A.max_seq + 3) & ~3), *red = part + GT;
+// Workgroup (query head h, 256 positions), wave w on 32 of them: 16 lanes hold
+// a cached row (4 components each), so a load instruction of the wave reads
+// four rows, 1 KiB in f32, and all 16 of a wave go out before its first score.
+// Each wave forms its scores, their softmax statistics and P.V by itself; the
+// workgroup's eight are merged in wave order (max, sum of weights, outputs) into
+// attp, and the O GEMV merges the splits while it reads its input.  The
+// former form -- a workgroup per head, a row per thread, then P.V down four
+// position slices -- was bound by one workgroup's load rate: 32.2 us at 700
+// positions of the 135M shape, 7.3 now (8.3 with 64 positions a wave: twice
+// the code, which runs once from a cold instruction cache).
+// The new position's k and v are taken from LDS (as the cache holds them:
+// f16-rounded for an f16 cache), so a group's heads do not wait for the one
+// that writes them to the cache.
+template <bool F16>
+__global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
+  __shared__ __attribute__((aligned(16))) float own[GAW][3 * GHD];  // each wave's q, new k, new v
+  __shared__ float part[GAW][GHD + 2];
+  const int done = A.cur->done, pos = A.cur->pos, rep = A.NH / A.NKV, n = pos + 1;  // one load
+  if (done) return;
+  const int h = blockIdx.x, kvh = h / rep, lane = tid() & 63, wv = tid() >> 6;
+  const int s0 = (int)blockIdx.y * GSPLIT;
+  if (s0 >= n) return;
   const size_t kb = g_kv_index(A, li, 0, kvh, 0), vb = g_kv_index(A, li, 1, kvh, 0);
-  if (tid() < GHD) {
-    const int d = tid();
-    const float *k = A.qkv + A.D + kvh * GHD, *v = A.qkv + A.D + A.NKV * GHD + kvh * GHD;
-    qs[d] = rope_at(A, A.qkv + h * GHD, d, pos);
-    float kr = rope_at(A, k, d, pos), vr = v[d];
-    if (A.kv_fp16) {
-      const __half kh = __float2half_rn(kr), vh = __float2half_rn(vr);
-      kr = __half2float(kh);
-      vr = __half2float(vh);
-      if (h % rep == 0) {
-        reinterpret_cast<__half *>(A.kv)[kb + (size_t)pos * GHD + d] = kh;
-        reinterpret_cast<__half *>(A.kv)[vb + (size_t)pos * GHD + d] = vh;
+  const int k0 = s0 + GAK * wv;  // this wave's positions k0 .. k0 + GAK - 1
+  const bool on = k0 < n;       // uniform in the wave
+  // q, k, v rows of the step, one component per lane (these loads first)
+  float *qs = own[wv], *kn = qs + GHD, *vn = kn + GHD;
+  const float *kq = A.qkv + A.D + kvh * GHD;
+  const float qv = rope_at(A, A.qkv + h * GHD, lane, pos);
+  float kv = rope_at(A, kq, lane, pos), vv = kq[A.NKV * GHD + lane];
+  const int grp = lane >> 4, d4 = 4 * (lane & 15);
+  uint4 kr[GAK / 4], vr[GAK / 4];
+  if (on) {
+#pragma unroll
+    for (int i = 0; i < GAK / 4; ++i) {
+      // rows at and past the new one are not used: a valid row in their place
+      const size_t off = (size_t)max(0, min(k0 + 4 * i + grp, pos - 1)) * GHD + d4;
+      if (F16) {
+        const uint2 a = *reinterpret_cast<const uint2 *>(reinterpret_cast<const __half *>(A.kv) + kb + off);
+        const uint2 b = *reinterpret_cast<const uint2 *>(reinterpret_cast<const __half *>(A.kv) + vb + off);
+        kr[i] = make_uint4(a.x, a.y, 0u, 0u);
+        vr[i] = make_uint4(b.x, b.y, 0u, 0u);
+      } else {
+        kr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(A.kv) + kb + off);
+        vr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(A.kv) + vb + off);
       }
-    } else if (h % rep == 0) {
-      reinterpret_cast<float *>(A.kv)[kb + (size_t)pos * GHD + d] = kr;
-      reinterpret_cast<float *>(A.kv)[vb + (size_t)pos * GHD + d] = vr;
     }
-    kn[d] = kr;
-    vn[d] = vr;
+  }
+  const bool writes = h % rep == 0 && pos >= k0 && pos < k0 + GAK;  // uniform in the wave
+  if (F16) {
+    const __half kh = __float2half_rn(kv), vh = __float2half_rn(vv);
+    kv = __half2float(kh);
+    vv = __half2float(vh);
+    if (writes) {
+      reinterpret_cast<__half *>(A.kv)[kb + (size_t)pos * GHD + lane] = kh;
+      reinterpret_cast<__half *>(A.kv)[vb + (size_t)pos * GHD + lane] = vh;
+    }
+  } else if (writes) {
+    reinterpret_cast<float *>(A.kv)[kb + (size_t)pos * GHD + lane] = kv;
+    reinterpret_cast<float *>(A.kv)[vb + (size_t)pos * GHD + lane] = vv;
+  }
+  qs[lane] = qv;
+  kn[lane] = kv;
+  vn[lane] = vv;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();  // the wave's own rows, read below by its other lanes
+  float m = -INFINITY, sum = 0.f;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+  auto row = [&](const uint4 &u) {
+    if (!F16)
+      return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
+    return make_float4(f16_bits(u.x & 0xffffu), f16_bits(u.x >> 16), f16_bits(u.y & 0xffffu), f16_bits(u.y >> 16));
+  };
+  if (on) {
+    const float4 q = *reinterpret_cast<const float4 *>(qs + d4), kl = *reinterpret_cast<const float4 *>(kn + d4),
+                 vl = *reinterpret_cast<const float4 *>(vn + d4);
+    float sc[GAK / 4];
+#pragma unroll
+    for (int i = 0; i < GAK / 4; ++i) {
+      const int key = k0 + 4 * i + grp;
+      const float4 k = key == pos ? kl : row(kr[i]);
+      const float d = row16_sum(__builtin_fmaf(q.w, k.w, __builtin_fmaf(q.z, k.z, __builtin_fmaf(q.y, k.y, q.x * k.x))));
+      sc[i] = key < n ? d * A.attn_scale : -INFINITY;
+      m = fmaxf(m, sc[i]);
+    }
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));  // finite: position k0 is in
+#pragma unroll
+    for (int i = 0; i < GAK / 4; ++i) {
+      const float p = expf(sc[i] - m);
+      const float4 v = k0 + 4 * i + grp == pos ? vl : row(vr[i]);
+      sum += p;
+      o.x = __builtin_fmaf(p, v.x, o.x);
+      o.y = __builtin_fmaf(p, v.y, o.y);
+      o.z = __builtin_fmaf(p, v.z, o.z);
+      o.w = __builtin_fmaf(p, v.w, o.w);
+    }
+#pragma unroll
+    for (int x = 16; x < 64; x *= 2) {
+      sum += __shfl_xor(sum, x);
+      o.x += __shfl_xor(o.x, x);
+      o.y += __shfl_xor(o.y, x);
+      o.z += __shfl_xor(o.z, x);
+      o.w += __shfl_xor(o.w, x);
+    }
+  }
+  if (lane < 16) {
+    part[wv][d4] = o.x;
+    part[wv][d4 + 1] = o.y;
+    part[wv][d4 + 2] = o.z;
+    part[wv][d4 + 3] = o.w;
+    if (lane == 0) {
+      part[wv][GHD] = m;
+      part[wv][GHD + 1] = sum;
+    }
   }
   __syncthreads();
-  float mx = -INFINITY;
-  for (int j = tid(); j < n; j += GT) {
-    float kr[GHD];
-    if (j == pos) {
+  if (wv != 0) return;
+  float mx = part[0][GHD];  // wave 0 has a position
 #pragma unroll
-      for (int e = 0; e < GHD; ++e) kr[e] = kn[e];
-    } else {
-      kv_row(A, kb + (size_t)j * GHD, kr);
-    }
-    float d = 0.f;
+  for (int w = 1; w < GAW; ++w) mx = fmaxf(mx, part[w][GHD]);
+  float l = 0.f, out = 0.f;
 #pragma unroll
-    for (int e = 0; e < GHD; ++e) d = __builtin_fmaf(qs[e], kr[e], d);
-    d *= A.attn_scale;
-    p[j] = d;
-    mx = fmaxf(mx, d);
+  for (int w = 0; w < GAW; ++w) {
+    const float f = expf(part[w][GHD] - mx);  // 0 for a wave without positions
+    l = __builtin_fmaf(part[w][GHD + 1], f, l);
+    out = __builtin_fmaf(part[w][lane], f, out);
   }
-  mx = block_max<GT>(mx, red);
-  float s = 0.f;
-  for (int j = tid(); j < n; j += GT) {
-    const float e = expf(p[j] - mx);
-    p[j] = e;
-    s += e;
+  float *p = A.attp + ((size_t)h * gridDim.y + blockIdx.y) * GAPS;
+  p[4 + lane] = out;
+  if (lane == 0) {
+    p[0] = mx;
+    p[1] = l;
   }
-  s = block_sum<GT>(s, red);  // (its barriers also order the p[] writes before the reads below)
-  const float inv = 1.0f / s;
-  const int d = tid() & (GHD - 1), sl = tid() / GHD;
-  float o = 0.f;
-  for (int j = sl; j < n; j += GT / GHD) {
-    const size_t off = vb + (size_t)j * GHD + d;
-    const float vv = j == pos ? vn[d]
-                              : (A.kv_fp16 ? __half2float(reinterpret_cast<const __half *>(A.kv)[off])
-                                           : reinterpret_cast<const float *>(A.kv)[off]);
-    o = __builtin_fmaf(p[j] * inv, vv, o);
-  }
-  part[tid()] = o;
-  __syncthreads();
-  if (tid() < GHD) A.att[h * GHD + tid()] = (part[tid()] + part[GHD + tid()]) + (part[2 * GHD + tid()] + part[3 * GHD + tid()]);
 }
 
 // First maximum of the step's logits row (infer.js:240-250: NaN never
@@ -315,8 +631,7 @@ __global__ __launch_bounds__(GAT) void k_g_argmax(GArgs A) {
   const int nban = rule ? *nb : 0, nrec = rule ? *nr : 0;
   float bv = -INFINITY;
   int bi = 0x7fffffff;
-  for (int i = tid(); i < A.V; i += GAT) {
-    float v = lg[i];
+  auto take = [&](float v, int i) {
     if (rule) {
       for (int k = 0; k < nban; ++k)
         if (ban[k] == i) {
@@ -335,7 +650,19 @@ __global__ __launch_bounds__(GAT) void k_g_argmax(GArgs A) {
       bv = v;
       bi = i;
     }
+  };
+  // 32 KiB of loads at a time (one workgroup: its loads in flight bound it;
+  // 49152 logits one by one took 19.4 us, 16 KiB at a time 9.5)
+  int i0 = 0;
+  constexpr int AB = 8;
+  for (; i0 + AB * GAT <= A.V; i0 += AB * GAT) {
+    float v[AB];
+#pragma unroll
+    for (int k = 0; k < AB; ++k) v[k] = lg[i0 + k * GAT + tid()];
+#pragma unroll
+    for (int k = 0; k < AB; ++k) take(v[k], i0 + k * GAT + tid());
   }
+  for (int i = i0 + tid(); i < A.V; i += GAT) take(lg[i], i);
   wave_argmax(bv, bi);
   __shared__ float wv_v[GAT / 64];
   __shared__ int wv_i[GAT / 64];
@@ -361,18 +688,40 @@ __global__ __launch_bounds__(GAT) void k_g_argmax(GArgs A) {
   }
 }
 
-// Rows per wave: about 2048 workgroups for the largest matrices.
-int g_rpw(int rows) { return std::max(1, (rows + 4 * 2048 - 1) / (4 * 2048)); }
+// Lanes per row: the fewest (8 or more, a power of two) that keep a lane's
+// chunks in registers -- g_cb, 6 for a LayerNorm's row in 8-chunk storages,
+// whose gains and shifts are held beside it -- else all 64.
+template <int KIND>
+int g_lanes(int cols, bool ln) {
+  const int nc = cols / 8, cb = ln ? std::min(6, g_cb<KIND>()) : g_cb<KIND>();
+  int L = 8;
+  while (L < 64 && (nc + L - 1) / L > cb) L *= 2;
+  return L;
+}
+
+template <int KIND, int EPI, int NORM>
+void launch_kind(GemvArgs a, hipStream_t s) {
+  a.L = g_lanes<KIND>(a.W.cols, NORM == GN_LN);
+  const int groups = (a.W.rows + 64 / a.L - 1) / (64 / a.L);
+  // one row group per wave up to 4096 waves (the input row is read by each
+  // wave: beyond that they would read more input than weights)
+  a.rp = std::max(1, (groups + 4095) / 4096);
+  const int waves = (groups + a.rp - 1) / a.rp;
+  hipLaunchKernelGGL((k_g_gemv<KIND, EPI, NORM>), dim3((waves + GT / 64 - 1) / (GT / 64)), dim3(GT),
+                     NORM == GN_SPLITS ? sizeof(float) * a.W.cols : 0, s, a);
+}
 
 template <int EPI, int NORM>
-int launch_gemv(const GemvArgs &a, hipStream_t s) {
-  const int rpw = g_rpw(a.W.rows);
-  GemvArgs b = a;
-  b.rpw = rpw;
-  const int grid = (a.W.rows + 4 * rpw - 1) / (4 * rpw);
-  const size_t lds = sizeof(float) * ((size_t)a.W.cols + 4);
-  hipLaunchKernelGGL((k_g_gemv<EPI, NORM>), dim3(grid), dim3(GT), lds, s, b);
-  return 0;
+void launch_gemv(const GemvArgs &a, hipStream_t s) {
+  switch (EPI == G_SWIGLU && a.W3.kind != a.W.kind ? G_MIXED : a.W.kind) {
+  case MLLM_F32: return launch_kind<MLLM_F32, EPI, NORM>(a, s);
+  case MLLM_F16: return launch_kind<MLLM_F16, EPI, NORM>(a, s);
+  case MLLM_BF16: return launch_kind<MLLM_BF16, EPI, NORM>(a, s);
+  case MLLM_Q8: return launch_kind<MLLM_Q8, EPI, NORM>(a, s);
+  case MLLM_Q8G32: return launch_kind<MLLM_Q8G32, EPI, NORM>(a, s);
+  case MLLM_Q4: return launch_kind<MLLM_Q4, EPI, NORM>(a, s);
+  default: return launch_kind<G_MIXED, EPI, NORM>(a, s);
+  }
 }
 
 GemvArgs gemv_args(const GMat &W, const float *x, const float *gains, float eps, const float *bias, float *y,
@@ -427,7 +776,7 @@ int g_step(const GArgs &A, bool lm, hipStream_t s) {
   const bool gpt2 = A.arch == 1;
   const GCursor *cur = A.cur;
   hipLaunchKernelGGL(k_g_embed, dim3(1), dim3(GT), 0, s, A);
-  const size_t att_lds = sizeof(float) * (3 * GHD + ((A.max_seq + 3) & ~3) + GT + 4);
+  const int nsplit = (A.max_seq + GSPLIT - 1) / GSPLIT;
   for (int li = 0; li < A.L; ++li) {
     const GLayer &w = A.layers[li];
     if (!(w.dbg & 1)) {
@@ -436,8 +785,13 @@ int g_step(const GArgs &A, bool lm, hipStream_t s) {
         launch_gemv<G_STORE, GN_LN>(q, s);
       else
         launch_gemv<G_STORE, GN_RMS>(q, s);
-      hipLaunchKernelGGL(k_g_attn, dim3(A.NH), dim3(GT), att_lds, s, A, li);
-      launch_gemv<G_RESID, GN_NONE>(gemv_args(w.proj, A.att, nullptr, 0.f, w.proj_b, A.x, cur), s);
+      if (A.kv_fp16)
+        hipLaunchKernelGGL(k_g_attn<true>, dim3(A.NH, nsplit), dim3(GAW * 64), 0, s, A, li);
+      else
+        hipLaunchKernelGGL(k_g_attn<false>, dim3(A.NH, nsplit), dim3(GAW * 64), 0, s, A, li);
+      GemvArgs o = gemv_args(w.proj, A.attp, nullptr, 0.f, w.proj_b, A.x, cur);
+      o.nsplit_max = nsplit;
+      launch_gemv<G_RESID, GN_SPLITS>(o, s);
     }
     if (!(w.dbg & 2)) {
       if (gpt2) {

@@ -113,7 +113,6 @@ struct GpItem {
   float4 a, b;      // RESID: residual, next gains; QKV: cos, sin; SWIGLU: b = the up rows' scales
 };
 
-__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
 __device__ __forceinline__ float el(const float4 &v, int e) { return e == 0 ? v.x : e == 1 ? v.y : e == 2 ? v.z : v.w; }
 
 template <int EPI>
@@ -121,13 +120,13 @@ __device__ __forceinline__ GpItem gp_item(const GpArgs &A, const GpGemm &G, int 
   GpItem I;
   const int row = 32 * rt + 4 * c;
   I.s0 = I.bias = I.a = I.b = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (G.s0) I.s0 = ld4(G.s0 + row);
-  if (EPI == GP_SWIGLU && G.s1) I.b = ld4(G.s1 + row);
-  if (G.bias) I.bias = ld4(G.bias + row);
+  if (G.s0) I.s0 = ld4u(G.s0 + row);
+  if (EPI == GP_SWIGLU && G.s1) I.b = ld4u(G.s1 + row);
+  if (G.bias) I.bias = ld4u(G.bias + row);
   t = min(t, G.n - 1);
   if (EPI == GP_RESID) {
-    I.a = ld4(A.x + (size_t)t * A.D + row);
-    if (G.gain) I.b = ld4(G.gain + row);
+    I.a = *reinterpret_cast<const float4 *>(A.x + (size_t)t * A.D + row);
+    if (G.gain) I.b = ld4u(G.gain + row);
   }
   if (EPI == GP_QKV && 4 * c < rd) {
     const size_t at = (size_t)(G.pos0 + t) * rd;

@@ -80,18 +80,6 @@ __device__ __forceinline__ void x_pin(float4 (&xv)[GX_BATCH]) {
   for (int i = 0; i < GX_BATCH; ++i) asm volatile("" : "+v"(xv[i].x), "+v"(xv[i].y), "+v"(xv[i].z), "+v"(xv[i].w));
 }
 
-// Sum over lpr (a power of two <= 64) neighbouring lanes; whole lpr-lane
-// segments are active.
-__device__ __forceinline__ float seg_sum(float a, int lpr) {
-  if (lpr > 1) a += dpp_f<0xB1>(a);    // lane ^ 1
-  if (lpr > 2) a += dpp_f<0x4E>(a);    // lane ^ 2
-  if (lpr > 4) a += dpp_f<0x141>(a);   // mirror within 8
-  if (lpr > 8) a += dpp_f<0x140>(a);   // mirror within 16
-  if (lpr > 16) a += __shfl_xor(a, 16);
-  if (lpr > 32) a += __shfl_xor(a, 32);
-  return a;
-}
-
 struct GemvGeom {
   int rows, cols, m;  // matrix shape; tokens
   int rpp, lpr;       // rows per pass; lanes per row sum (power of two <= 64)
