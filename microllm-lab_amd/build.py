@@ -41,7 +41,7 @@ HIP_SOURCES = ["mllm_ops.hip", "mllm_engine.hip", "mllm_prefill.hip", "mllm_gene
                "mllm_gprompt.hip"]
 # per-source flags: the prefill kernels consume their matrix-core results in
 # VALU epilogues, so the results go to VGPRs (no AGPR-to-VGPR copies)
-EXTRA_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("mllm_prefill.hip", "mllm_gprompt.hip")}
+EXTRA_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for f in ("mllm_ops.hip", "mllm_prefill.hip", "mllm_gprompt.hip")}
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = os.environ.get("MLLM_OFFLOAD_ARCH", "gfx950")
 HIP_FLAGS = [

@@ -8,6 +8,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 
@@ -278,6 +279,217 @@ __global__ __launch_bounds__(WGT) void k_gemv_q4_argmax(const uint8_t *__restric
     // every row NaN leaves i at INT_MAX; row 0 NaN wins in any case
     *out = coh_ldi(nan0, 0) || i == 0x7fffffff ? 0 : i;
     __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// ---------------------------------------------------------------- Q4 GEMM on the int8 matrix cores
+// y[t][r] = W x[t] for many tokens, every row with the bits of k_gemv_q4.
+//
+// The GEMV's integers are three signed bytes, xi = 65536 h + 256 m + l
+// (|xi| <= Q6MAX < 2^23), so a group's exact dot is three
+// v_mfma_i32_32x32x32_i8 -- K = 32 is one group -- combined modulo 2^32 by two
+// shift-adds; then the GEMV's own ((float)dot * sx) * w_scale, one add a group,
+// and its order of additions: lane partial l of L sums groups l, l + L, ...,
+// and the segment tree is formed depth first, so one partial per tree level is
+// live instead of L of them.  (A group whose values are all below 2.3e-32, past
+// the GEMV's range, may saturate differently.)
+//
+// Wave: 32 weight rows (lane j of a half: row j) x 32 tokens (value v: token
+// 8 (v / 4) + 4 hh + v % 4).  A workgroup's waves share its 32 tokens, whose
+// planes and scales are staged in LDS for as many lane partials as fit, in
+// operand order: slot, plane: 64 lanes of 16 bytes, lane 32 hh + j the elements
+// 0 2 4 6 1 3 5 7 8 10 12 14 9 11 13 15 of half hh of the token's group (the
+// order in which the packed nibbles come apart).
+//
+// What bounds it: the chain of a workgroup's own steps -- staging in two to
+// five parts, then one wave per SIMD through the groups, six VALU operations
+// per output and group -- until the launch fills the chip (about 1000 tokens).
+// The GEMV kernel, eight tokens a launch, spends 33 operations per output and
+// group: 2560 x 960, 301 tokens 288 us there, 27.8 here; 2048 tokens 2148 and
+// 89.  The weights go through LDS because a wave's own loads touch 64 cache
+// lines per group for 20 bytes of each (35 us that way).
+constexpr int GMS = 20;                    // staged group slots
+constexpr int GMB = 3 * 1024 + 128;        // bytes per slot of the tokens: three planes, 32 scales
+constexpr int GMW = GMS / 4;               // rows' chunks of weights in flight while staging
+constexpr int GMX = 8;                     // float4s of x in flight while staging
+// bytes per slot of the weights: a workgroup's rows, 16 packed bytes and a scale each
+__host__ __device__ constexpr int gemm_wslot(int nw) { return nw * 32 * 20; }
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// Four packed nibbles (one per byte) as signed bytes q - 8.
+__device__ __forceinline__ int nib_s8(uint32_t n) {
+  return (int)((((n & 0x0F0F0F0Fu) | 0x80808080u) - 0x08080808u) ^ 0x80808080u);
+}
+
+// LV: levels of the summation tree at most (L <= 2^LV).
+template <int NW, int LV>
+__global__ __launch_bounds__(NW * 64) void k_gemm_q4(const uint8_t *__restrict__ packed,
+                                                     const float *__restrict__ scale, const float *__restrict__ x,
+                                                     float *__restrict__ y, int t, int m, int n, int L, int K, int lgc,
+                                                     int nrb) {
+  extern __shared__ float4 smem4[];
+  const int LC = 1 << lgc, tot = LC * K;  // lane partials and groups staged at a time
+  uint8_t *sm = reinterpret_cast<uint8_t *>(smem4), *swq = sm + tot * GMB;
+  float *sws = reinterpret_cast<float *>(swq + tot * NW * 32 * 16);
+  const int ng = n >> 5, tile = blockIdx.x / nrb, rb = blockIdx.x - tile * nrb;
+  const int lane = threadIdx.x & 63, j = lane & 31, hh = lane >> 5, wv = threadIdx.x >> 6;
+  const int row0 = rb * NW * 32, row = row0 + wv * 32 + j, T0 = tile * 32;
+  const uint32_t magic = K > 1 ? (uint32_t)(((1ull << 32) + K - 1) / K) : 0u;
+  auto div_k = [&](uint32_t v) { return K > 1 ? (int)__umulhi(v, magic) : (int)v; };  // v / K for small v
+  float a[16], lv[LV][16];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) a[v] = 0.f;
+  const int q = threadIdx.x & 7, odd = q & 1;
+  // a pair of lanes holds elements 0 1 2 3 and 4 5 6 7: the even one writes the
+  // even elements' planes, the odd one the odd ones'
+  for (int l0 = 0; l0 < L; l0 += LC) {
+    // the weights of the staged groups, LC neighbouring groups of a row by
+    // neighbouring lanes, in flight over the tokens' staging
+    // (half of them at a time: the registers beside the tree's)
+    v4i wq[GMW];
+    float ws[GMW];
+    auto w_item = [&](int it, int &slot, int &r) {  // item -> (slot, row of the workgroup), its group
+      const uint32_t idx = threadIdx.x + it * (NW * 64), rk = idx >> lgc;
+      r = div_k(rk);
+      const int k = (int)rk - r * K, c = (int)(idx & (LC - 1));
+      slot = c * K + k;
+      return min(l0 + c + k * L, ng - 1);  // past the end: a valid group, unused
+    };
+    auto w_load = [&](int i0) {
+#pragma unroll
+      for (int u = 0; u < GMW; ++u)
+        if (2 * (i0 + u) < tot) {
+          int slot, r;
+          const int g = w_item(i0 + u, slot, r);
+          const size_t at = (size_t)min(row0 + r, m - 1) * ng + g;
+          wq[u] = *reinterpret_cast<const v4i *>(packed + 16 * at);
+          ws[u] = scale[at];
+        }
+    };
+    auto w_store = [&](int i0) {
+#pragma unroll
+      for (int u = 0; u < GMW; ++u)
+        if (2 * (i0 + u) < tot) {
+          int slot, r;
+          w_item(i0 + u, slot, r);
+          if (r < NW * 32) {
+            *reinterpret_cast<v4i *>(swq + (slot * NW * 32 + r) * 16) = wq[u];
+            sws[slot * NW * 32 + r] = ws[u];
+          }
+        }
+    };
+    w_load(0);
+    if (l0) __syncthreads();  // the previous groups are consumed
+    const int tok = (threadIdx.x >> 3) & 31;
+    const float *xt = x + (size_t)min(T0 + tok, t - 1) * n + 4 * q;
+    auto slot_group = [&](int slot) {
+      const int l = div_k((uint32_t)slot);
+      return l0 + l + (slot - l * K) * L;
+    };
+    for (int s0 = threadIdx.x >> 8, turn = 0; s0 < tot; s0 += GMX * NW / 4, ++turn) {
+      if (turn == 1) {  // the second half of the weights in flight over the rest
+        w_store(0);
+        w_load(GMW);
+      }
+      float4 xv[GMX];
+#pragma unroll
+      for (int u = 0; u < GMX; ++u)
+        xv[u] = *reinterpret_cast<const float4 *>(xt + 32 * min(slot_group(min(s0 + u * (NW / 4), tot - 1)), ng - 1));
+#pragma unroll
+      for (int u = 0; u < GMX; ++u) {
+        const int slot = s0 + u * (NW / 4);
+        if (slot >= tot) break;  // uniform in the wave
+        const float4 v = xv[u];
+        const float am = max8(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+        const float inv = q6_inv(am), e[4] = {v.x, v.y, v.z, v.w};
+        // byte p of xi + 0x808080, its top bit flipped, is the signed byte p of xi
+        uint32_t b[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) b[k] = (uint32_t)(min(max((int)__builtin_rintf(e[k] * inv), -8388608), 8355711) + 0x808080);
+        const uint32_t own0 = odd ? b[1] : b[0], own1 = odd ? b[3] : b[2];
+        const uint32_t got0 = (uint32_t)dpp_i<0xB1>((int)(odd ? b[0] : b[1]));
+        const uint32_t got1 = (uint32_t)dpp_i<0xB1>((int)(odd ? b[2] : b[3]));
+        // even lane: own0 own1 got0 got1; odd lane: got0 got1 own0 own1
+        const uint32_t f0 = odd ? got0 : own0, f1 = odd ? got1 : own1, g0 = odd ? own0 : got0, g1 = odd ? own1 : got1;
+        const uint32_t fa = __builtin_amdgcn_perm(f1, f0, 0x05010400u), fc = __builtin_amdgcn_perm(f1, f0, 0x0c0c0602u);
+        const uint32_t ga = __builtin_amdgcn_perm(g1, g0, 0x05010400u), gc = __builtin_amdgcn_perm(g1, g0, 0x0c0c0602u);
+        uint8_t *o = sm + (size_t)slot * GMB + (32 * (q >> 2) + tok) * 16 + 4 * (q & 3);
+        *reinterpret_cast<uint32_t *>(o) = __builtin_amdgcn_perm(gc, fc, 0x05040100u) ^ 0x80808080u;
+        *reinterpret_cast<uint32_t *>(o + 1024) = __builtin_amdgcn_perm(ga, fa, 0x07060302u) ^ 0x80808080u;
+        *reinterpret_cast<uint32_t *>(o + 2048) = __builtin_amdgcn_perm(ga, fa, 0x05040100u) ^ 0x80808080u;
+        if (q == 0) *reinterpret_cast<float *>(sm + (size_t)slot * GMB + 3072 + 4 * tok) = am * (1.0f / Q6MAX);
+      }
+    }
+    if (tot <= GMX * NW / 4) {
+      w_store(0);
+      w_load(GMW);
+    }
+    w_store(GMW);
+    __syncthreads();
+    int l = l0, k = 0;
+    for (int i = 0; i < tot; ++i) {
+        if (l + k * L < ng) {
+          const uint8_t *sp = sm + (size_t)i * GMB;
+          const int wr = i * NW * 32 + wv * 32 + j;
+          const uint2 w = *reinterpret_cast<const uint2 *>(swq + wr * 16 + 8 * hh);
+          const float wsc = sws[wr];
+          const v4i b = {nib_s8(w.x), nib_s8(w.x >> 4), nib_s8(w.y), nib_s8(w.y >> 4)};
+          const v16i z = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+          v16i d[3];
+#pragma unroll
+          for (int p = 0; p < 3; ++p)
+            d[p] = __builtin_amdgcn_mfma_i32_32x32x32_i8(*reinterpret_cast<const v4i *>(sp + 1024 * p + 16 * lane), b,
+                                                         z, 0, 0, 0);
+          const float4 *sx4 = reinterpret_cast<const float4 *>(sp + 3072) + hh;
+          float f[16];
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const float4 s4 = sx4[2 * c];
+            const float sx[4] = {s4.x, s4.y, s4.z, s4.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int v = 4 * c + e;
+              uint32_t hm = ((uint32_t)d[0][v] << 8) + (uint32_t)d[1][v];
+              asm("" : "+v"(hm));  // two shift-adds instead of two shifts and an add3
+              f[v] = ((float)(int)((hm << 8) + (uint32_t)d[2][v]) * sx[e]) * wsc;
+            }
+          }
+          if (k == 0) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) a[v] = f[v];
+          } else {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) a[v] = a[v] + f[v];
+          }
+        } else if (k == 0) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) a[v] = 0.f;
+        }
+        if (++k < K) continue;
+        k = 0;
+        // the tree: partial l joins the finished subtrees on its left
+        bool more = true;
+#pragma unroll
+        for (int lev = 0; lev < LV; ++lev)
+          if (more) {
+            if (l & (1 << lev)) {
+#pragma unroll
+              for (int v = 0; v < 16; ++v) a[v] = lv[lev][v] + a[v];
+            } else {
+#pragma unroll
+              for (int v = 0; v < 16; ++v) lv[lev][v] = a[v];
+              more = false;
+            }
+          }
+        ++l;
+      }
+  }
+  if (row >= m) return;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int tok = T0 + 8 * (v >> 2) + 4 * hh + (v & 3);
+    if (tok < t) y[(size_t)tok * m + row] = a[v];
   }
 }
 
@@ -725,11 +937,40 @@ int amx_scratch_for(int dev, size_t need, unsigned char **out) {
   return 0;
 }
 
+// Tokens from which a GEMM takes the matrix cores.  Up to a few hundred tokens
+// that launch's time is one workgroup's own (16 us at 576 columns, 26 at 960, 60
+// at 2560), and the GEMV kernel needs 8, 7.6 and 15 us per eight tokens: 24
+// tokens 29 / 23 / 46 us against 16 / 26 / 60, 32 tokens 38 / 31 / 61 against
+// 16 / 26 / 60.
+constexpr int kGemmTok = 32;
+
+int gemm_q4_tiles(const Q4SegPlan &pl, int t, int m, int n, const uint8_t *packed, const float *scale, const float *x,
+                  float *y, hipStream_t st) {
+  // eight waves share a tile's staging where that still gives a workgroup per
+  // CU, else four
+  const long tiles = (t + 31) / 32;
+  const int nw = pl.L <= 16 && tiles * ((m + 255) / 256) >= device_wg_cap() / 8 ? 8 : 4;
+  // lane partials staged at a time: as many as the slots and 160 KB of LDS take
+  int lgc = 0;
+  const int slots = std::min(GMS, (int)(160 * 1024 / (GMB + gemm_wslot(nw))));
+  while ((1 << lgc) < pl.L && (2 << lgc) * pl.K <= slots) ++lgc;
+  const int nrb = (m + 32 * nw - 1) / (32 * nw);
+  MLLM_CHECK(tiles * nrb < (1l << 31), "%d tokens x %d rows exceed a launch", t, m);
+  const auto kern = nw == 8 ? k_gemm_q4<8, 4> : pl.L <= 16 ? k_gemm_q4<4, 4> : k_gemm_q4<4, 6>;
+  const size_t lds = (size_t)(pl.K << lgc) * (GMB + gemm_wslot(nw));
+  if (int rc = launch_dyn(kern, dim3(1), lds, st, "k_gemm_q4")) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(tiles * nrb)), dim3(64 * nw), lds, st, packed, scale, x, y, t, m, n, pl.L,
+                     pl.K, lgc, nrb);
+  MLLM_HIP(hipGetLastError());
+  return 0;
+}
+
 int q4_gemm(int t, int m, int n, const uint8_t *packed, const float *scale, const float *x, float *y,
             hipStream_t st) {
   MLLM_CHECK((size_t)m * n / 2 < (1ull << 31), "matrix of %zu bytes exceeds 2 GiB", (size_t)m * n / 2);
   const int ng = n / 32;
   const Q4SegPlan pl = q4_seg_plan(n, m, 1);
+  if (t >= kGemmTok) return gemm_q4_tiles(pl, t, m, n, packed, scale, x, y, st);
   const int P = q4_seg_pick_p(pl, m, 1);
   const int ntiles = (m + pl.rpp * P - 1) / (pl.rpp * P);
   for (int t0 = 0; t0 < t;) {
