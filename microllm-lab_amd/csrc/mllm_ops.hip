@@ -641,28 +641,53 @@ __global__ __launch_bounds__(WGT) void k_gemv_q8i_batched(const int8_t *const *_
 }
 
 // ---------------------------------------------------------------- f32 GEMV
-// One wavefront per row, lanes over float4s, fixed-pattern wave reduction.
+typedef float v4fl __attribute__((ext_vector_type(4)));
+// R rows per wavefront, lanes over float4s, fixed-pattern wave reduction (a
+// row's sum does not depend on R).  Bound by the matrix read: one row per wave
+// and ordinary loads took 22.6 us for 49152 x 576 (5.0 TB/s), loads past the
+// caches 21.3, four rows per wave (their loads in flight together) 18.0 (6.3
+// TB/s).  Matrices of fewer rows keep the ordinary loads: the caches hold them
+// between calls.
+template <int R>
 __global__ __launch_bounds__(WG) void k_gemv_f32(const float *__restrict__ w, const float *__restrict__ x,
                                                   float *__restrict__ y, int rows, int cols) {
   const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * (WG / 64) + (threadIdx.x >> 6);
+  const int row = (blockIdx.x * (WG / 64) + (threadIdx.x >> 6)) * R;
   if (row >= rows) return;
-  const float *wr = w + (size_t)row * cols;
-  float acc = 0.f;
+  const float *wr[R];
+  float acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    wr[r] = w + (size_t)min(row + r, rows - 1) * cols;
+    acc[r] = 0.f;
+  }
   if ((cols & 3) == 0) {
     for (int k = lane * 4; k < cols; k += 256) {
-      const float4 a = *reinterpret_cast<const float4 *>(wr + k);
       const float4 b = *reinterpret_cast<const float4 *>(x + k);
-      acc = __builtin_fmaf(a.x, b.x, acc);
-      acc = __builtin_fmaf(a.y, b.y, acc);
-      acc = __builtin_fmaf(a.z, b.z, acc);
-      acc = __builtin_fmaf(a.w, b.w, acc);
+      v4fl a[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const v4fl *p = reinterpret_cast<const v4fl *>(wr[r] + k);
+        a[r] = R > 1 ? __builtin_nontemporal_load(p) : *p;
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        acc[r] = __builtin_fmaf(a[r].x, b.x, acc[r]);
+        acc[r] = __builtin_fmaf(a[r].y, b.y, acc[r]);
+        acc[r] = __builtin_fmaf(a[r].z, b.z, acc[r]);
+        acc[r] = __builtin_fmaf(a[r].w, b.w, acc[r]);
+      }
     }
   } else {
-    for (int k = lane; k < cols; k += 64) acc = __builtin_fmaf(wr[k], x[k], acc);
+    for (int k = lane; k < cols; k += 64)
+#pragma unroll
+      for (int r = 0; r < R; ++r) acc[r] = __builtin_fmaf(wr[r][k], x[k], acc[r]);
   }
-  acc = wave_sum(acc);
-  if (lane == 0) y[row] = acc;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const float s = wave_sum(acc[r]);
+    if (lane == 0 && row + r < rows) y[row + r] = s;
+  }
 }
 
 // ---------------------------------------------------------------- elementwise
@@ -686,20 +711,43 @@ __global__ __launch_bounds__(WG) void k_silu_mul(int n, float *__restrict__ a, c
   }
 }
 
-// One thread per packed byte: two weights, each (nib - 8) * sc rounded once.
+// Four weights per thread and turn, each (nib - 8) * sc rounded once: rows and
+// their scales are contiguous, so quad i of the matrix has scale i / 8 and the
+// position needs no division.  Bound by the stores (16 bytes per 2.5 read): a
+// thread per byte with 8-byte stores and a 64-bit division took 41.4 us for
+// 49152 x 576 (3.2 TB/s), ordinary stores this way 30.6, stores past the caches
+// 19.5 (6.7 TB/s).  An output that the L2s hold keeps the ordinary stores: its
+// reader finds it there.
+constexpr int DQN = 4;                       // quads per thread, WG apart
+constexpr size_t kStreamBytes = 32u << 20;   // the eight L2s
+enum { DQ_A8 = 0, DQ_A16 = 1, DQ_STREAM = 2 };  // out 8- or 16-byte aligned; 16 and larger than the L2s
+template <int MODE>
 __global__ __launch_bounds__(WG) void k_dequant_q4(const uint8_t *__restrict__ packed, const float *__restrict__ scale,
-                                                    float *__restrict__ out, size_t nbytes, int cols) {
-  const size_t i = (size_t)blockIdx.x * WG + threadIdx.x;
-  if (i >= nbytes) return;
-  const int b = packed[i];
-  const size_t e = 2 * i;
-  const size_t row = e / cols;
-  const int col = (int)(e - row * cols);
-  const float sc = scale[row * (cols >> 5) + (col >> 5)];
-  float2 v;
-  v.x = (float)((b & 15) - 8) * sc;
-  v.y = (float)((b >> 4) - 8) * sc;
-  *reinterpret_cast<float2 *>(out + e) = v;
+                                                    float *__restrict__ out, size_t quads) {
+  const size_t i0 = (size_t)blockIdx.x * (WG * DQN) + threadIdx.x;
+  unsigned short b[DQN];
+  float s[DQN];
+#pragma unroll
+  for (int k = 0; k < DQN; ++k) {
+    const size_t i = min(i0 + (size_t)k * WG, quads - 1);
+    __builtin_memcpy(&b[k], packed + 2 * i, 2);  // any byte boundary
+    s[k] = scale[i >> 3];
+  }
+#pragma unroll
+  for (int k = 0; k < DQN; ++k) {
+    const size_t i = i0 + (size_t)k * WG;
+    if (i >= quads) break;
+    const float4 v = make_float4((float)((int)(b[k] & 15) - 8) * s[k], (float)((int)((b[k] >> 4) & 15) - 8) * s[k],
+                                 (float)((int)((b[k] >> 8) & 15) - 8) * s[k], (float)((int)(b[k] >> 12) - 8) * s[k]);
+    if (MODE == DQ_STREAM) {
+      __builtin_nontemporal_store((v4fl){v.x, v.y, v.z, v.w}, reinterpret_cast<v4fl *>(out) + i);
+    } else if (MODE == DQ_A16) {
+      reinterpret_cast<float4 *>(out)[i] = v;
+    } else {
+      reinterpret_cast<float2 *>(out)[2 * i] = make_float2(v.x, v.y);
+      reinterpret_cast<float2 *>(out)[2 * i + 1] = make_float2(v.z, v.w);
+    }
+  }
 }
 
 // ---------------------------------------------------------------- host side
@@ -1161,9 +1209,10 @@ extern "C" int mllm_gemv_f32(int m, int n, const float *w, const float *x, float
   MLLM_CHECK(m > 0 && n > 0, "invalid shape m=%d n=%d", m, n);
   MLLM_CHECK(w && x && y, "null pointer");
   MLLM_CHECK((n & 3) != 0 || (((uintptr_t)w | (uintptr_t)x) & 15) == 0, "w and x must be 16-byte aligned");
-  const int rows_per_wg = WG / 64;
-  hipLaunchKernelGGL(k_gemv_f32, dim3((m + rows_per_wg - 1) / rows_per_wg), dim3(WG), 0, as_stream(stream), w, x, y,
-                     m, n);
+  // four rows per wave where that still leaves four waves per SIMD
+  const int R = m >= 4 * 16 * (device_wg_cap() / 8) ? 4 : 1, per_wg = R * (WG / 64);
+  hipLaunchKernelGGL(R == 4 ? k_gemv_f32<4> : k_gemv_f32<1>, dim3((m + per_wg - 1) / per_wg), dim3(WG), 0,
+                     as_stream(stream), w, x, y, m, n);
   MLLM_HIP(hipGetLastError());
   return 0;
 }
@@ -1191,9 +1240,11 @@ extern "C" int mllm_dequant_q4(int m, int n, const uint8_t *packed, const float 
   MLLM_CHECK(n % 32 == 0, "n=%d not a multiple of 32", n);
   MLLM_CHECK(packed && scale && out, "null pointer");
   MLLM_CHECK(((uintptr_t)out & 7) == 0, "out must be 8-byte aligned");
-  const size_t nbytes = (size_t)m * n / 2;
-  hipLaunchKernelGGL(k_dequant_q4, dim3((unsigned)((nbytes + WG - 1) / WG)), dim3(WG), 0, as_stream(stream), packed,
-                     scale, out, nbytes, n);
+  const size_t quads = (size_t)m * n / 4, blocks = (quads + WG * DQN - 1) / (WG * DQN);
+  const auto kern = ((uintptr_t)out & 15) != 0       ? k_dequant_q4<DQ_A8>
+                    : quads * 16 > kStreamBytes ? k_dequant_q4<DQ_STREAM>
+                                                : k_dequant_q4<DQ_A16>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(WG), 0, as_stream(stream), packed, scale, out, quads);
   MLLM_HIP(hipGetLastError());
   return 0;
 }
