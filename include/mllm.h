@@ -73,7 +73,7 @@ int mllm_gemv_q4(int m, int n, const uint8_t *packed, const float *scale, int gr
  * computes it (bit-identical), and *argmax = the first index of the maximum
  * of y (best = 0, bestV = y[0], then each later row strictly larger; NaN
  * rows never win).  argmax is a device pointer.  The per-workgroup maxima and
- * a completion counter live in a scratch buffer that the library allocates
+ * the completion counter live in a scratch buffer that the library allocates
  * per device on first use; calls on one device must not overlap. */
 int mllm_gemv_q4_argmax(int m, int n, const uint8_t *packed, const float *scale, int group, const float *x, float *y,
                         int32_t *argmax, void *stream);

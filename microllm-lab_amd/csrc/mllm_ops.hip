@@ -203,20 +203,46 @@ __global__ __launch_bounds__(WGT) void k_gemv_q4_batched(const uint8_t *const *_
   q4_gemv_tile<WGT, P, K>(packed[b], scale[b], xv[b], yv[b], G, blockIdx.x, reinterpret_cast<uint32_t *>(smem4));
 }
 
-// y = W x (one token) and the first index of its maximum, in one launch
-// (infer.js:597-600 + argmax, infer.js:240-250: best = 0, bestV = y[0], then
-// every later row that is strictly larger; a NaN row never wins, and a NaN
-// y[0] keeps index 0).  Each workgroup reduces its tile's rows to a (value,
-// row) pair in the scratch buffer; the last workgroup to finish (a counter in
-// the scratch) reduces the pairs and writes the index.  Scratch layout
-// (bytes): [0, 4) the counter, which every completed launch leaves at 0;
-// [4, 8) row 0 is NaN (tile 0 writes it); [64, 64 + 4 ntiles) the tiles'
-// values, then ntiles rows.  Two launches that share a scratch buffer must
-// not overlap.
+// y = W x (one token) and the first index of its maximum (infer.js:597-600 +
+// argmax, infer.js:240-250: best = 0, bestV = y[0], then every later row that is
+// strictly larger; a NaN row never wins, and a NaN y[0] keeps index 0).  Each
+// workgroup of the GEMV reduces its tile's rows to a (value, row) pair in the
+// scratch buffer, and the pairs are reduced
+//   ONE   by the last workgroup to finish (a counter in the scratch): one
+//         launch, but three device-scope round trips after the last tile -- the
+//         pair's store, the count, the pairs;
+//   else  by a second launch of one workgroup.
+// Measured, us a call, ONE and two launches: 63 tiles (4000 x 576) 5.9 and 6.6,
+// 250 tiles (16000 x 576) 8.0 and 6.7, 768 (49152 x 960) 15.6 and 10.0: the
+// round trips grow with the workgroups that contend for the counter, the second
+// launch costs the host 1.3 us.  kAmxTwo tiles and more take two launches.
+// Scratch layout (bytes): [0, 4) the counter, which every completed call leaves
+// at 0; [4, 8) row 0 is NaN (tile 0 writes it); [64, 64 + 4 ntiles) the tiles'
+// values, then ntiles rows.  Two calls that share a scratch buffer must not
+// overlap.
 constexpr size_t kAmxHead = 64;
+constexpr int kAmxTwo = 128;
 __host__ __device__ constexpr size_t amx_scratch_bytes(int ntiles) { return kAmxHead + 8 * (size_t)ntiles; }
 
-template <int WGT, int P, int K>
+// The workgroup's first maximum, in thread 0.
+template <int NT>
+__device__ __forceinline__ void block_argmax(float &v, int &i, float *wv, int *wi) {
+  const int t = threadIdx.x;
+  wave_argmax(v, i);
+  if ((t & 63) == 0) {
+    wv[t >> 6] = v;
+    wi[t >> 6] = i;
+  }
+  __syncthreads();
+  if (t == 0)
+    for (int w = 1; w < NT / 64; ++w)
+      if (amax_better(wv[w], wi[w], v, i)) {
+        v = wv[w];
+        i = wi[w];
+      }
+}
+
+template <int WGT, int P, int K, bool ONE>
 __global__ __launch_bounds__(WGT) void k_gemv_q4_argmax(const uint8_t *__restrict__ packed,
                                                         const float *__restrict__ scale, const float *__restrict__ x,
                                                         float *__restrict__ y, GemvGeom G, unsigned char *scratch,
@@ -233,19 +259,16 @@ __global__ __launch_bounds__(WGT) void k_gemv_q4_argmax(const uint8_t *__restric
   const int t = threadIdx.x;
   float v = rm.v;
   int i = rm.i;
-  wave_argmax(v, i);
-  if ((t & 63) == 0) {
-    wv[t >> 6] = v;
-    wi[t >> 6] = i;
+  block_argmax<WGT>(v, i, wv, wi);
+  if (!ONE) {
+    if (t != 0) return;
+    if (blockIdx.x == 0) *nan0 = rm.nan0 ? 1 : 0;  // thread 0 of tile 0 summed row 0
+    tv[blockIdx.x] = v;
+    ti[blockIdx.x] = i;
+    return;
   }
-  if (blockIdx.x == 0 && t == 0) coh_sti(nan0, 0, rm.nan0 ? 1 : 0);  // thread 0 of tile 0 summed row 0
-  __syncthreads();
   if (t == 0) {
-    for (int w = 1; w < WGT / 64; ++w)
-      if (amax_better(wv[w], wi[w], v, i)) {
-        v = wv[w];
-        i = wi[w];
-      }
+    if (blockIdx.x == 0) coh_sti(nan0, 0, rm.nan0 ? 1 : 0);
     coh_stf(tv, 4u * blockIdx.x, v);
     coh_sti(ti, 4u * blockIdx.x, i);
     wait_stores();  // the pair (and nan0) are visible before the count is
@@ -263,23 +286,35 @@ __global__ __launch_bounds__(WGT) void k_gemv_q4_argmax(const uint8_t *__restric
       i = ki;
     }
   }
-  wave_argmax(v, i);
   __syncthreads();
-  if ((t & 63) == 0) {
-    wv[t >> 6] = v;
-    wi[t >> 6] = i;
-  }
-  __syncthreads();
+  block_argmax<WGT>(v, i, wv, wi);
   if (t == 0) {
-    for (int w = 1; w < WGT / 64; ++w)
-      if (amax_better(wv[w], wi[w], v, i)) {
-        v = wv[w];
-        i = wi[w];
-      }
     // every row NaN leaves i at INT_MAX; row 0 NaN wins in any case
     *out = coh_ldi(nan0, 0) || i == 0x7fffffff ? 0 : i;
     __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+constexpr int AMT = 1024;  // threads of the reducing workgroup
+__global__ __launch_bounds__(AMT) void k_argmax_tiles(const unsigned char *__restrict__ scratch, int ntiles,
+                                                      int32_t *out) {
+  __shared__ float wv[AMT / 64];
+  __shared__ int wi[AMT / 64];
+  const float *tv = reinterpret_cast<const float *>(scratch + kAmxHead);
+  const int *ti = reinterpret_cast<const int *>(scratch + kAmxHead + 4 * (size_t)ntiles);
+  const int t = threadIdx.x, nan0 = *reinterpret_cast<const int *>(scratch + 4);
+  float v = -INFINITY;
+  int i = 0x7fffffff;
+  for (int k = t; k < ntiles; k += AMT) {
+    const float kv = tv[k];
+    const int ki = ti[k];
+    if (amax_better(kv, ki, v, i)) {
+      v = kv;
+      i = ki;
+    }
+  }
+  block_argmax<AMT>(v, i, wv, wi);
+  if (t == 0) *out = nan0 || i == 0x7fffffff ? 0 : i;
 }
 
 // ---------------------------------------------------------------- Q4 GEMM on the int8 matrix cores
@@ -919,8 +954,11 @@ size_t q4_seg_lds(int ng, int m) { return sizeof(uint32_t) * (size_t)m * ng * Q6
 template <int WGT, int P, int K>
 int q4_launch_argmax(dim3 grid, size_t lds, hipStream_t st, const uint8_t *packed, const float *scale, const float *x,
                      float *y, const GemvGeom &G, unsigned char *scratch, int32_t *out) {
-  if (int rc = launch_dyn(k_gemv_q4_argmax<WGT, P, K>, grid, lds, st, "k_gemv_q4_argmax")) return rc;
-  hipLaunchKernelGGL((k_gemv_q4_argmax<WGT, P, K>), grid, dim3(WGT), lds, st, packed, scale, x, y, G, scratch, out);
+  const bool two = (int)grid.x >= kAmxTwo;
+  const auto kern = two ? k_gemv_q4_argmax<WGT, P, K, false> : k_gemv_q4_argmax<WGT, P, K, true>;
+  if (int rc = launch_dyn(kern, grid, lds, st, "k_gemv_q4_argmax")) return rc;
+  hipLaunchKernelGGL(kern, grid, dim3(WGT), lds, st, packed, scale, x, y, G, scratch, out);
+  if (two) hipLaunchKernelGGL(k_argmax_tiles, dim3(1), dim3(AMT), 0, st, scratch, (int)grid.x, out);
   MLLM_HIP(hipGetLastError());
   return 0;
 }

@@ -341,7 +341,7 @@ __global__ __launch_bounds__(64) void k_pf_final(const float *x, int K, int t, c
 // A wave computes two 32-row sub-tiles (sub-tile 1 is either the next 32
 // rows of the same matrix -- a 64-row head of attn.qkv, 64 rows of the
 // others -- or the same rows of a second matrix: mlp.w3 beside mlp.w1) for
-// 32 tokens.  Workgroup: GWG / 64 waves, one token tile; with KS > 1, KS waves
+// 32 tokens.  Workgroup: gemm_threads(KS) / 64 waves, one token tile; with KS > 1, KS waves
 // share a row range and take consecutive slices of the groups, and their
 // sums are added in slice order through LDS (deterministic) before the
 // epilogue -- more waves for the GEMMs with few row ranges.
@@ -382,7 +382,9 @@ constexpr int GPF = MLLM_PF_GPF;  // groups of loads in flight per wave
 #ifndef MLLM_PF_GWG
 #define MLLM_PF_GWG 256
 #endif
-constexpr int GWG = MLLM_PF_GWG;  // threads per GEMM workgroup (waves sharing one token tile)
+// threads per GEMM workgroup (waves sharing one token tile): eight slices are
+// a workgroup of their own
+constexpr int gemm_threads(int ks) { return ks == 8 ? 512 : MLLM_PF_GWG; }
 
 struct Pieces {
   v8h p0a, p0b, p1a, p1b, p2a, p2b;  // piece 0 .. 2, K half a / b
@@ -413,7 +415,8 @@ __device__ __forceinline__ void pf_group_acc(const Pieces &x, uint2 w, float c, 
 }
 
 template <int EPI, int KS>
-__global__ __launch_bounds__(GWG) void k_pf_gemm(PfArgs A, PfGemm G) {
+__global__ __launch_bounds__(gemm_threads(KS)) void k_pf_gemm(PfArgs A, PfGemm G) {
+  constexpr int GWG = gemm_threads(KS);
   __shared__ float red[KS > 1 ? GWG * 32 : 1];
   const int wv = tid() >> 6, lane = tid() & 63, j = lane & 31, hh = lane >> 5;
   const int ks = wv % KS;
@@ -457,21 +460,28 @@ __global__ __launch_bounds__(GWG) void k_pf_gemm(PfArgs A, PfGemm G) {
   float acc0[16], acc1[16];
 #pragma unroll
   for (int v = 0; v < 16; ++v) acc0[v] = acc1[v] = 0.f;
-  // the loads of group g + GPF go out before group g is computed
-  GemmLd ring[GPF];
+  // the loads of group g + NR go out before group g is computed
+  constexpr int NR = GPF;
+  GemmLd ring[NR];
   if (active) {
     // (groups past ge are loaded and not used: the tiled matrices and the
-    // activation tiles carry GPF groups of padding)
+    // activation tiles carry NR groups of padding)
 #pragma unroll
-    for (int i = 0; i < GPF; ++i) ring[i] = load(gb + i);
-    for (int g0 = gb; g0 < ge; g0 += GPF)
+    for (int i = 0; i < NR; ++i) ring[i] = load(KS < 8 ? gb + i : min(gb + i, ge - 1));
+    for (int g0 = gb; g0 < ge; g0 += NR)
 #pragma unroll
-      for (int i = 0; i < GPF; ++i) {
+      for (int i = 0; i < NR; ++i) {
         if (g0 + i >= ge) break;
-        const GemmLd cur = ring[i];
-        ring[i] = load(g0 + i + GPF);
-        pf_group_acc(cur.x, cur.w0, cur.c0, acc0);
-        pf_group_acc(cur.x, cur.w1, cur.c1, acc1);
+        if constexpr (KS < 8) {
+          const GemmLd cur = ring[i];
+          ring[i] = load(g0 + i + NR);
+          pf_group_acc(cur.x, cur.w0, cur.c0, acc0);
+          pf_group_acc(cur.x, cur.w1, cur.c1, acc1);
+        } else {  // short slices: nothing is read past their end
+          pf_group_acc(ring[i].x, ring[i].w0, ring[i].c0, acc0);
+          pf_group_acc(ring[i].x, ring[i].w1, ring[i].c1, acc1);
+          if (g0 + i + NR < ge) ring[i] = load(g0 + i + NR);
+        }
       }
   }
   if (KS > 1) {
@@ -479,7 +489,7 @@ __global__ __launch_bounds__(GWG) void k_pf_gemm(PfArgs A, PfGemm G) {
     // lanes of a wave touch 1 KiB of consecutive LDS per access, so no two
     // lanes of a pass share a bank
     v4f *red4 = reinterpret_cast<v4f *>(red);
-    if (ks > 0) {
+    if (ks > 0 || KS == 8) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         red4[q * GWG + tid()] = v4f{acc0[4 * q], acc0[4 * q + 1], acc0[4 * q + 2], acc0[4 * q + 3]};
@@ -487,9 +497,30 @@ __global__ __launch_bounds__(GWG) void k_pf_gemm(PfArgs A, PfGemm G) {
       }
     }
     __syncthreads();
+    if constexpr (KS == 8) {
+      // a wave per quad sums its eight slices, in the same order
+      v4f *p = red4 + (tid() >> 6) * GWG + (tid() & 63);
+      v4f t[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) t[k] = p[64 * k];
+#pragma unroll
+      for (int k = 1; k < 8; ++k) t[0] = t[0] + t[k];
+      p[0] = t[0];
+      __syncthreads();
+      if (ks > 0) return;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const v4f a = red4[q * GWG + tid()], b = red4[(4 + q) * GWG + tid()];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          acc0[4 * q + e] = a[e];
+          acc1[4 * q + e] = b[e];
+        }
+      }
+    }
     if (ks > 0) return;
 #pragma unroll
-    for (int k = 1; k < KS; ++k) {
+    for (int k = 1; k < (KS == 8 ? 1 : KS); ++k) {
       const int o = tid() + 64 * k;  // the same lane of slice k's wave
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -919,19 +950,30 @@ void launch_quant(const PfArgs &A, const float *src, int K, const float *g, int 
 #ifndef MLLM_PF_MINSLICE
 #define MLLM_PF_MINSLICE 8
 #endif
+#ifndef MLLM_PF_SMALL
+#define MLLM_PF_SMALL 256
+#endif
 // Group slices per row range (KS, 1, 2 or 4): doubled while the launch has
 // fewer than MLLM_PF_WAVES row waves and every slice keeps MLLM_PF_MINSLICE
 // groups (1024 and 8 measured best: 2048 or 4096 waves gave longer prompts).
+// Launches of at most MLLM_PF_SMALL row waves -- short prompts -- take eight
+// slices, three groups or so each, in one round of loads: they are bound by
+// the latency of a wave's group loop.  Prompt us, four slices at most -> eight:
+// GPT-2 124M 33 tokens 1226 -> 978, 128 1344 -> 1083; 135M 33 tokens 2506 ->
+// 1986, 200 2933 -> 2475; 360M 100 tokens 3333 -> 2808.  With 512 row waves as
+// the line 1000 tokens took 2378 instead of 2153, with 128 the 128 tokens 1161.
 template <int EPI>
 void launch_gemm(const PfArgs &A, const PfGemm &G, hipStream_t s) {
   const int tt = (G.n + 31) / 32 - G.tt0, rw = (G.rows + G.rstep - 1) / G.rstep;
   int ks = 1;
   while (ks < 4 && rw * tt * ks < MLLM_PF_WAVES && G.ng / (2 * ks) >= MLLM_PF_MINSLICE) ks *= 2;
-  const int per_wg = (GWG / 64 / ks) * G.rstep;
+  if (rw * tt <= MLLM_PF_SMALL && G.ng >= 16) ks = 8;
+  const int gwg = gemm_threads(ks), per_wg = (gwg / 64 / ks) * G.rstep;
   const dim3 grid((G.rows + per_wg - 1) / per_wg, tt);
-  if (ks == 1) hipLaunchKernelGGL((k_pf_gemm<EPI, 1>), grid, dim3(GWG), 0, s, A, G);
-  if (ks == 2) hipLaunchKernelGGL((k_pf_gemm<EPI, 2>), grid, dim3(GWG), 0, s, A, G);
-  if (ks == 4) hipLaunchKernelGGL((k_pf_gemm<EPI, 4>), grid, dim3(GWG), 0, s, A, G);
+  if (ks == 1) hipLaunchKernelGGL((k_pf_gemm<EPI, 1>), grid, dim3(gwg), 0, s, A, G);
+  if (ks == 2) hipLaunchKernelGGL((k_pf_gemm<EPI, 2>), grid, dim3(gwg), 0, s, A, G);
+  if (ks == 4) hipLaunchKernelGGL((k_pf_gemm<EPI, 4>), grid, dim3(gwg), 0, s, A, G);
+  if (ks == 8) hipLaunchKernelGGL((k_pf_gemm<EPI, 8>), grid, dim3(gwg), 0, s, A, G);
 }
 
 PfGemm gemm_same(const PfMat &W, int n, const float *bias, float *out, int ldo) {

@@ -111,3 +111,36 @@ def test_gemv_f32_rows_per_wave(n):
     assert got[m] == 7.0 and np.array_equal(got[:1000], y1.cpu().numpy())
     bound = (n + 8) * 2.0**-24 * (np.abs(w).astype(np.float64) @ np.abs(x).astype(np.float64))
     assert (np.abs(got[:m] - w.astype(np.float64) @ x.astype(np.float64)) <= bound).all()
+
+
+@gpu
+@pytest.mark.parametrize("rows", [16256, 16257, 16384, 16385])
+@pytest.mark.parametrize("kind", ["first of ties", "nan0", "nan rows", "all nan"])
+def test_argmax_on_both_sides_of_two_launches(rows, kind):
+    """128 rows a tile: 127 tiles (one launch) and 128 or 129 (two), called
+    twice on the same scratch, the index by infer.js:240-250."""
+    rng = np.random.default_rng(rows)
+    n = 64
+    packed, sc = pgw.quant_q4(rng.standard_normal((rows, n)).astype(np.float32))
+    x = rng.standard_normal(n).astype(np.float32)
+    if kind == "first of ties":
+        best = int(np.argmax(pgw.dequant_q4(packed, sc) @ x))
+        packed[[rows - 1, rows // 2]] = packed[best]
+        sc[[rows - 1, rows // 2]] = sc[best]
+    elif kind == "nan0":
+        sc[0, 0] = np.nan
+    elif kind == "nan rows":
+        sc[1::5, 1] = np.nan
+    else:
+        sc[:, 0] = np.nan
+    dp, ds, dx = (torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (packed, sc, x))
+    y = torch.empty(rows, dtype=torch.float32, device="cuda")
+    i = torch.full((1,), -5, dtype=torch.int32, device="cuda")
+    print(f"argmax rows={rows} {kind}", flush=True)
+    for _ in range(2):
+        i.fill_(-5)
+        abi.call("mllm_gemv_q4_argmax", rows, n, ptr(dp), ptr(ds), 32, ptr(dx), ptr(y), ptr(i), None)
+        torch.cuda.synchronize()
+        v = y.cpu().numpy()
+        want = 0 if np.isnan(v[0]) or np.isnan(v).all() else int(np.nanargmax(v))
+        assert int(i.item()) == want

@@ -295,3 +295,23 @@ def test_batched_prompt_every_length_vs_oracle(oracle_lib):
     ref.close()
     print(f"every length: worst {max(rel.values()):.2e}", flush=True)
     assert max(rel.values()) <= PREFILL_TOL, {n: r for n, r in rel.items() if r > PREFILL_TOL}
+
+
+@gpu
+@pytest.mark.parametrize("n", [2, 31, 33, 64])
+def test_short_prompt_slices_vs_oracle(oracle_lib, n):
+    """Short prompts run their GEMMs in eight group slices from 16 groups on:
+    rows of 16 (two groups a slice), 18 and 34 groups (uneven slices)."""
+    for arch, d, ff in (("llama", 512, 576), ("gpt2", 576, 1088)):
+        h = d // 64
+        bundle = build(arch, seed=31, n_layers=2, d_model=d, n_heads=h, n_kv_heads=h if arch == "gpt2" else 4,
+                       d_ff=ff, max_seq_len=80)
+        g = mllm.PetitGPT(bundle)
+        ref = oracle_lib.OracleModel(bundle)
+        ids = [int(v) for v in np.random.default_rng(n).integers(0, bundle.cfg.vocab_size, n)]
+        lg, lr = g.forwardPrompt(ids).copy(), ref.forward_prompt(ids)
+        g.destroy()
+        ref.close()
+        rel = float(np.abs(lg - lr).max()) / float(np.abs(lr).max())
+        print(f"short prompt {arch} n={n}: {rel:.2e}", flush=True)
+        assert rel <= PREFILL_TOL, rel
