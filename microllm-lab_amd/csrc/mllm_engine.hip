@@ -70,6 +70,7 @@ namespace mllm {
 constexpr int HD = 64;     // head dimension of every supported config
 constexpr int ACH = 256;   // positions per attention split (one per thread)
 constexpr int MAXT = 16;   // tokens per pass (upper bound; LDS sets the real one)
+static_assert(MAXT == kGenericTokens, "the generic pass's rows");
 constexpr int APS = 68;    // floats per attention partial: m, l, pad, pad, acc[64]
 constexpr int APT = 66;    // tagged pairs per attention partial of the persistent kernels: m, l, acc[64]
 constexpr int TC = 2;      // chunk registers per thread of an LM tile (TC * WG chunks)
@@ -3464,11 +3465,11 @@ int generic_create(mllm_model *M) {
   }
   const size_t kv_bytes = (size_t)L * 2 * NKV * c.max_seq_len * HD * (c.kv_fp16 ? 2 : 4);
   int rc = dev_alloc(M, &A.kv, kv_bytes);
-  if (!rc) rc = dev_alloc(M, (void **)&A.x, sizeof(float) * D);
-  if (!rc) rc = dev_alloc(M, (void **)&A.qkv, sizeof(float) * (D + 2 * kvd));
+  if (!rc) rc = dev_alloc(M, (void **)&A.x, sizeof(float) * kGenericTokens * D);
+  if (!rc) rc = dev_alloc(M, (void **)&A.qkv, sizeof(float) * kGenericTokens * (D + 2 * kvd));
   if (!rc)
-    rc = dev_alloc(M, (void **)&A.attp, sizeof(float) * NH * ((c.max_seq_len + kGenericSplit - 1) / kGenericSplit) * kGenericPart);
-  if (!rc) rc = dev_alloc(M, (void **)&A.h, sizeof(float) * FF);
+    rc = dev_alloc(M, (void **)&A.attp, sizeof(float) * kGenericTokens * NH * ((c.max_seq_len + kGenericSplit - 1) / kGenericSplit) * kGenericPart);
+  if (!rc) rc = dev_alloc(M, (void **)&A.h, sizeof(float) * kGenericTokens * FF);
   if (!rc) rc = dev_alloc(M, (void **)&M->d_logits, sizeof(float) * MAXT * (size_t)V);
   if (!rc) rc = dev_alloc(M, (void **)&A.res, sizeof(int) * MAXT);
   if (!rc) rc = dev_alloc(M, (void **)&A.cur, sizeof(GCursor));
@@ -4022,6 +4023,7 @@ static int g_begin(mllm_model *M, const int32_t *ids, int n, int pos0, int chain
   GCursor &c = *M->h_gcur;
   memset(&c, 0, sizeof c);
   c.pos_next = pos0;
+  c.pos = pos0;
   c.chain = chain;
   c.rows = rows;
   c.tok = first;
@@ -4034,11 +4036,11 @@ static int g_begin(mllm_model *M, const int32_t *ids, int n, int pos0, int chain
 }
 
 static int g_enqueue(mllm_model *M, bool lm) {
-  if (M->exec_mode == 2) return g_step(M->g, lm, M->stream);
+  if (M->exec_mode == 2) return g_step(M->g, lm, 1, M->stream);
   hipGraphExec_t &ge = M->g_graph[lm ? 1 : 0];
   if (!ge) {
     MLLM_HIP(hipStreamBeginCapture(M->stream, hipStreamCaptureModeThreadLocal));
-    const int rc = g_step(M->g, lm, M->stream);
+    const int rc = g_step(M->g, lm, 1, M->stream);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(M->stream, &g);
     if (rc || e != hipSuccess) {
@@ -4061,8 +4063,12 @@ static int g_enqueue(mllm_model *M, bool lm) {
 static int g_run(mllm_model *M, const int32_t *ids, int n, int pos0, bool rows, float *logits, int32_t *argmax) {
   if (int rc = g_begin(M, ids, n, pos0, 0, rows ? 1 : 0, 0, 0, -1)) return rc;
   MLLM_HIP(hipEventRecord(M->ev0, M->stream));
-  for (int t = 0; t < n; ++t)
-    if (int rc = g_enqueue(M, rows || t == n - 1)) return rc;
+  if (rows && n > 1) {  // a verify pass: each kernel once for all its tokens
+    if (int rc = g_step(M->g, true, n, M->stream)) return rc;
+  } else {
+    for (int t = 0; t < n; ++t)
+      if (int rc = g_enqueue(M, rows || t == n - 1)) return rc;
+  }
   MLLM_HIP(hipEventRecord(M->ev1, M->stream));
   MLLM_HIP(hipStreamSynchronize(M->stream));
   MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
@@ -4083,7 +4089,7 @@ static int g_prompt(mllm_model *M, const int32_t *ids, int n, float *logits, int
     const int m = std::min(M->gp.tc, n - p0);
     if (int rc = gp_layers(M->gp, ids + p0, m, p0, p0 + m == n, &row, M->stream)) return rc;
   }
-  if (int rc = g_head(M->g, row, M->stream)) return rc;
+  if (int rc = g_head(M->g, row, 1, M->stream)) return rc;
   MLLM_HIP(hipEventRecord(M->ev1, M->stream));
   MLLM_HIP(hipStreamSynchronize(M->stream));
   MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));

@@ -46,6 +46,7 @@ struct GCursor {
 
 // Positions per attention workgroup, and the floats of its partial.
 constexpr int kGenericSplit = 256, kGenericPart = 68;
+constexpr int kGenericTokens = 16;  // tokens of a pass at most
 
 struct GArgs {
   int arch, L, D, NH, NKV, FF, V, max_seq, kv_fp16;
@@ -55,8 +56,8 @@ struct GArgs {
   GMat lm;               // tied lm_head (and the embedding rows)
   const float *norm_f, *wpe, *sf, *rope_cos, *rope_sin;
   void *kv;                  // [L][2][NKV][max_seq][64], f32 or f16 (the engine's cache)
-  float *x, *qkv, *h;        // one token's rows: [D], [D + 2 NKV 64], [FF]
-  float *attp;               // [NH][splits of max_seq][kGenericPart] attention partials
+  float *x, *qkv, *h;        // a pass's rows: [kGenericTokens][D], [..][D + 2 NKV 64], [..][FF]
+  float *attp;               // [kGenericTokens][NH][splits of max_seq][kGenericPart] attention partials
   float *logits;             // [rows][V]
   int *res;                  // argmax per logits row
   GCursor *cur;
@@ -64,16 +65,20 @@ struct GArgs {
   int *hist;                 // chained calls: the history, then the ids emitted
 };
 
-// Enqueue one token's step: embedding of the cursor's token at its
+// Enqueue one token's step (m = 1): embedding of the cursor's token at its
 // position, every layer, and with lm the final norm, the lm_head (logits
 // row: the cursor's i with rows set, else 0) and the argmax (res[row]; in
 // chained calls the chain's bookkeeping).  In chained calls every kernel
 // returns at once once an EOS has been emitted.
-int g_step(const GArgs &A, bool lm, hipStream_t s);
+// With m > 1 a pass of m tokens (verify): ids[0 .. m) at positions pos .. of a
+// cursor whose pos is set and whose i is 0, logits and argmax of every row.
+// Each kernel runs once for all tokens, and every token's arithmetic is the
+// single step's, so its row is bit-identical.
+int g_step(const GArgs &A, bool lm, int m, hipStream_t s);
 
 // The end of a step from the residual row x: the final norm, the lm_head
 // (logits row as in g_step) and the argmax.
-int g_head(const GArgs &A, const float *x, hipStream_t s);
+int g_head(const GArgs &A, const float *x, int m, hipStream_t s);
 
 // y[rows] = W . x[cols] (model.gemv for any storage).
 int g_gemv(const GMat &W, const float *x, float *y, hipStream_t s);

@@ -143,13 +143,15 @@ struct GemvArgs {
   const GCursor *cur;
   int lm;              // 1: y is the logits, row cur->i when cur->rows (verify)
   int nsplit_max;      // GN_SPLITS: partials per head in x
+  int m, xs;           // tokens of the pass and the stride of their inputs (outputs: W.rows)
 };
 
 // The attention's output row from its splits' partials (infer.js:466-495) into
 // LDS: a thread per four components, its splits' loads four at a time.
-__device__ __forceinline__ void merge_splits(const GemvArgs &a, int ns, float *sx) {
+__device__ __forceinline__ void merge_splits(const GemvArgs &a, int tok, float *sx) {
+  const int ns = (a.cur->pos + tok) / GSPLIT + 1;
   for (int i = tid(); i < (a.W.cols >> 2); i += GT) {
-    const float *p = a.x + (size_t)(i >> 4) * a.nsplit_max * GAPS;
+    const float *p = a.x + (size_t)tok * a.xs + (size_t)(i >> 4) * a.nsplit_max * GAPS;
     float mx = -INFINITY, l = 0.f;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
     for (int s0 = 0; s0 < ns; s0 += 4) {
@@ -231,6 +233,7 @@ __global__ __launch_bounds__(GT) void k_g_gemv(GemvArgs a) {
   auto chunk = [&](int k) { return min(l + k * L, nc - 1); };  // past the row: a valid chunk, its input taken as 0
   auto row_of = [&](int g) { return min(g * rpw + seg, rows - 1); };
   const GCursor *cur = a.cur;
+  const int tok = blockIdx.y;  // passes of several tokens: a weight row's workgroups meet it in the caches
   if (nch <= CB) {
     // every load of the first rows and of the input row, then the rest
     Raw<KIND> w[CB], w3[EPI == G_SWIGLU ? CB : 1];
@@ -246,7 +249,7 @@ __global__ __launch_bounds__(GT) void k_g_gemv(GemvArgs a) {
     if (NORM != GN_SPLITS) {
 #pragma unroll
       for (int k = 0; k < CB; ++k)
-        if (k < nch) in8(a.x, chunk(k), x[k]);
+        if (k < nch) in8(a.x + (size_t)tok * a.xs, chunk(k), x[k]);
     }
     load(g0);
     if (NORM == GN_RMS || NORM == GN_LN) {
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(GT) void k_g_gemv(GemvArgs a) {
       for (int k = 0; k < CB; ++k)
         if (k < nch) vec8(a.gains, chunk(k), gv[k]);
     }
-    float *y = a.y;
+    float *y = a.y + (size_t)tok * rows;
     RowEnd E = row_end<EPI>(a, y, row_of(g0));
     loads_first();
     if (cur) {
@@ -262,7 +265,7 @@ __global__ __launch_bounds__(GT) void k_g_gemv(GemvArgs a) {
       if (a.lm && cur->rows) y += (size_t)cur->i * rows;
     }
     if (NORM == GN_SPLITS) {
-      merge_splits(a, cur->pos / GSPLIT + 1, sx);
+      merge_splits(a, tok, sx);
       __syncthreads();
 #pragma unroll
       for (int k = 0; k < CB; ++k)
@@ -348,12 +351,12 @@ __global__ __launch_bounds__(GT) void k_g_gemv(GemvArgs a) {
   }
   // rows past the registers (L = 64): the moments first, then CB chunks at a time
   if (cur && stopped(cur)) return;
-  float *y = a.y + (a.lm && cur->rows ? (size_t)cur->i * rows : 0);
+  float *y = a.y + (a.lm && cur->rows ? (size_t)cur->i * rows : 0) + (size_t)tok * rows;
   if (NORM == GN_SPLITS) {
-    merge_splits(a, cur->pos / GSPLIT + 1, sx);
+    merge_splits(a, tok, sx);
     __syncthreads();
   }
-  const float *x = NORM == GN_SPLITS ? sx : a.x;
+  const float *x = NORM == GN_SPLITS ? sx : a.x + (size_t)tok * a.xs;
   float scale = 1.f, mean = 0.f;
   if (NORM == GN_RMS || NORM == GN_LN) {
     float s = 0.f;
@@ -424,10 +427,14 @@ __device__ __forceinline__ size_t g_kv_index(const GArgs &A, int li, int which, 
 __global__ __launch_bounds__(GT) void k_g_embed(GArgs A) {
   GCursor *cur = A.cur;
   if (stopped(cur)) return;
-  const int D = A.D, pos = cur->pos_next, ti = cur->i_next;
+  // a pass of several tokens (a workgroup each) starts from a cursor that the
+  // host has set and leaves it alone
+  const bool pass = gridDim.x > 1;
+  const int D = A.D, pos = pass ? cur->pos + (int)blockIdx.x : cur->pos_next, ti = pass ? (int)blockIdx.x : cur->i_next;
   const int id = cur->chain ? cur->tok : A.ids[ti];
+  float *x = A.x + (size_t)blockIdx.x * D;
   __syncthreads();  // every thread has read the cursor
-  if (tid() == 0) {
+  if (tid() == 0 && !pass) {
     cur->pos = pos;
     cur->i = ti;
     cur->pos_next = pos + 1;
@@ -447,7 +454,7 @@ __global__ __launch_bounds__(GT) void k_g_embed(GArgs A) {
         if (quant && A.sf) v = v / A.sf[i];
         v = v + A.wpe[(size_t)min(pos, A.max_seq - 1) * D + i];
       }
-      A.x[i] = v;
+      x[i] = v;
     }
   }
 }
@@ -479,7 +486,8 @@ template <bool F16>
 __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
   __shared__ __attribute__((aligned(16))) float own[GAW][3 * GHD];  // each wave's q, new k, new v
   __shared__ float part[GAW][GHD + 2];
-  const int done = A.cur->done, pos = A.cur->pos, rep = A.NH / A.NKV, n = pos + 1;  // one load
+  const int tok = blockIdx.z;
+  const int done = A.cur->done, pos = A.cur->pos + tok, rep = A.NH / A.NKV, n = pos + 1;  // one load
   if (done) return;
   const int h = blockIdx.x, kvh = h / rep, lane = tid() & 63, wv = tid() >> 6;
   const int s0 = (int)blockIdx.y * GSPLIT;
@@ -489,8 +497,8 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
   const bool on = k0 < n;       // uniform in the wave
   // q, k, v rows of the step, one component per lane (these loads first)
   float *qs = own[wv], *kn = qs + GHD, *vn = kn + GHD;
-  const float *kq = A.qkv + A.D + kvh * GHD;
-  const float qv = rope_at(A, A.qkv + h * GHD, lane, pos);
+  const float *qkv = A.qkv + (size_t)tok * (A.D + 2 * A.NKV * GHD), *kq = qkv + A.D + kvh * GHD;
+  const float qv = rope_at(A, qkv + h * GHD, lane, pos);
   float kv = rope_at(A, kq, lane, pos), vv = kq[A.NKV * GHD + lane];
   const int grp = lane >> 4, d4 = 4 * (lane & 15);
   uint4 kr[GAK / 4], vr[GAK / 4];
@@ -510,7 +518,8 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
       }
     }
   }
-  const bool writes = h % rep == 0 && pos >= k0 && pos < k0 + GAK;  // uniform in the wave
+  // (passes of several tokens: k_g_kv has written them)
+  const bool writes = gridDim.z == 1 && h % rep == 0 && pos >= k0 && pos < k0 + GAK;  // uniform in the wave
   if (F16) {
     const __half kh = __float2half_rn(kv), vh = __float2half_rn(vv);
     kv = __half2float(kh);
@@ -590,11 +599,29 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
     l = __builtin_fmaf(part[w][GHD + 1], f, l);
     out = __builtin_fmaf(part[w][lane], f, out);
   }
-  float *p = A.attp + ((size_t)h * gridDim.y + blockIdx.y) * GAPS;
+  float *p = A.attp + (((size_t)tok * A.NH + h) * gridDim.y + blockIdx.y) * GAPS;
   p[4 + lane] = out;
   if (lane == 0) {
     p[0] = mx;
     p[1] = l;
+  }
+}
+
+// A pass of several tokens: their k and v rows to the cache before the
+// attention, whose later tokens read the earlier ones' from there (a
+// workgroup's 64 lanes: one KV head of one token).
+template <bool F16>
+__global__ __launch_bounds__(GHD) void k_g_kv(GArgs A, int li) {
+  const int kvh = blockIdx.x, tok = blockIdx.y, pos = A.cur->pos + tok, lane = tid();
+  const float *kq = A.qkv + (size_t)tok * (A.D + 2 * A.NKV * GHD) + A.D + kvh * GHD;
+  const float kv = rope_at(A, kq, lane, pos), vv = kq[A.NKV * GHD + lane];
+  const size_t kb = g_kv_index(A, li, 0, kvh, pos) + lane, vb = g_kv_index(A, li, 1, kvh, pos) + lane;
+  if (F16) {
+    reinterpret_cast<__half *>(A.kv)[kb] = __float2half_rn(kv);
+    reinterpret_cast<__half *>(A.kv)[vb] = __float2half_rn(vv);
+  } else {
+    reinterpret_cast<float *>(A.kv)[kb] = kv;
+    reinterpret_cast<float *>(A.kv)[vb] = vv;
   }
 }
 
@@ -607,7 +634,7 @@ __global__ __launch_bounds__(GAT) void k_g_argmax(GArgs A) {
   extern __shared__ int lists[];
   GCursor *cur = A.cur;
   if (stopped(cur)) return;
-  const int row = cur->rows ? cur->i : 0, chained = cur->chain;
+  const int row = (cur->rows ? cur->i : 0) + (int)blockIdx.x, chained = cur->chain;
   const float *lg = A.logits + (size_t)row * A.V;
   const bool rule = chained && cur->gpt2_rule;
   int *nb = lists, *nr = lists + 1, *rec = lists + 2, *ban = lists + 34;
@@ -707,7 +734,7 @@ void launch_kind(GemvArgs a, hipStream_t s) {
   // wave: beyond that they would read more input than weights)
   a.rp = std::max(1, (groups + 4095) / 4096);
   const int waves = (groups + a.rp - 1) / a.rp;
-  hipLaunchKernelGGL((k_g_gemv<KIND, EPI, NORM>), dim3((waves + GT / 64 - 1) / (GT / 64)), dim3(GT),
+  hipLaunchKernelGGL((k_g_gemv<KIND, EPI, NORM>), dim3((waves + GT / 64 - 1) / (GT / 64), a.m), dim3(GT),
                      NORM == GN_SPLITS ? sizeof(float) * a.W.cols : 0, s, a);
 }
 
@@ -725,8 +752,10 @@ void launch_gemv(const GemvArgs &a, hipStream_t s) {
 }
 
 GemvArgs gemv_args(const GMat &W, const float *x, const float *gains, float eps, const float *bias, float *y,
-                   const GCursor *cur) {
+                   const GCursor *cur, int m = 1, int xs = 0) {
   GemvArgs a{};
+  a.m = m;
+  a.xs = xs;
   a.W = W;
   a.x = x;
   a.gains = gains;
@@ -760,51 +789,49 @@ int g_gemv(const GMat &W, const float *x, float *y, hipStream_t s) {
   return 0;
 }
 
-int g_head(const GArgs &A, const float *x, hipStream_t s) {
-  GemvArgs f = gemv_args(A.lm, x, A.norm_f, A.eps, nullptr, A.logits, A.cur);
+int g_head(const GArgs &A, const float *x, int m, hipStream_t s) {
+  GemvArgs f = gemv_args(A.lm, x, A.norm_f, A.eps, nullptr, A.logits, A.cur, m, A.D);
   f.lm = 1;
   if (A.arch == 1)
     launch_gemv<G_STORE, GN_LN>(f, s);
   else
     launch_gemv<G_STORE, GN_RMS>(f, s);
-  hipLaunchKernelGGL(k_g_argmax, dim3(1), dim3(GAT), sizeof(int) * (34 + (size_t)A.max_seq), s, A);
+  hipLaunchKernelGGL(k_g_argmax, dim3(m), dim3(GAT), sizeof(int) * (34 + (size_t)A.max_seq), s, A);
   MLLM_HIP(hipGetLastError());
   return 0;
 }
 
-int g_step(const GArgs &A, bool lm, hipStream_t s) {
+int g_step(const GArgs &A, bool lm, int m, hipStream_t s) {
   const bool gpt2 = A.arch == 1;
   const GCursor *cur = A.cur;
-  hipLaunchKernelGGL(k_g_embed, dim3(1), dim3(GT), 0, s, A);
+  hipLaunchKernelGGL(k_g_embed, dim3(m), dim3(GT), 0, s, A);
   const int nsplit = (A.max_seq + GSPLIT - 1) / GSPLIT;
   for (int li = 0; li < A.L; ++li) {
     const GLayer &w = A.layers[li];
     if (!(w.dbg & 1)) {
-      GemvArgs q = gemv_args(w.qkv, A.x, w.n1, A.eps, w.qkv_b, A.qkv, cur);
+      GemvArgs q = gemv_args(w.qkv, A.x, w.n1, A.eps, w.qkv_b, A.qkv, cur, m, A.D);
       if (gpt2)
         launch_gemv<G_STORE, GN_LN>(q, s);
       else
         launch_gemv<G_STORE, GN_RMS>(q, s);
-      if (A.kv_fp16)
-        hipLaunchKernelGGL(k_g_attn<true>, dim3(A.NH, nsplit), dim3(GAW * 64), 0, s, A, li);
-      else
-        hipLaunchKernelGGL(k_g_attn<false>, dim3(A.NH, nsplit), dim3(GAW * 64), 0, s, A, li);
-      GemvArgs o = gemv_args(w.proj, A.attp, nullptr, 0.f, w.proj_b, A.x, cur);
+      if (m > 1) hipLaunchKernelGGL(A.kv_fp16 ? k_g_kv<true> : k_g_kv<false>, dim3(A.NKV, m), dim3(GHD), 0, s, A, li);
+      hipLaunchKernelGGL(A.kv_fp16 ? k_g_attn<true> : k_g_attn<false>, dim3(A.NH, nsplit, m), dim3(GAW * 64), 0, s, A, li);
+      GemvArgs o = gemv_args(w.proj, A.attp, nullptr, 0.f, w.proj_b, A.x, cur, m, A.NH * nsplit * GAPS);
       o.nsplit_max = nsplit;
       launch_gemv<G_RESID, GN_SPLITS>(o, s);
     }
     if (!(w.dbg & 2)) {
       if (gpt2) {
-        launch_gemv<G_GELU, GN_LN>(gemv_args(w.w1, A.x, w.n2, A.eps, w.fc_b, A.h, cur), s);
+        launch_gemv<G_GELU, GN_LN>(gemv_args(w.w1, A.x, w.n2, A.eps, w.fc_b, A.h, cur, m, A.D), s);
       } else {
-        GemvArgs u = gemv_args(w.w1, A.x, w.n2, A.eps, nullptr, A.h, cur);
+        GemvArgs u = gemv_args(w.w1, A.x, w.n2, A.eps, nullptr, A.h, cur, m, A.D);
         u.W3 = w.w3;
         launch_gemv<G_SWIGLU, GN_RMS>(u, s);
       }
-      launch_gemv<G_RESID, GN_NONE>(gemv_args(w.w2, A.h, nullptr, 0.f, w.mproj_b, A.x, cur), s);
+      launch_gemv<G_RESID, GN_NONE>(gemv_args(w.w2, A.h, nullptr, 0.f, w.mproj_b, A.x, cur, m, A.FF), s);
     }
   }
-  if (lm) return g_head(A, A.x, s);
+  if (lm) return g_head(A, A.x, m, s);
   MLLM_HIP(hipGetLastError());
   return 0;
 }

@@ -273,6 +273,9 @@ __global__ __launch_bounds__(64 * GPW) void k_gp_gemm(GpArgs A, GpGemm G) {
         const int kvh = is_k ? head - A.NH : head - A.NH - A.NKV;
         const size_t k = ((((size_t)G.li * 2 + (is_k ? 0 : 1)) * A.NKV + kvh) * A.max_seq + pos) * GPHD + 4 * c;
         if (A.kv_fp16) {
+          // the cache holds the float32 value rounded: not formed in one rounding
+#pragma unroll
+          for (int e = 0; e < 4; ++e) asm("" : "+v"(y[e]));
           const __half2 a = __floats2half2_rn(y[0], y[1]), b = __floats2half2_rn(y[2], y[3]);
           *reinterpret_cast<uint2 *>(reinterpret_cast<__half *>(A.kv) + k) =
               make_uint2(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b));

@@ -77,3 +77,30 @@ def test_argmax_vs_logits(vocab):
         lg = g.forwardPrompt([t, 1]) if t == 0 else g.forwardDecode(t)
         assert g.last_argmax == int(np.argmax(lg))
     g.destroy()
+
+
+@gpu
+@pytest.mark.parametrize("kind", ["f32", "f16", "q8", "q8g32", "q4"])
+@pytest.mark.parametrize("arch,kv_fp16", [("llama", False), ("llama", True), ("gpt2", False)])
+def test_verify_pass_rows_bit_identical_to_decode(arch, kv_fp16, kind):
+    """A pass of 2, 7 and 16 tokens over an attention split's edge, rows in and
+    past a lane's registers: logits, argmax and the cache it leaves (read by the
+    next decode) as single steps give them, bit for bit."""
+    h = 6
+    bundle = build(arch, 54, kind=kind, group=64, n_layers=2, vocab_size=700, d_model=64 * h, n_heads=h,
+                   n_kv_heads=h if arch == "gpt2" else 2, d_ff=4160, max_seq_len=300,
+                   **({"bias_std": 0.02} if arch == "gpt2" else {}))
+    g = mllm.PetitGPT(bundle, kv_fp16=kv_fp16)
+    ids = [int(v) for v in np.random.default_rng(55).integers(0, 700, 280)]
+    print(f"verify {arch} {kind} fp16={kv_fp16}", flush=True)
+    for n, m in ((2, 2), (30, 7), (250, 16)):
+        g.forwardPrompt(ids[:n])
+        am, lg = g.forwardVerify(ids[n:n + m], want_logits=True)
+        after = g.forwardDecode(ids[n + m]).copy()
+        g.cacheLen = n
+        for i in range(m):
+            row = g.forwardDecode(ids[n + i])
+            assert np.array_equal(row.view(np.uint32), lg[i].view(np.uint32)), (n, m, i)
+            assert am[i] == g.last_argmax
+        assert np.array_equal(after.view(np.uint32), g.forwardDecode(ids[n + m]).view(np.uint32))
+    g.destroy()
