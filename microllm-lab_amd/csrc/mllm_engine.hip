@@ -132,6 +132,42 @@ struct PassState {
   int res[MAXT];  // argmax per lm row
 };
 
+// A call's inputs and outputs cross between host and device in these kernels.
+// What a call starts from is a kernel argument, and its outputs are stored to
+// pinned host memory from the device, behind the pass in the same stream, so
+// that the host waits once.  Copies by the runtime, each of them awaited (the
+// state's or the ids' from host memory, error flags, logits, argmax), cost 45 to
+// 60 us a call more: a five-row verify pass of the 135M Q4 model 753 -> 705 us, a
+// per-row Q8 token of that shape 860 -> 822, a 33-token GPT-2 prompt 1022 -> 964,
+// 16 chained tokens 6737 -> 6648.
+__global__ __launch_bounds__(64) void k_put_state(PassState s, PassState *to) {
+  if (threadIdx.x == 0) *to = s;
+}
+
+struct GCall {
+  GCursor c;
+  int n, ids[kGenericTokens];
+};
+__global__ __launch_bounds__(64) void k_put_cursor(GCall s, GCursor *to, int *ids) {
+  if (threadIdx.x) return;
+  *to = s.c;
+#pragma unroll
+  for (int t = 0; t < kGenericTokens; ++t)
+    if (t < s.n) ids[t] = s.ids[t];
+}
+
+__global__ __launch_bounds__(256) void k_fetch(const uint32_t *a, unsigned na, const uint32_t *b, unsigned nb,
+                                               uint32_t *out) {
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i < na)
+    out[i] = a[i];
+  else if (i - na < nb)
+    out[i] = b[i - na];
+}
+
+// Words before the logits in the host's copy of a call's outputs.
+constexpr size_t kOutHead = sizeof(PassState) / 4 > MAXT ? sizeof(PassState) / 4 : MAXT;
+
 struct DecParams {
   int arch, L, D, NH, NKV, FF, V, max_seq, kv_fp16, nsplit_max, nchunk;
   float eps, attn_scale;
@@ -2862,7 +2898,9 @@ struct mllm_model {
   float *d_logits = nullptr;
   int *d_hist = nullptr;
   PassState *d_st = nullptr;
-  PassState *h_st = nullptr;  // pinned
+  PassState h_st = {};  // the state that the next pass starts from
+  uint32_t *h_out = nullptr;  // pinned: a call's outputs
+  size_t h_out_words = 0;
   float *d_gemv_x = nullptr, *d_gemv_y = nullptr;
   DecParams P{};
   int cache_len = 0;
@@ -2906,7 +2944,6 @@ struct mllm_model {
   // their batched prompts (mllm_gprompt.hip): gp.tc = 0 where there are none
   GpArgs gp{};
   std::vector<GpLayer> gp_layer;
-  GCursor *h_gcur = nullptr;         // pinned: the cursor a call starts from
   hipGraphExec_t g_graph[2] = {};    // one step without / with the lm_head (exec mode 1)
 };
 
@@ -3013,8 +3050,29 @@ int get_f32(mllm_model *M, const std::string &n, size_t count, const float **out
 int upload_state(mllm_model *M) {
   // kernel-per-phase passes tag their handoff values below every tag a later
   // persistent launch waits for (its epochs start at flow_epoch + 1)
-  M->h_st->tag0 = (int)((uint32_t)M->flow_epoch * (uint32_t)TAGL);
-  MLLM_HIP(hipMemcpyAsync(M->d_st, M->h_st, sizeof(PassState), hipMemcpyHostToDevice, M->stream));
+  M->h_st.tag0 = (int)((uint32_t)M->flow_epoch * (uint32_t)TAGL);
+  hipLaunchKernelGGL(k_put_state, dim3(1), dim3(64), 0, M->stream, M->h_st, M->d_st);
+  MLLM_HIP(hipGetLastError());
+  return 0;
+}
+
+// Enqueues the copy of a call's outputs, na words of a and nb of b, to
+// M->h_out; they are there once the stream is synchronised.
+int fetch(mllm_model *M, const void *a, size_t na, const void *b, size_t nb) {
+  if (na + nb > M->h_out_words) return set_error(MLLM_ERR_INVALID, "outputs of %zu words", na + nb);
+  hipLaunchKernelGGL(k_fetch, dim3((unsigned)((na + nb + 255) / 256)), dim3(256), 0, M->stream,
+                     static_cast<const uint32_t *>(a), (unsigned)na, static_cast<const uint32_t *>(b), (unsigned)nb,
+                     M->h_out);
+  MLLM_HIP(hipGetLastError());
+  return 0;
+}
+
+// Pinned room for the outputs of any call: the pass state or the rows'
+// argmaxima, then the logits rows or the chained ids.
+int alloc_outputs(mllm_model *M) {
+  M->h_out_words = kOutHead + std::max((size_t)MAXT * M->cfg.vocab_size, (size_t)M->cfg.max_seq_len + 1);
+  if (hipHostMalloc((void **)&M->h_out, M->h_out_words * 4, hipHostMallocDefault) != hipSuccess)
+    return set_error(MLLM_ERR_HIP, "pinned outputs");
   return 0;
 }
 
@@ -3110,8 +3168,8 @@ int launch_flow(mllm_model *M, int steps) {
   void *args[] = {&M->P, &F};
   // k_flow3<false> while every position of the chain lies in the first
   // attention split (no split merges), k_flow3<true> past it
-  const FlowKernel kern = !use_flow3(M, M->h_st->pos0)               ? kFlowKernels[M->aq_idx]
-                          : M->h_st->pos0 + steps - 1 < ACH ? k_flow3<false>
+  const FlowKernel kern = !use_flow3(M, M->h_st.pos0)               ? kFlowKernels[M->aq_idx]
+                          : M->h_st.pos0 + steps - 1 < ACH ? k_flow3<false>
                                                                       : k_flow3<true>;
   if (M->exec_mode == 4) {
     // the same kernel and grid through an ordinary launch (profilers that do
@@ -3220,21 +3278,22 @@ int enqueue_pass_phases(mllm_model *M, int m, bool lm) {
   return 0;
 }
 
-int check_device_err(mllm_model *M) {
-  int err[2] = {0, 0};
-  MLLM_HIP(hipMemcpy(err, &M->d_st->err, sizeof(err), hipMemcpyDeviceToHost));
-  if (err[0] || err[1]) {
+// The error flags of the pass state that fetch() brought to M->h_out.
+int check_device_err(mllm_model *M, PassState *st) {
+  memcpy(st, M->h_out, sizeof *st);
+  if (st->err || st->bad_tok) {
     int zero[2] = {0, 0};
     MLLM_HIP(hipMemcpy(&M->d_st->err, zero, sizeof(zero), hipMemcpyHostToDevice));
-    return set_error(MLLM_ERR_DEVICE, err[0] ? "decode kernel reported an error"
-                                             : "chained decode produced no finite maximum logit");
+    return set_error(MLLM_ERR_DEVICE, st->err ? "decode kernel reported an error"
+                                              : "chained decode produced no finite maximum logit");
   }
   return 0;
 }
 
 // Run one pass of m tokens starting at pos0.  lm_rows: 0 none, 1 last, 2 all.
-int run_pass(mllm_model *M, const int32_t *ids, int m, int pos0, int lm_rows) {
-  PassState &s = *M->h_st;
+// logits / argmax, where given: of those rows.
+int run_pass(mllm_model *M, const int32_t *ids, int m, int pos0, int lm_rows, float *logits, int32_t *argmax) {
+  PassState &s = M->h_st;
   memset(&s, 0, sizeof s);
   s.pos0 = pos0;
   s.ntok = m;
@@ -3250,10 +3309,17 @@ int run_pass(mllm_model *M, const int32_t *ids, int m, int pos0, int lm_rows) {
   if (rc == kFlowFellBack) rc = enqueue_pass_phases(M, m, lm_rows != 0);
   if (rc) return rc;
   MLLM_HIP(hipEventRecord(M->ev1, M->stream));
+  const int row = lm_rows == 2 ? 0 : m - 1, nrows = m - row;
+  const size_t words = logits ? (size_t)nrows * M->cfg.vocab_size : 0;
+  if (int rf = fetch(M, M->d_st, sizeof(PassState) / 4, M->d_logits + (size_t)row * M->cfg.vocab_size, words)) return rf;
   MLLM_HIP(hipStreamSynchronize(M->stream));
   MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
   M->last_tokens = m;
-  return check_device_err(M);
+  PassState out;
+  if (int re = check_device_err(M, &out)) return re;
+  if (logits) memcpy(logits, M->h_out + sizeof(PassState) / 4, words * 4);
+  if (argmax) memcpy(argmax, &out.res[row], sizeof(int32_t) * nrows);
+  return 0;
 }
 
 int check_ids(const mllm_model *M, const int32_t *ids, int n) {
@@ -3480,7 +3546,7 @@ int generic_create(mllm_model *M) {
   if (rc) return rc;
   MLLM_HIP(hipMemset(A.kv, 0, kv_bytes));
   MLLM_HIP(hipMemset(A.cur, 0, sizeof(GCursor)));
-  MLLM_HIP(hipHostMalloc((void **)&M->h_gcur, sizeof(GCursor), hipHostMallocDefault));
+  if (int ro = alloc_outputs(M)) return ro;
   A.logits = M->d_logits;
   A.ids = M->d_ids;
   A.hist = M->d_hist;
@@ -3671,8 +3737,7 @@ extern "C" int mllm_model_create(const mllm_config *cfg, const void *payload, ui
   if (!rc) rc = dev_alloc(M, (void **)&M->d_gemv_x, sizeof(float) * std::max(FF, D) * 4);
   if (!rc) rc = dev_alloc(M, (void **)&M->d_gemv_y, sizeof(float) * std::max((size_t)V, (size_t)std::max(FF, D + 2 * kvd)));
   if (rc) return fail(rc);
-  if (hipHostMalloc((void **)&M->h_st, sizeof(PassState), hipHostMallocDefault) != hipSuccess)
-    return fail(set_error(MLLM_ERR_HIP, "pinned state"));
+  if ((rc = alloc_outputs(M))) return fail(rc);
   if (hipMemset(M->d_st, 0, sizeof(PassState)) != hipSuccess ||
       hipMemset(P.xa, 0, tagged_bytes[0]) != hipSuccess || hipMemset(P.xb, 0, tagged_bytes[1]) != hipSuccess ||
       hipMemset(P.opart, 0, tagged_bytes[2]) != hipSuccess || hipMemset(P.dpart, 0, tagged_bytes[3]) != hipSuccess ||
@@ -3875,9 +3940,8 @@ extern "C" int mllm_model_destroy(mllm_model *M) {
   if (M->chain_graph) hipGraphExecDestroy(M->chain_graph);
   for (hipGraphExec_t &ge : M->g_graph)
     if (ge) hipGraphExecDestroy(ge);
-  if (M->h_gcur) hipHostFree(M->h_gcur);
+  if (M->h_out) hipHostFree(M->h_out);
   for (void *p : M->allocs) hipFree(p);
-  if (M->h_st) hipHostFree(M->h_st);
   for (hipEvent_t e : M->prof_ev) (void)hipEventDestroy(e);
   if (M->ev0) hipEventDestroy(M->ev0);
   if (M->ev1) hipEventDestroy(M->ev1);
@@ -4007,21 +4071,13 @@ extern "C" int mllm_set_prefill(mllm_model *M, int min_tokens, int chunk_tokens)
 
 extern "C" uint64_t mllm_model_device_bytes(const mllm_model *M) { return M ? M->device_bytes : 0; }
 
-static int fetch_outputs(mllm_model *M, int row, int nrows, float *logits, int32_t *argmax) {
-  if (logits)
-    MLLM_HIP(hipMemcpy(logits, M->d_logits + (size_t)row * M->cfg.vocab_size,
-                       sizeof(float) * (size_t)nrows * M->cfg.vocab_size, hipMemcpyDeviceToHost));
-  if (argmax) MLLM_HIP(hipMemcpy(argmax, &M->d_st->res[row], sizeof(int32_t) * nrows, hipMemcpyDeviceToHost));
-  return 0;
-}
-
 // The kind-generic step: a call writes the cursor it starts from, then
 // enqueues one step per token -- replayed from a captured graph (exec mode
-// 1) or launched directly (mode 2).
+// 1) or launched directly (mode 2) -- or one verify pass.
 static int g_begin(mllm_model *M, const int32_t *ids, int n, int pos0, int chain, int rows, int first, int n_hist,
                    int eos) {
-  GCursor &c = *M->h_gcur;
-  memset(&c, 0, sizeof c);
+  GCall call = {};
+  GCursor &c = call.c;
   c.pos_next = pos0;
   c.pos = pos0;
   c.chain = chain;
@@ -4030,8 +4086,14 @@ static int g_begin(mllm_model *M, const int32_t *ids, int n, int pos0, int chain
   c.n_hist = n_hist;
   c.eos = eos;
   c.gpt2_rule = M->cfg.arch == 1;
-  MLLM_HIP(hipMemcpyAsync(M->g.cur, &c, sizeof c, hipMemcpyHostToDevice, M->stream));
-  if (ids) MLLM_HIP(hipMemcpyAsync(M->d_ids, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, M->stream));
+  if (ids && n <= kGenericTokens) {
+    call.n = n;
+    memcpy(call.ids, ids, sizeof(int32_t) * n);
+  } else if (ids) {
+    MLLM_HIP(hipMemcpyAsync(M->d_ids, ids, sizeof(int32_t) * n, hipMemcpyHostToDevice, M->stream));
+  }
+  hipLaunchKernelGGL(k_put_cursor, dim3(1), dim3(64), 0, M->stream, call, M->g.cur, M->d_ids);
+  MLLM_HIP(hipGetLastError());
   return 0;
 }
 
@@ -4058,6 +4120,20 @@ static int g_enqueue(mllm_model *M, bool lm) {
   return 0;
 }
 
+// The end of a call on generic kernels: nr logits rows and argmaxima.
+static int g_finish(mllm_model *M, int n, int nr, float *logits, int32_t *argmax) {
+  const size_t words = logits ? (size_t)nr * M->cfg.vocab_size : 0;
+  MLLM_HIP(hipEventRecord(M->ev1, M->stream));
+  if (logits || argmax)
+    if (int rc = fetch(M, M->g.res, nr, M->d_logits, words)) return rc;
+  MLLM_HIP(hipStreamSynchronize(M->stream));
+  MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
+  M->last_tokens = n;
+  if (argmax) memcpy(argmax, M->h_out, sizeof(int32_t) * nr);
+  if (logits) memcpy(logits, M->h_out + nr, words * 4);
+  return 0;
+}
+
 // ids[0..n) at positions pos0..: logits and argmax of every row (rows:
 // verify) or of the last token only.
 static int g_run(mllm_model *M, const int32_t *ids, int n, int pos0, bool rows, float *logits, int32_t *argmax) {
@@ -4069,15 +4145,7 @@ static int g_run(mllm_model *M, const int32_t *ids, int n, int pos0, bool rows, 
     for (int t = 0; t < n; ++t)
       if (int rc = g_enqueue(M, rows || t == n - 1)) return rc;
   }
-  MLLM_HIP(hipEventRecord(M->ev1, M->stream));
-  MLLM_HIP(hipStreamSynchronize(M->stream));
-  MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
-  M->last_tokens = n;
-  const int nr = rows ? n : 1;
-  if (logits)
-    MLLM_HIP(hipMemcpy(logits, M->d_logits, sizeof(float) * (size_t)nr * M->cfg.vocab_size, hipMemcpyDeviceToHost));
-  if (argmax) MLLM_HIP(hipMemcpy(argmax, M->g.res, sizeof(int32_t) * nr, hipMemcpyDeviceToHost));
-  return 0;
+  return g_finish(M, n, rows ? n : 1, logits, argmax);
 }
 
 // A prompt of a kind-generic model through the batched path, in chunks.
@@ -4090,13 +4158,7 @@ static int g_prompt(mllm_model *M, const int32_t *ids, int n, float *logits, int
     if (int rc = gp_layers(M->gp, ids + p0, m, p0, p0 + m == n, &row, M->stream)) return rc;
   }
   if (int rc = g_head(M->g, row, 1, M->stream)) return rc;
-  MLLM_HIP(hipEventRecord(M->ev1, M->stream));
-  MLLM_HIP(hipStreamSynchronize(M->stream));
-  MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
-  M->last_tokens = n;
-  if (logits) MLLM_HIP(hipMemcpy(logits, M->d_logits, sizeof(float) * (size_t)M->cfg.vocab_size, hipMemcpyDeviceToHost));
-  if (argmax) MLLM_HIP(hipMemcpy(argmax, M->g.res, sizeof(int32_t), hipMemcpyDeviceToHost));
-  return 0;
+  return g_finish(M, n, 1, logits, argmax);
 }
 
 extern "C" int mllm_forward_prompt(mllm_model *M, const int32_t *ids, int n, float *logits, int32_t *argmax) {
@@ -4119,21 +4181,24 @@ extern "C" int mllm_forward_prompt(mllm_model *M, const int32_t *ids, int n, flo
       if (int rc = pf_layers(M->pf, ids + p0, m, p0, p0 + m == n, M->stream)) return rc;
     }
     MLLM_HIP(hipEventRecord(M->ev1, M->stream));
+    const size_t words = logits ? (size_t)M->cfg.vocab_size : 0;
+    if (logits || argmax)
+      if (int rc = fetch(M, M->d_st->res, 1, M->d_logits, words)) return rc;
     MLLM_HIP(hipStreamSynchronize(M->stream));
     MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev_pf, M->ev1));
     M->last_tokens = n;
     M->cache_len = n;
-    return fetch_outputs(M, 0, 1, logits, argmax);
+    if (argmax) memcpy(argmax, M->h_out, sizeof(int32_t));
+    if (logits) memcpy(logits, M->h_out + 1, words * 4);
+    return 0;
   }
-  int last_rows = 0;
   for (int p0 = 0; p0 < n; p0 += M->max_pass) {
     const int m = std::min(M->max_pass, n - p0);
     const bool last = p0 + m == n;
-    if (int rc = run_pass(M, ids + p0, m, p0, last ? 1 : 0)) return rc;
-    last_rows = m;
+    if (int rc = run_pass(M, ids + p0, m, p0, last ? 1 : 0, last ? logits : nullptr, last ? argmax : nullptr)) return rc;
   }
   M->cache_len = n;
-  return fetch_outputs(M, last_rows - 1, 1, logits, argmax);
+  return 0;
 }
 
 extern "C" int mllm_forward_decode(mllm_model *M, int32_t id, float *logits, int32_t *argmax) {
@@ -4145,9 +4210,9 @@ extern "C" int mllm_forward_decode(mllm_model *M, int32_t id, float *logits, int
     M->cache_len += 1;
     return 0;
   }
-  if (int rc = run_pass(M, &id, 1, M->cache_len, 1)) return rc;
+  if (int rc = run_pass(M, &id, 1, M->cache_len, 1, logits, argmax)) return rc;
   M->cache_len += 1;
-  return fetch_outputs(M, 0, 1, logits, argmax);
+  return 0;
 }
 
 extern "C" int mllm_forward_verify(mllm_model *M, const int32_t *ids, int n, int32_t *argmax, float *logits) {
@@ -4160,9 +4225,9 @@ extern "C" int mllm_forward_verify(mllm_model *M, const int32_t *ids, int n, int
     M->cache_len += n;
     return 0;
   }
-  if (int rc = run_pass(M, ids, n, M->cache_len, 2)) return rc;
+  if (int rc = run_pass(M, ids, n, M->cache_len, 2, logits, argmax)) return rc;
   M->cache_len += n;
-  return fetch_outputs(M, 0, n, logits, argmax);
+  return 0;
 }
 
 extern "C" int mllm_decode_chain(mllm_model *M, int32_t first, int n_steps, int32_t eos_id, const int32_t *hist,
@@ -4182,18 +4247,19 @@ extern "C" int mllm_decode_chain(mllm_model *M, int32_t first, int n_steps, int3
     for (int i = 0; i < n_steps; ++i)
       if (int rc = g_enqueue(M, true)) return rc;
     MLLM_HIP(hipEventRecord(M->ev1, M->stream));
+    if (int rc = fetch(M, M->g.cur, sizeof(GCursor) / 4, M->d_hist + n_hist, n_steps)) return rc;
     MLLM_HIP(hipStreamSynchronize(M->stream));
     MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
     GCursor c;
-    MLLM_HIP(hipMemcpy(&c, M->g.cur, sizeof c, hipMemcpyDeviceToHost));
+    memcpy(&c, M->h_out, sizeof c);
     MLLM_CHECK(c.emitted >= 1 && c.emitted <= n_steps, "chain emitted %d ids of %d steps", c.emitted, n_steps);
-    MLLM_HIP(hipMemcpy(out_ids, M->d_hist + n_hist, sizeof(int32_t) * c.emitted, hipMemcpyDeviceToHost));
+    memcpy(out_ids, M->h_out + sizeof(GCursor) / 4, sizeof(int32_t) * c.emitted);
     *n_out = c.emitted;
     M->last_tokens = c.emitted;
     M->cache_len += c.emitted;
     return 0;
   }
-  PassState &s = *M->h_st;
+  PassState &s = M->h_st;
   memset(&s, 0, sizeof s);
   s.pos0 = M->cache_len;
   s.ntok = 1;
@@ -4216,12 +4282,13 @@ extern "C" int mllm_decode_chain(mllm_model *M, int32_t first, int n_steps, int3
   }
   if (rc) return rc;
   MLLM_HIP(hipEventRecord(M->ev1, M->stream));
+  if (int rf = fetch(M, M->d_st, sizeof(PassState) / 4, M->d_hist + n_hist, n_steps)) return rf;
   MLLM_HIP(hipStreamSynchronize(M->stream));
   MLLM_HIP(hipEventElapsedTime(&M->last_ms, M->ev0, M->ev1));
-  if (int rc = check_device_err(M)) return rc;
-  MLLM_HIP(hipMemcpy(&s, M->d_st, sizeof(PassState), hipMemcpyDeviceToHost));
+  if (int re = check_device_err(M, &s)) return re;
   const int emitted = s.n_hist - n_hist;
-  MLLM_HIP(hipMemcpy(out_ids, M->d_hist + n_hist, sizeof(int32_t) * emitted, hipMemcpyDeviceToHost));
+  MLLM_CHECK(emitted >= 0 && emitted <= n_steps, "chain emitted %d ids of %d steps", emitted, n_steps);
+  memcpy(out_ids, M->h_out + sizeof(PassState) / 4, sizeof(int32_t) * emitted);
   *n_out = emitted;
   M->last_tokens = emitted;
   M->cache_len += emitted;
@@ -4241,7 +4308,7 @@ extern "C" int mllm_profile_decode(mllm_model *M, int32_t first, int n_steps, fl
     M->prof_ev.assign(2 * per_step, nullptr);
     for (auto &e : M->prof_ev) MLLM_HIP(hipEventCreate(&e));
   }
-  PassState &s = *M->h_st;
+  PassState &s = M->h_st;
   memset(&s, 0, sizeof s);
   s.pos0 = M->cache_len;
   s.ntok = 1;
@@ -4264,8 +4331,9 @@ extern "C" int mllm_profile_decode(mllm_model *M, int32_t first, int n_steps, fl
       cnt[phases[k].first] += 1;
     }
   }
-  if (int rc = check_device_err(M)) return rc;
-  MLLM_HIP(hipMemcpy(&s, M->d_st, sizeof(PassState), hipMemcpyDeviceToHost));
+  if (int rc = fetch(M, M->d_st, sizeof(PassState) / 4, M->d_st, 0)) return rc;
+  MLLM_HIP(hipStreamSynchronize(M->stream));
+  if (int rc = check_device_err(M, &s)) return rc;
   M->cache_len += n_steps;
   for (int ph = 0; ph < PH_COUNT; ++ph) phase_us[ph] = cnt[ph] ? (float)(sum[ph] / cnt[ph] * 1000.0) : 0.f;
   return 0;

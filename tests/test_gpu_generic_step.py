@@ -104,3 +104,41 @@ def test_verify_pass_rows_bit_identical_to_decode(arch, kv_fp16, kind):
             assert am[i] == g.last_argmax
         assert np.array_equal(after.view(np.uint32), g.forwardDecode(ids[n + m]).view(np.uint32))
     g.destroy()
+
+
+@gpu
+@pytest.mark.parametrize("kind", ["q4", "q8"])
+@pytest.mark.parametrize("vocab", [64, 641])
+def test_outputs_of_every_call_shape(kind, vocab):
+    """Both engines' outputs at the host: 1 to 16 rows, with and without the
+    logits or the argmax, after larger calls and chains of every short length."""
+    import ctypes as C
+    from mllm import abi
+    g = mllm.PetitGPT(build("llama", 57, kind=kind, n_layers=2, vocab_size=vocab, max_seq_len=64))
+    ids = [int(v) for v in np.random.default_rng(58).integers(0, vocab, 64)]
+    print(f"outputs {kind} V={vocab}", flush=True)
+    rows = np.empty((40, vocab), np.float32)
+    g.forwardPrompt(ids[:4])
+    for i in range(40):
+        rows[i] = g.forwardDecode(ids[4 + i])
+        assert g.last_argmax == int(rows[i].argmax())
+    for m in (16, 1, 2, 15, 3):
+        g.cacheLen = 4
+        am, lg = g.forwardVerify(ids[4:4 + m], want_logits=True)
+        assert np.array_equal(lg.view(np.uint32), rows[:m].view(np.uint32)) and am == [int(v) for v in rows[:m].argmax(1)]
+        g.cacheLen = 4
+        assert g.forwardVerify(ids[4:4 + m])[0] == am
+    a = np.array(ids[:5], np.int32)
+    for call, lead in (("mllm_forward_decode", (ids[4],)), ("mllm_forward_prompt", (a.ctypes.data, 5))):
+        out, am = np.zeros(vocab, np.float32), C.c_int32(-1)
+        for lp, ap in ((out.ctypes.data, None), (None, C.byref(am)), (None, None)):
+            g.cacheLen = 4
+            abi.call(call, g._h, *lead, lp, ap)
+            assert g.cacheLen == 5
+        assert am.value == int(out.argmax())
+    g.cacheLen = 4
+    chain = g.decodeChain(ids[4], 20)
+    for n in (1, 7, 19):
+        g.cacheLen = 4
+        assert g.decodeChain(ids[4], n) == chain[:n]
+    g.destroy()
