@@ -212,16 +212,18 @@ __global__ __launch_bounds__(WGT) void k_gemv_q4_batched(const uint8_t *const *_
 //         launch, but three device-scope round trips after the last tile -- the
 //         pair's store, the count, the pairs;
 //   else  by a second launch of one workgroup.
-// Measured, us a call, ONE and two launches: 63 tiles (4000 x 576) 5.9 and 6.6,
-// 250 tiles (16000 x 576) 8.0 and 6.7, 768 (49152 x 960) 15.6 and 10.0: the
-// round trips grow with the workgroups that contend for the counter, the second
-// launch costs the host 1.3 us.  kAmxTwo tiles and more take two launches.
+// Measured, us a call, ONE: 63 tiles (4000 x 576) 5.9, 250 (32000 x 320) 8.1, 332
+// (42402 x 320) 9.4, 500 (32000 x 576) 11.2, 663 (42402 x 576) 13.6, 768 (49152 x
+// 960) 15.6: the round trips grow with the workgroups that contend for the
+// counter.  Two launches: 6.6, 7.1, 7.7, 7.5, 8.3 and 9.7 where the host keeps up,
+// 10 to 11 for any of them where its two launches take that long.  kAmxTwo is
+// where two are no slower on either host.
 // Scratch layout (bytes): [0, 4) the counter, which every completed call leaves
 // at 0; [4, 8) row 0 is NaN (tile 0 writes it); [64, 64 + 4 ntiles) the tiles'
 // values, then ntiles rows.  Two calls that share a scratch buffer must not
 // overlap.
 constexpr size_t kAmxHead = 64;
-constexpr int kAmxTwo = 128;
+constexpr int kAmxTwo = 448;  // tiles from which there are two launches
 __host__ __device__ constexpr size_t amx_scratch_bytes(int ntiles) { return kAmxHead + 8 * (size_t)ntiles; }
 
 // The workgroup's first maximum, in thread 0.

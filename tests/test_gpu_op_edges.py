@@ -114,10 +114,10 @@ def test_gemv_f32_rows_per_wave(n):
 
 
 @gpu
-@pytest.mark.parametrize("rows", [16256, 16257, 16384, 16385])
+@pytest.mark.parametrize("rows", [57216, 57344, 57345])
 @pytest.mark.parametrize("kind", ["first of ties", "nan0", "nan rows", "all nan"])
 def test_argmax_on_both_sides_of_two_launches(rows, kind):
-    """128 rows a tile: 127 tiles (one launch) and 128 or 129 (two), called
+    """128 rows a tile: 447 tiles (one launch) and 448 or 449 (two), called
     twice on the same scratch, the index by infer.js:240-250."""
     rng = np.random.default_rng(rows)
     n = 64
