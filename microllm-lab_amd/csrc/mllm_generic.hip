@@ -502,11 +502,14 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
   float kv = rope_at(A, kq, lane, pos), vv = kq[A.NKV * GHD + lane];
   const int grp = lane >> 4, d4 = 4 * (lane & 15);
   uint4 kr[GAK / 4], vr[GAK / 4];
-  if (on) {
+  if (on && pos == 0) {  // no cached row: row 0 is an earlier call's, or being written
+#pragma unroll
+    for (int i = 0; i < GAK / 4; ++i) kr[i] = vr[i] = make_uint4(0u, 0u, 0u, 0u);
+  } else if (on) {
 #pragma unroll
     for (int i = 0; i < GAK / 4; ++i) {
       // rows at and past the new one are not used: a valid row in their place
-      const size_t off = (size_t)max(0, min(k0 + 4 * i + grp, pos - 1)) * GHD + d4;
+      const size_t off = (size_t)min(k0 + 4 * i + grp, pos - 1) * GHD + d4;
       if (F16) {
         const uint2 a = *reinterpret_cast<const uint2 *>(reinterpret_cast<const __half *>(A.kv) + kb + off);
         const uint2 b = *reinterpret_cast<const uint2 *>(reinterpret_cast<const __half *>(A.kv) + vb + off);
@@ -561,7 +564,10 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
 #pragma unroll
     for (int i = 0; i < GAK / 4; ++i) {
       const float p = expf(sc[i] - m);
-      const float4 v = k0 + 4 * i + grp == pos ? vl : row(vr[i]);
+      // a position past the new one has weight 0 and a value of 0: 0 times the
+      // row loaded in its place is NaN where that row holds an infinity
+      const int key = k0 + 4 * i + grp;
+      const float4 v = key < pos ? row(vr[i]) : key == pos ? vl : make_float4(0.f, 0.f, 0.f, 0.f);
       sum += p;
       o.x = __builtin_fmaf(p, v.x, o.x);
       o.y = __builtin_fmaf(p, v.y, o.y);

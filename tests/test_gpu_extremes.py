@@ -1,0 +1,63 @@
+"""The kind-generic models on values at the ends of float32's and f16's ranges:
+what one call leaves in the KV cache or computes for one token must not reach
+results that do not depend on it."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+import mllm
+from mllm import pgw
+
+gpu = pytest.mark.gpu
+A, B = 5, 9  # tokens: only A's embedding has component 0
+
+
+def bits(a):
+    return np.array(a, np.float32).view(np.uint32)
+
+
+def edited(arch, edit, seed=61, **kw):
+    """An f32 model whose matrices edit(w) changes in place; w(name): a matrix."""
+    model = {k: kw.pop(k) for k in ("bias_std", "std") if k in kw}
+    b = pgw.parse_pgw(pgw.make_model(pgw.small_config(arch, **kw), seed=seed, kind="f32", **model))
+    buf = bytearray(b.buffer)
+
+    def w(name):
+        t = b.tensors[name]
+        n = int(np.prod(t["shape"]))
+        return np.frombuffer(buf, np.float32, n, b.payload_off + t["offset"]).reshape(t["shape"])
+
+    edit(w)
+    return dataclasses.replace(b, buffer=bytes(buf))
+
+
+@gpu
+@pytest.mark.parametrize("kv_fp16", [False, True])
+@pytest.mark.parametrize("calls", ["prompt 1", "prompt 2", "verify"])
+def test_first_position_ignores_the_old_cache(calls, kv_fp16):
+    """Token A leaves an infinite value row (and NaN in the deeper layers) at
+    position 0.  Calls that start there again give a fresh model's bits."""
+    def edit(w):
+        w("lm_head")[:, 0] = 0.0
+        w("lm_head")[A, 0] = 1.0
+        v = w("blocks.0.attn.qkv")
+        v[192 + 64:, 0] = 3e38  # value rows: infinite for A, untouched for the others
+
+    bundle = edited("llama", edit, d_model=192, n_heads=3, n_kv_heads=1)
+    print(f"old cache {calls} fp16={kv_fp16}", flush=True)
+
+    def results(g):
+        if calls == "verify":
+            g.cacheLen = 0
+            return g.forwardVerify([B, 11, 12], want_logits=True)[1]
+        first = g.forwardPrompt([B] if calls == "prompt 1" else [B, 11]).copy()
+        return np.stack([first, g.forwardDecode(13).copy()])
+
+    fresh, used = (mllm.PetitGPT(bundle, kv_fp16=kv_fp16) for _ in range(2))
+    want = results(fresh)
+    assert np.isfinite(want).all()
+    assert not np.isfinite(used.forwardPrompt([A])).any()
+    assert np.array_equal(bits(results(used)), bits(want))
+    fresh.destroy()
+    used.destroy()
