@@ -146,6 +146,12 @@ struct GemvArgs {
   int m, xs;           // tokens of the pass and the stride of their inputs (outputs: W.rows)
 };
 
+// What a part of the keys subtracts from its scores: their maximum, or 0 where
+// all of them are -inf, so that these keys weigh exp(-inf) = 0 and not
+// exp(-inf + inf) = NaN.  (All keys of a row so: 0 / 0 at the end, as
+// infer.js:227-238 gives it.)
+__device__ __forceinline__ float score_ref(float mx) { return mx == -INFINITY ? 0.f : mx; }
+
 // The attention's output row from its splits' partials (infer.js:466-495) into
 // LDS: a thread per four components, its splits' loads four at a time.
 __device__ __forceinline__ void merge_splits(const GemvArgs &a, int tok, float *sx) {
@@ -166,11 +172,11 @@ __device__ __forceinline__ void merge_splits(const GemvArgs &a, int tok, float *
         u[k] = *reinterpret_cast<const float4 *>(q + 4 + 4 * (i & 15));
       }
       const float mn = fmaxf(mx, fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])));
-      const float f0 = expf(mx - mn);  // 0 at first
+      const float ref = score_ref(mn), f0 = expf(mx - ref);  // 0 at first
       l *= f0, o.x *= f0, o.y *= f0, o.z *= f0, o.w *= f0;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const float f = expf(m[k] - mn);
+        const float f = expf(m[k] - ref);
         l = __builtin_fmaf(ls[k], f, l);
         o.x = __builtin_fmaf(u[k].x, f, o.x), o.y = __builtin_fmaf(u[k].y, f, o.y);
         o.z = __builtin_fmaf(u[k].z, f, o.z), o.w = __builtin_fmaf(u[k].w, f, o.w);
@@ -560,10 +566,11 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
       m = fmaxf(m, sc[i]);
     }
     m = fmaxf(m, __shfl_xor(m, 16));
-    m = fmaxf(m, __shfl_xor(m, 32));  // finite: position k0 is in
+    m = fmaxf(m, __shfl_xor(m, 32));
+    const float ref = score_ref(m);
 #pragma unroll
     for (int i = 0; i < GAK / 4; ++i) {
-      const float p = expf(sc[i] - m);
+      const float p = expf(sc[i] - ref);
       // a position past the new one has weight 0 and a value of 0: 0 times the
       // row loaded in its place is NaN where that row holds an infinity
       const int key = k0 + 4 * i + grp;
@@ -595,13 +602,14 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
   }
   __syncthreads();
   if (wv != 0) return;
-  float mx = part[0][GHD];  // wave 0 has a position
+  float mx = part[0][GHD];
 #pragma unroll
   for (int w = 1; w < GAW; ++w) mx = fmaxf(mx, part[w][GHD]);
+  const float ref = score_ref(mx);
   float l = 0.f, out = 0.f;
 #pragma unroll
   for (int w = 0; w < GAW; ++w) {
-    const float f = expf(part[w][GHD] - mx);  // 0 for a wave without positions
+    const float f = expf(part[w][GHD] - ref);  // 0 for a wave without positions
     l = __builtin_fmaf(part[w][GHD + 1], f, l);
     out = __builtin_fmaf(part[w][lane], f, out);
   }

@@ -61,3 +61,40 @@ def test_first_position_ignores_the_old_cache(calls, kv_fp16):
     assert np.array_equal(bits(results(used)), bits(want))
     fresh.destroy()
     used.destroy()
+
+
+def rel(a, b):
+    return float(np.abs(a - b).max()) / float(np.abs(b).max())
+
+
+@gpu
+@pytest.mark.parametrize("n", [32, 256, 1024])
+@pytest.mark.parametrize("how", ["step"])
+def test_minus_infinite_scores_weigh_nothing(oracle_lib, how, n):
+    """The keys 0 .. n-1 are infinite in an f16 cache and score -inf for the last
+    token, whose own key is finite and alone in its 32 positions (n = 256: in its
+    256, n = 1024: in the fifth split).  They get weight 0, as in the oracle,
+    where the same scores are about -1e6."""
+    def edit(w):
+        w("lm_head")[:, 0] = 0.0
+        w("lm_head")[A, 0] = w("lm_head")[B, 0] = 1.0  # B too, so that its query has component 31
+        w("lm_head")[:, 1] = 0.0
+        w("lm_head")[A, 1] = 1.0
+        qkv = w("blocks.0.attn.qkv")
+        qkv[[31, 128 + 31]] = 0.0  # component 31 turns by less than 0.2 over 1100 positions
+        qkv[31, 0] = -1.0
+        qkv[128 + 31, 1] = 1e5     # A's keys only
+
+    bundle = edited("llama", edit, n_layers=1, max_seq_len=1100)
+    print(f"-inf scores {how} n={n}", flush=True)
+    g = mllm.PetitGPT(bundle, kv_fp16=True)
+    ref = oracle_lib.OracleModel(bundle)
+    if how == "step":
+        g.forwardPrompt([A] * n)
+        got = g.forwardDecode(B).copy()
+    else:
+        got = g.forwardPrompt([A] * n + [B]).copy()
+    want = ref.forward_prompt([A] * n + [B])
+    g.destroy()
+    ref.close()
+    assert rel(got, want) <= 5e-3  # the f16 cache
