@@ -16,7 +16,7 @@
 //   QKV    y = r_t (W (x g)): planes of x g from the kernel that formed x,
 //          r_t = 1 / sqrt(mean x^2 + eps) from that kernel's per-64-column
 //          sums; epilogue RoPE, q, K and V to the cache
-//   ATTN   mllm_prefill.hip's attention, its output written as planes
+//   ATTN   causal attention in float32, its output written as planes
 //   O      x += W_o o; planes of x g2 and the sums of squares of x
 //   UP     gate and up rows of the same units: silu(g) u as planes
 //   DOWN   x += W_2 h; planes of x g1' (the next layer's norm) and the sums
@@ -48,7 +48,6 @@
 #include "mllm_host.h"
 #include "mllm_kinds.h"
 #include "mllm_planes.h"
-#include "mllm_prefill.h"
 
 namespace mllm {
 namespace {
@@ -385,6 +384,198 @@ __global__ __launch_bounds__(WG) void k_gp_ln(GpArgs A, const float *g, int t0, 
   }
 }
 
+// ---------------------------------------------------------------- attention
+// Workgroup (32-query tile, query head), its 32-key blocks dealt round-robin to
+// GAS waves.  Per block, on the float32 matrix cores:
+//   S^T = K Q^T    v_mfma_f32_32x32x2_f32, A = the keys (lane: key j), B = the
+//                  queries; step (c, e) takes dimensions 8c + e and 8c + 4 + e
+//   O^T += V^T P^T A = the values (lane: dimension j), B = the weights straight
+//                  from the S^T registers: value v of lane half hh is key
+//                  8 (v / 4) + 4 hh + v % 4
+// so that a lane holds one query's scores and outputs, and a wave needs no LDS
+// until the end, where the waves' (outputs, max, sum) meet, in wave order, a
+// thread per four outputs.
+//
+// Float32 operands, sums, softmax weights and exponentials throughout, as in
+// k_g_attn: keys, values and queries of any magnitude keep their 24 bits.
+// (Halves of f16 pairs, as the Q4 prompts take them, end at 65504 and lose bits
+// below 2^-13.)
+constexpr int GAS = 8;
+
+// Cache elements as loaded: four components of a key, one of a value.
+template <bool F16>
+struct KvRaw;
+template <>
+struct KvRaw<false> {
+  typedef float4 K;
+  typedef float V;
+  static __device__ __forceinline__ float4 k4(const float4 &r) { return r; }
+  static __device__ __forceinline__ float f(float r) { return r; }
+};
+template <>
+struct KvRaw<true> {
+  typedef uint2 K;
+  typedef unsigned short V;
+  static __device__ __forceinline__ float4 k4(const uint2 &r) {
+    return make_float4(f16_bits(r.x & 0xffffu), f16_bits(r.x >> 16), f16_bits(r.y & 0xffffu), f16_bits(r.y >> 16));
+  }
+  static __device__ __forceinline__ float f(unsigned short r) { return f16_bits(r); }
+};
+constexpr size_t kAttnLds = sizeof(float) * GAS * (GPT + 64);
+
+__device__ __forceinline__ v16f mfma_f32(float a, float b, v16f c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
+// What a part of the keys subtracts from its scores: 0 where all are -inf (they
+// weigh 0; with the maximum itself they would weigh exp(-inf + inf) = NaN).
+__device__ __forceinline__ float score_ref(float mx) { return mx == -INFINITY ? 0.f : mx; }
+
+template <bool F16>
+__global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, int pos0, int tt0) {
+  extern __shared__ __attribute__((aligned(16))) float buf[];  // [GAS][GPT] outputs, [GAS][2][32] (max, sum)
+  const int T0 = (tt0 + (int)(gridDim.x - 1 - blockIdx.x)) * 32;  // the longest tiles first
+  const int hq = blockIdx.y, kvh = hq / (A.NH / A.NKV);
+  const int wv = __builtin_amdgcn_readfirstlane(tid() >> 6), lane = tid() & 63, j = lane & 31, hh = lane >> 5;
+  const int qpos = pos0 + T0 + j, qlast = pos0 + min(T0 + 32, n) - 1;  // last key any query of the tile sees
+  const int nb = (qlast >> 5) + 1, used = min(nb, GAS);
+  const size_t kb = (((size_t)li * 2) * A.NKV + kvh) * A.max_seq * GPHD, vb = kb + (size_t)A.NKV * A.max_seq * GPHD;
+  float4 q[8];
+  typename KvRaw<F16>::K kr[8];
+  typename KvRaw<F16>::V vr[2][16];
+  // keys past qlast are masked: a valid row in their place
+  auto load_k = [&](int b) {
+    const size_t at = kb + (size_t)min(32 * b + j, qlast) * GPHD + 4 * hh;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) kr[c] = static_cast<const typename KvRaw<F16>::K *>(A.kv)[(at + 8 * c) >> 2];
+  };
+  auto load_v = [&](int b) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const size_t at = vb + (size_t)min(32 * b + 8 * (v >> 2) + 4 * hh + (v & 3), qlast) * GPHD + j;
+      vr[0][v] = static_cast<const typename KvRaw<F16>::V *>(A.kv)[at];
+      vr[1][v] = static_cast<const typename KvRaw<F16>::V *>(A.kv)[at + 32];
+    }
+  };
+  {
+    const float *qr = A.q + (size_t)min(T0 + j, n - 1) * A.D + hq * GPHD + 4 * hh;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) q[c] = *reinterpret_cast<const float4 *>(qr + 8 * c);
+  }
+  if (wv < nb) {
+    load_k(wv);
+    load_v(wv);
+  }
+  float m = -INFINITY, l = 0.f;
+  v16f o[2];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) o[0][v] = o[1][v] = 0.f;
+  for (int b = wv; b < nb; b += GAS) {
+    v16f s;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) s[v] = 0.f;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float4 k = KvRaw<F16>::k4(kr[c]);
+      s = mfma_f32(k.x, q[c].x, s);
+      s = mfma_f32(k.y, q[c].y, s);
+      s = mfma_f32(k.z, q[c].z, s);
+      s = mfma_f32(k.w, q[c].w, s);
+    }
+    if (b + GAS < nb) load_k(b + GAS);
+    const bool masked = 32 * b + 31 > pos0 + T0;  // the block reaches past a query of the tile
+    float mx = m;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      s[v] *= A.attn_scale;
+      if (masked && 32 * b + 8 * (v >> 2) + 4 * hh + (v & 3) > qpos) s[v] = -INFINITY;
+      mx = fmaxf(mx, s[v]);
+    }
+    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    const float ref = score_ref(mx), alpha = expf(m - ref);
+    float ps = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      s[v] = expf(s[v] - ref);
+      ps += s[v];
+    }
+    l = l * alpha + (ps + __shfl_xor(ps, 32));
+    if (__any(mx != m)) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        o[0][v] *= alpha;
+        o[1][v] *= alpha;
+      }
+    }
+    m = mx;
+    bool whole = true;
+    if (masked) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) whole &= finite(KvRaw<F16>::f(vr[0][v])) && finite(KvRaw<F16>::f(vr[1][v]));
+    }
+    if (__all(whole)) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        o[0] = mfma_f32(KvRaw<F16>::f(vr[0][v]), s[v], o[0]);
+        o[1] = mfma_f32(KvRaw<F16>::f(vr[1][v]), s[v], o[1]);
+      }
+    } else {
+      // An infinity or NaN among the values of a block with masked keys: their
+      // weight is 0 and 0 times it NaN, in the rows of queries that do not see
+      // it.  It is left out of the products, and counted for the queries that
+      // do: those are NaN.
+      for (int d = 0; d < 2; ++d) {
+        v16f hit, sum = o[d];
+#pragma unroll
+        for (int v = 0; v < 16; ++v) hit[v] = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const float val = KvRaw<F16>::f(d == 0 ? vr[0][v] : vr[1][v]);
+          const bool sees = 32 * b + 8 * (v >> 2) + 4 * hh + (v & 3) <= qpos;
+          sum = mfma_f32(finite(val) ? val : 0.f, s[v], sum);
+          hit = mfma_f32(finite(val) ? 0.f : 1.f, sees ? 1.f : 0.f, hit);
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const float r = hit[v] > 0.f ? NAN : sum[v];
+          if (d == 0) o[0][v] = r;
+          else o[1][v] = r;
+        }
+      }
+    }
+    if (b + GAS < nb) load_v(b + GAS);
+  }
+  // value v of lane (j, hh): query j, dimension 8 (v / 4) + 4 hh + v % 4 of either half
+  float *ml = buf + GAS * GPT;
+  if (wv < used) {
+    float *mine = buf + wv * GPT + j * 68 + 4 * hh;
+#pragma unroll
+    for (int d = 0; d < 2; ++d)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<float4 *>(mine + 32 * d + 8 * g) =
+            make_float4(o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]);
+    ml[wv * 64 + 32 * hh + j] = hh ? l : m;
+  }
+  __syncthreads();
+  const int jt = tid() >> 4, c = tid() & 15;
+  if (T0 + jt >= n) return;
+  float M = -INFINITY;
+  for (int w = 0; w < used; ++w) M = fmaxf(M, ml[w * 64 + jt]);
+  M = score_ref(M);
+  float L = 0.f, r[4] = {0.f, 0.f, 0.f, 0.f};
+  for (int w = 0; w < used; ++w) {
+    const float f = expf(ml[w * 64 + jt] - M);
+    const float4 u = *reinterpret_cast<const float4 *>(buf + w * GPT + jt * 68 + 4 * c);
+    L = __builtin_fmaf(ml[w * 64 + 32 + jt], f, L);
+    r[0] = __builtin_fmaf(u.x, f, r[0]), r[1] = __builtin_fmaf(u.y, f, r[1]);
+    r[2] = __builtin_fmaf(u.z, f, r[2]), r[3] = __builtin_fmaf(u.w, f, r[3]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = r[e] / L;
+  planes_store4(A.pxo + ((size_t)(T0 >> 5) * (A.D >> 5) + 2 * hq) * BPX, jt, c, r);
+}
+
 // Thread = one lane's 16 bytes of every plane: eight columns of one row.
 __global__ __launch_bounds__(WG) void k_gp_tile(GMat W, int np, uint8_t *dst) {
   const int ng = W.cols >> 5;
@@ -503,6 +694,8 @@ int gp_init() {
     for (GpKernel k : row)
       MLLM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)gp_lds(GPW)));
+  for (const void *k : {reinterpret_cast<const void *>(k_gp_attn<false>), reinterpret_cast<const void *>(k_gp_attn<true>)})
+    MLLM_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kAttnLds));
   return 0;
 }
 
@@ -513,16 +706,6 @@ int gp_layers(const GpArgs &A, const int32_t *ids, int n, int pos0, bool last, c
   const bool gpt2 = A.arch == 1;
   const int ntt = (n + 31) / 32, ngd = A.D >> 5;
   hipLaunchKernelGGL(k_gp_embed, dim3(n), dim3(WG), 0, s, A, gpt2 ? nullptr : A.layers[0].n1, pos0);
-  PfArgs P{};
-  P.D = A.D;
-  P.NH = A.NH;
-  P.NKV = A.NKV;
-  P.max_seq = A.max_seq;
-  P.kv_fp16 = A.kv_fp16;
-  P.attn_scale = A.attn_scale;
-  P.kv = A.kv;
-  P.q = A.q;
-  P.opx = A.pxo;
   auto ln = [&](const float *g, int t0) {
     hipLaunchKernelGGL(k_gp_ln, dim3((n - t0 + WG / 64 - 1) / (WG / 64)), dim3(WG), 0, s, A, g, t0, n);
   };
@@ -539,7 +722,8 @@ int gp_layers(const GpArgs &A, const int32_t *ids, int n, int pos0, bool last, c
     if (final_layer && !last) break;
     // the prompt's last token needs its own tile of the last layer only
     const int tt0 = final_layer ? ntt - 1 : 0;
-    pf_attention(P, li, n, pos0, tt0, s);
+    hipLaunchKernelGGL(A.kv_fp16 ? k_gp_attn<true> : k_gp_attn<false>, dim3(ntt - tt0, A.NH), dim3(64 * GAS), kAttnLds, s,
+                       A, li, n, pos0, tt0);
     GpGemm O = gemm_of(W.proj, n, tt0, A.pxo);
     O.bias = gpt2 ? W.proj_b : nullptr;
     O.gain = gpt2 ? nullptr : W.n2;

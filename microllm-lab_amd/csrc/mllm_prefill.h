@@ -43,7 +43,6 @@ struct PfArgs {
   float *q;      // [tc][D] roped queries
   float *att;    // [tc][D] attention output
   float *h;      // [tc][FF] MLP activation
-  uint8_t *opx;  // set: the attention writes its output here as bf16 planes (mllm_planes.h) instead of att
   uint8_t *px;   // per 32-token tile: [K / 32][3 pieces x 2 K halves][64 lanes][16 B] f16, then [32] int exponents
 };
 
@@ -54,11 +53,6 @@ struct PfArgs {
 // `stream` into dst (pf_tiled_bytes(W) bytes) and describes it in *out.
 size_t pf_tiled_bytes(const PfMat &W);
 int pf_tile(const PfMat &W, void *dst, PfMat *out, hipStream_t stream);
-
-// One layer's causal attention for tokens [32 tt0, n) at positions pos0 ..:
-// queries A.q, keys and values from the cache, output to A.att or A.opx.
-// At most 4 query heads per KV head.
-void pf_attention(const PfArgs &A, int li, int n, int pos0, int tt0, hipStream_t stream);
 
 // Shapes the kernels take: head_dim 64, at most 4 query heads per KV head,
 // d_model and d_ff multiples of 64 up to 4096.

@@ -49,7 +49,6 @@
 
 #include "mllm_device.h"
 #include "mllm_host.h"
-#include "mllm_planes.h"
 #include "mllm_prefill.h"
 
 namespace mllm {
@@ -669,7 +668,7 @@ constexpr int SCH = 4;   // staged 8-value chunks per thread and super-block (32
 // others one); NSET = 4 with rep 3 puts three waves on every SIMD and takes
 // twice the keys per staging round.  (NSET = 4 needs rep <= 3 and the f16
 // cache: 4 rep waves of an f32 cache's registers would not fit.)
-template <bool SPLIT_KV, int NSET, bool OPX>
+template <bool SPLIT_KV, int NSET>
 __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int li, int n, int pos0, int tt0) {
   constexpr int KSB = 32 * NSET;    // keys per super-block
   constexpr int VROW = KSB + 4;     // halves per staged value column (KSB keys + pad)
@@ -867,7 +866,6 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
       l = l + mrg0[(s - 1) * MSET + 33] * a[s];
     }
     float *out = A.att + (size_t)(T0 + j) * A.D + hq * PF_HD + 4 * hh;
-    uint8_t *opx = OPX ? A.opx + ((size_t)(T0 >> 5) * (A.D >> 5) + 2 * hq) * BPX : nullptr;
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       float r[8];
@@ -882,15 +880,8 @@ __global__ __launch_bounds__(NSET == 4 ? 768 : 512) void k_pf_attn(PfArgs A, int
         r[e] = r0 / l;
         r[4 + e] = r1 / l;
       }
-      if (OPX) {
-        // dimensions 8g + 4hh .. +3 of the head's first and second group of 32
-        const float u0[4] = {r[0], r[1], r[2], r[3]}, u1[4] = {r[4], r[5], r[6], r[7]};
-        planes_store4(opx, j, 2 * g + hh, u0);
-        planes_store4(opx + BPX, j, 2 * g + hh, u1);
-      } else {
-        *reinterpret_cast<float4 *>(out + 8 * g) = make_float4(r[0], r[1], r[2], r[3]);
-        *reinterpret_cast<float4 *>(out + 32 + 8 * g) = make_float4(r[4], r[5], r[6], r[7]);
-      }
+      *reinterpret_cast<float4 *>(out + 8 * g) = make_float4(r[0], r[1], r[2], r[3]);
+      *reinterpret_cast<float4 *>(out + 32 + 8 * g) = make_float4(r[4], r[5], r[6], r[7]);
     }
   }
 }
@@ -1045,22 +1036,15 @@ void pf_carve(PfArgs &A, void *base, int tc) {
   A.px = p;
 }
 
-template <bool OPX>
+// One layer's causal attention for tokens [32 tt0, n) at positions pos0 ..
 static void launch_attention(const PfArgs &A, int li, int n, int pos0, int tt0, hipStream_t s) {
   const int nqt = (n + QTL - 1) / QTL, rep = A.NH / A.NKV;
   if (A.kv_fp16 && rep <= 3)
-    hipLaunchKernelGGL((k_pf_attn<false, 4, OPX>), dim3(nqt - tt0, A.NKV), dim3(256 * rep), 0, s, A, li, n, pos0, tt0);
+    hipLaunchKernelGGL((k_pf_attn<false, 4>), dim3(nqt - tt0, A.NKV), dim3(256 * rep), 0, s, A, li, n, pos0, tt0);
   else if (A.kv_fp16)
-    hipLaunchKernelGGL((k_pf_attn<false, 2, OPX>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
+    hipLaunchKernelGGL((k_pf_attn<false, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
   else
-    hipLaunchKernelGGL((k_pf_attn<true, 2, OPX>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
-}
-
-void pf_attention(const PfArgs &A, int li, int n, int pos0, int tt0, hipStream_t s) {
-  if (A.opx)
-    launch_attention<true>(A, li, n, pos0, tt0, s);
-  else
-    launch_attention<false>(A, li, n, pos0, tt0, s);
+    hipLaunchKernelGGL((k_pf_attn<true, 2>), dim3(nqt - tt0, A.NKV), dim3(128 * rep), 0, s, A, li, n, pos0, tt0);
 }
 
 int pf_layers(const PfArgs &A, const int32_t *ids, int n, int pos0, bool last, hipStream_t s) {
@@ -1088,7 +1072,7 @@ int pf_layers(const PfArgs &A, const int32_t *ids, int n, int pos0, bool last, h
     const bool final_layer = li == A.L - 1;
     if (final_layer && !last) break;
     const int tt0 = final_layer ? nqt - 1 : 0, t0 = tt0 * QTL;
-    pf_attention(A, li, n, pos0, tt0, s);
+    launch_attention(A, li, n, pos0, tt0, s);
     launch_quant<NORM_NONE>(A, A.att, A.D, nullptr, t0, n, s);
     PfGemm O = gemm_same(W.proj, n, gpt2 ? W.proj_b : nullptr, A.x, A.D);
     O.tt0 = tt0;

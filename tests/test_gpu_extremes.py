@@ -69,7 +69,7 @@ def rel(a, b):
 
 @gpu
 @pytest.mark.parametrize("n", [32, 256, 1024])
-@pytest.mark.parametrize("how", ["step"])
+@pytest.mark.parametrize("how", ["step", "prompt"])
 def test_minus_infinite_scores_weigh_nothing(oracle_lib, how, n):
     """The keys 0 .. n-1 are infinite in an f16 cache and score -inf for the last
     token, whose own key is finite and alone in its 32 positions (n = 256: in its
@@ -98,3 +98,58 @@ def test_minus_infinite_scores_weigh_nothing(oracle_lib, how, n):
     g.destroy()
     ref.close()
     assert rel(got, want) <= 5e-3  # the f16 cache
+
+
+@gpu
+@pytest.mark.parametrize("arch", ["llama", "gpt2"])
+@pytest.mark.parametrize("v,qk", [(-10, 0), (-30, 0), (17, 0), (60, 0), (0, -30), (0, 20), (0, 60), (-20, -20)])
+def test_prompt_attention_at_any_magnitude(oracle_lib, arch, v, qk):
+    """Value rows times 2^v with the output projection times 2^-v, query rows
+    times 2^-qk with key rows times 2^qk: the same function.  Last logits of a
+    batched prompt and of a step after it within 2e-6 of the float64 oracle's
+    scale (float32 roundings, 2e-7 to 6e-7 measured)."""
+    def edit(w):
+        for i in range(2):
+            q = w(f"blocks.{i}.attn.qkv")
+            q[:128] *= 2.0 ** -qk
+            q[128:-64 * kv] *= 2.0 ** qk
+            q[-64 * kv:] *= 2.0 ** v
+            w(f"blocks.{i}.attn.proj")[:] *= 2.0 ** -v
+
+    kv = 1 if arch == "llama" else 2
+    bundle = edited(arch, edit, max_seq_len=160)
+    ids = [int(t) for t in np.random.default_rng(62).integers(0, 512, 101)]
+    print(f"magnitude {arch} v=2^{v} qk=2^{qk}", flush=True)
+    g = mllm.PetitGPT(bundle)
+    ref = oracle_lib.OracleModel(bundle)
+    w = [rel(g.forwardPrompt(ids[:100]), ref.forward_prompt(ids[:100])),
+         rel(g.forwardDecode(ids[100]), ref.forward_decode(ids[100]))]
+    g.destroy()
+    ref.close()
+    assert max(w) <= 2e-6, w
+
+
+@gpu
+@pytest.mark.parametrize("kv_fp16", [False, True])
+@pytest.mark.parametrize("at", [21, 60])
+def test_infinite_value_stays_with_later_tokens(at, kv_fp16):
+    """Token A's value row is infinite.  The cache rows of the prompt's tokens
+    before it serve a step after a roll-back as those of a prompt without it do
+    (to 2e-6 of the logits' scale: the products' split over waves may differ;
+    f16 cache: a rounding the other way)."""
+    def edit(w):
+        w("lm_head")[:, 0] = 0.0
+        w("lm_head")[A, 0] = 1.0
+        w("blocks.0.attn.qkv")[128 + 64:, 0] = 3e38
+
+    bundle = edited("llama", edit, max_seq_len=128)
+    ids = [int(t) for t in np.random.default_rng(63).integers(10, 512, 90)]
+    print(f"infinite value at {at} fp16={kv_fp16}", flush=True)
+    g = mllm.PetitGPT(bundle, kv_fp16=kv_fp16)
+    g.forwardPrompt(ids[:at])
+    want = g.forwardDecode(B).copy()
+    assert not np.isfinite(g.forwardPrompt(ids[:at] + [A] + ids[at:])).any()
+    g.cacheLen = at
+    got = g.forwardDecode(B).copy()
+    g.destroy()
+    assert rel(got, want) <= (5e-3 if kv_fp16 else 2e-6)
