@@ -400,26 +400,48 @@ __global__ __launch_bounds__(WG) void k_gp_ln(GpArgs A, const float *g, int t0, 
 // k_g_attn: keys, values and queries of any magnitude keep their 24 bits.
 // (Halves of f16 pairs, as the Q4 prompts take them, end at 65504 and lose bits
 // below 2^-13.)
+//
+// What bounds it: 64 MFMAs of 64 cycles a block, from about 1000 tokens on, with
+// 400 VALU instructions of softmax between them and two waves on a SIMD; below,
+// the launch and one latency per eight blocks.  At 2000 tokens of the 135M shape
+// 72 us a launch (34 TFLOP/s over the unmasked half): 116 with a clamp and a
+// 64-bit address per load, instead of resources that end after the last row, and
+// the heads of a tile apart in the grid.  The f16-pair kernel, whose units have
+// sixteen times the rate: prompts of 200 tokens 1.83 ms (now 1.67), 1000 3.85
+// (3.19), 2000 6.42 (5.61); with an f16 cache 1.69 (1.68) and 2000 4.82 (5.68).
 constexpr int GAS = 8;
 
-// Cache elements as loaded: four components of a key, one of a value.
+// Cache elements as loaded, four components of a key (k) and one of a value
+// (v) at byte `off` of a head's rows; past the rows of the resource: 0.
 template <bool F16>
 struct KvRaw;
 template <>
 struct KvRaw<false> {
   typedef float4 K;
   typedef float V;
-  static __device__ __forceinline__ float4 k4(const float4 &r) { return r; }
-  static __device__ __forceinline__ float f(float r) { return r; }
+  static __device__ __forceinline__ K k(__amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(K, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  }
+  static __device__ __forceinline__ V v(__amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(V, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+  }
+  static __device__ __forceinline__ float4 k4(const K &r) { return r; }
+  static __device__ __forceinline__ float f(V r) { return r; }
 };
 template <>
 struct KvRaw<true> {
   typedef uint2 K;
   typedef unsigned short V;
-  static __device__ __forceinline__ float4 k4(const uint2 &r) {
+  static __device__ __forceinline__ K k(__amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(K, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+  }
+  static __device__ __forceinline__ V v(__amdgpu_buffer_rsrc_t r, int off) {
+    return (V)__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0);
+  }
+  static __device__ __forceinline__ float4 k4(const K &r) {
     return make_float4(f16_bits(r.x & 0xffffu), f16_bits(r.x >> 16), f16_bits(r.y & 0xffffu), f16_bits(r.y >> 16));
   }
-  static __device__ __forceinline__ float f(unsigned short r) { return f16_bits(r); }
+  static __device__ __forceinline__ float f(V r) { return f16_bits(r); }
 };
 constexpr size_t kAttnLds = sizeof(float) * GAS * (GPT + 64);
 
@@ -434,27 +456,32 @@ __device__ __forceinline__ float score_ref(float mx) { return mx == -INFINITY ? 
 template <bool F16>
 __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, int pos0, int tt0) {
   extern __shared__ __attribute__((aligned(16))) float buf[];  // [GAS][GPT] outputs, [GAS][2][32] (max, sum)
-  const int T0 = (tt0 + (int)(gridDim.x - 1 - blockIdx.x)) * 32;  // the longest tiles first
-  const int hq = blockIdx.y, kvh = hq / (A.NH / A.NKV);
+  const int T0 = (tt0 + (int)(gridDim.y - 1 - blockIdx.y)) * 32;  // the longest tiles first
+  const int hq = blockIdx.x, kvh = hq / (A.NH / A.NKV);
   const int wv = __builtin_amdgcn_readfirstlane(tid() >> 6), lane = tid() & 63, j = lane & 31, hh = lane >> 5;
   const int qpos = pos0 + T0 + j, qlast = pos0 + min(T0 + 32, n) - 1;  // last key any query of the tile sees
   const int nb = (qlast >> 5) + 1, used = min(nb, GAS);
-  const size_t kb = (((size_t)li * 2) * A.NKV + kvh) * A.max_seq * GPHD, vb = kb + (size_t)A.NKV * A.max_seq * GPHD;
+  constexpr int ES = F16 ? 2 : 4, ROW = ES * GPHD;  // bytes of an element, of a row
+  const size_t hb = (size_t)A.max_seq * ROW;         // of a head
+  uint8_t *kp = static_cast<uint8_t *>(A.kv) + ((size_t)li * 2 * A.NKV + kvh) * hb;
+  // resources that end after row qlast: what the last block reads past it is 0
+  const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(kp, (short)0, (qlast + 1) * ROW, 0x00020000);
+  const __amdgpu_buffer_rsrc_t vres =
+      __builtin_amdgcn_make_buffer_rsrc(kp + A.NKV * hb, (short)0, (qlast + 1) * ROW, 0x00020000);
   float4 q[8];
   typename KvRaw<F16>::K kr[8];
   typename KvRaw<F16>::V vr[2][16];
-  // keys past qlast are masked: a valid row in their place
   auto load_k = [&](int b) {
-    const size_t at = kb + (size_t)min(32 * b + j, qlast) * GPHD + 4 * hh;
+    const int at = (32 * b + j) * ROW + 4 * hh * ES;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) kr[c] = static_cast<const typename KvRaw<F16>::K *>(A.kv)[(at + 8 * c) >> 2];
+    for (int c = 0; c < 8; ++c) kr[c] = KvRaw<F16>::k(kres, at + 8 * c * ES);
   };
   auto load_v = [&](int b) {
+    const int at = (32 * b + 4 * hh) * ROW + j * ES;
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-      const size_t at = vb + (size_t)min(32 * b + 8 * (v >> 2) + 4 * hh + (v & 3), qlast) * GPHD + j;
-      vr[0][v] = static_cast<const typename KvRaw<F16>::V *>(A.kv)[at];
-      vr[1][v] = static_cast<const typename KvRaw<F16>::V *>(A.kv)[at + 32];
+      vr[0][v] = KvRaw<F16>::v(vres, at + (8 * (v >> 2) + (v & 3)) * ROW);
+      vr[1][v] = KvRaw<F16>::v(vres, at + (8 * (v >> 2) + (v & 3)) * ROW + 32 * ES);
     }
   };
   {
@@ -722,7 +749,7 @@ int gp_layers(const GpArgs &A, const int32_t *ids, int n, int pos0, bool last, c
     if (final_layer && !last) break;
     // the prompt's last token needs its own tile of the last layer only
     const int tt0 = final_layer ? ntt - 1 : 0;
-    hipLaunchKernelGGL(A.kv_fp16 ? k_gp_attn<true> : k_gp_attn<false>, dim3(ntt - tt0, A.NH), dim3(64 * GAS), kAttnLds, s,
+    hipLaunchKernelGGL(A.kv_fp16 ? k_gp_attn<true> : k_gp_attn<false>, dim3(A.NH, ntt - tt0), dim3(64 * GAS), kAttnLds, s,
                        A, li, n, pos0, tt0);
     GpGemm O = gemm_of(W.proj, n, tt0, A.pxo);
     O.bias = gpt2 ? W.proj_b : nullptr;
