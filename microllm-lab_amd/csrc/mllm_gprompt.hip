@@ -215,10 +215,14 @@ __global__ __launch_bounds__(64 * GPW) void k_gp_gemm(GpArgs A, GpGemm G) {
   float *mine = buf + ks * GPT + j * 68 + 4 * hh;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    *reinterpret_cast<float4 *>(mine + 8 * q) = make_float4(h0[4 * q] + l0[4 * q], h0[4 * q + 1] + l0[4 * q + 1],
-                                                            h0[4 * q + 2] + l0[4 * q + 2], h0[4 * q + 3] + l0[4 * q + 3]);
-    *reinterpret_cast<float4 *>(mine + 32 + 8 * q) = make_float4(h1[4 * q] + l1[4 * q], h1[4 * q + 1] + l1[4 * q + 1],
-                                                                 h1[4 * q + 2] + l1[4 * q + 2], h1[4 * q + 3] + l1[4 * q + 3]);
+    float y[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      y[e] = plane_sum(h0[4 * q + e], l0[4 * q + e]);
+      y[4 + e] = plane_sum(h1[4 * q + e], l1[4 * q + e]);
+    }
+    *reinterpret_cast<float4 *>(mine + 8 * q) = make_float4(y[0], y[1], y[2], y[3]);
+    *reinterpret_cast<float4 *>(mine + 32 + 8 * q) = make_float4(y[4], y[5], y[6], y[7]);
   }
   __syncthreads();
   if (KS > 1) {
@@ -404,7 +408,7 @@ __global__ __launch_bounds__(WG) void k_gp_ln(GpArgs A, const float *g, int t0, 
 // What bounds it: 64 MFMAs of 64 cycles a block, from about 1000 tokens on, with
 // 400 VALU instructions of softmax between them and two waves on a SIMD; below,
 // the launch and one latency per eight blocks.  At 2000 tokens of the 135M shape
-// 72 us a launch (34 TFLOP/s over the unmasked half): 116 with a clamp and a
+// 72 us a launch (64 TFLOP/s over the unmasked half): 116 with a clamp and a
 // 64-bit address per load, instead of resources that end after the last row, and
 // the heads of a tile apart in the grid.  The f16-pair kernel, whose units have
 // sixteen times the rate: prompts of 200 tokens 1.83 ms (now 1.67), 1000 3.85

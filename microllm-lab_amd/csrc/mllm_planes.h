@@ -15,6 +15,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <math.h>
 #include <stdint.h>
 
 namespace mllm {
@@ -25,14 +26,22 @@ typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 typedef float v2fl __attribute__((ext_vector_type(2)));
 
 // The planes of two values, packed (the first in the low half).  The first
-// plane is taken from the value cut to bf16's largest, so that a finite value
-// past it keeps finite planes.
+// plane of a finite value is taken from the value cut to bf16's largest, so that
+// one past it keeps finite planes.  An infinity or NaN is itself in the first
+// plane and NaN in the others: a sum of first-plane products that is not finite
+// is the result, without the other planes' products (plane_sum).
+__device__ __forceinline__ float bf16_cut(float v) {
+  constexpr float M = 3.3895313892515355e38f;
+  return fabsf(v) < INFINITY ? __builtin_amdgcn_fmed3f(v, -M, M) : v;
+}
+__device__ __forceinline__ float plane_sum(float first, float rest) {
+  return fabsf(first) < INFINITY ? first + rest : first;
+}
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2fl){a, b}, v2bf));  // nearest even
 }
 __device__ __forceinline__ void bf16_split2(float a, float b, uint32_t (&p)[3]) {
-  constexpr float M = 3.3895313892515355e38f;
-  p[0] = bf16_pair(__builtin_amdgcn_fmed3f(a, -M, M), __builtin_amdgcn_fmed3f(b, -M, M));
+  p[0] = bf16_pair(bf16_cut(a), bf16_cut(b));
   a -= __uint_as_float(p[0] << 16);
   b -= __uint_as_float(p[0] & 0xffff0000u);
   p[1] = bf16_pair(a, b);

@@ -153,3 +153,30 @@ def test_infinite_value_stays_with_later_tokens(at, kv_fp16):
     got = g.forwardDecode(B).copy()
     g.destroy()
     assert rel(got, want) <= (5e-3 if kv_fp16 else 2e-6)
+
+
+@gpu
+@pytest.mark.parametrize("kind", ["f32", "f16", "bf16", "q8"])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("name", ["attn.qkv", "attn.proj", "mlp.w1", "mlp.w3", "mlp.w2"])
+def test_prompt_shows_non_finite_weights(name, value, kind):
+    """One infinite or NaN weight (q8: row scale) of layer 0 leaves no finite
+    logit in a batched prompt, as in the token steps."""
+    b = pgw.parse_pgw(pgw.make_model(pgw.small_config(), seed=64, kind=kind))
+    buf = bytearray(b.buffer)
+    t = b.tensors["blocks.0." + name]
+    row = -1 if name == "attn.qkv" else 7  # a value row
+    if kind == "q8":
+        np.frombuffer(buf, np.float32, t["shape"][0], b.payload_off + t["scaleOffset"])[row] = value
+    else:
+        bits16 = {"f16": int(np.float16(value).view(np.uint16)), "bf16": int(np.float32(value).view(np.uint32)) >> 16}
+        dt = np.float32 if kind == "f32" else np.uint16
+        m = np.frombuffer(buf, dt, int(np.prod(t["shape"])), b.payload_off + t["offset"]).reshape(t["shape"])
+        m[row, 3] = value if kind == "f32" else bits16[kind]
+    g = mllm.PetitGPT(dataclasses.replace(b, buffer=bytes(buf)))
+    print(f"weight {name} {kind} {value}", flush=True)
+    batch = g.forwardPrompt([3, 1, 4, 1, 5]).copy()
+    steps = [g.forwardPrompt([3, 1])] + [g.forwardDecode(t) for t in (4, 1, 5)]
+    assert not np.isfinite(steps[-1]).any()
+    assert not np.isfinite(batch).any()
+    g.destroy()
