@@ -169,7 +169,8 @@ typedef struct mllm_model mllm_model;
  * from a copy of the layer matrices as bf16 planes (2, 4 or 6 bytes per
  * weight: bf16 and per-row Q8, f16, the others); models with more than 4
  * query heads per KV head or d_ff not a multiple of 64, and a device without
- * room for the copy, keep the token steps. */
+ * room for the copy, keep the token steps, and mllm_set_prefill(model, 0, 0)
+ * goes back to them and frees the copy. */
 int mllm_model_create(const mllm_config *cfg, const void *payload, uint64_t payload_nbytes,
                       const mllm_tensor *tensors, int n_tensors, mllm_model **out);
 /* GpuPetitGPT.destroy (webgpu.js:1284-1297); NULL is accepted. */
@@ -272,7 +273,10 @@ int mllm_set_debug(mllm_model *model, int max_layers, int no_attn, int no_mlp, i
  * the tokens per chunk; later chunks read the earlier ones' keys from the
  * cache.  Models with more than 4 query heads per KV head, or d_model / d_ff
  * not multiples of 64, keep the pass path (min_tokens > 0 then returns
- * MLLM_ERR_UNSUPPORTED). */
+ * MLLM_ERR_UNSUPPORTED).  A kind-generic model (mllm_model_create) has no
+ * threshold to move: min_tokens = 0 gives its prompts to the token steps for
+ * good and frees the copy that the batches read, min_tokens > 0 returns
+ * MLLM_ERR_UNSUPPORTED. */
 int mllm_set_prefill(mllm_model *model, int min_tokens, int chunk_tokens);
 
 /* GpuPetitGPT.lastTiming {n, gpuMs} (webgpu.js:1143-1160): the time between

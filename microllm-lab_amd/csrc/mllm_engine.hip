@@ -2944,6 +2944,8 @@ struct mllm_model {
   // their batched prompts (mllm_gprompt.hip): gp.tc = 0 where there are none
   GpArgs gp{};
   std::vector<GpLayer> gp_layer;
+  void *gp_buf = nullptr;            // their matrices and work buffers
+  size_t gp_bytes = 0;
   hipGraphExec_t g_graph[2] = {};    // one step without / with the lm_head (exec mode 1)
 };
 
@@ -3442,22 +3444,35 @@ int generic_prompt_create(mllm_model *M) {
   const size_t work = gp_buffer_bytes(P, tc);
   size_t bytes = work;
   for (const Job &j : jobs) bytes += gp_tiled_bytes(j.src->rows, j.src->cols, j.np);
-  void *buf = nullptr;
-  if (hipMalloc(&buf, bytes) != hipSuccess) {
+  if (hipMalloc(&M->gp_buf, bytes) != hipSuccess) {
     (void)hipGetLastError();
+    M->gp_buf = nullptr;
     return 0;
   }
-  M->allocs.push_back(buf);
+  M->gp_bytes = bytes;
   M->device_bytes += bytes;
   if (int rc = gp_init()) return rc;
-  uint8_t *at = static_cast<uint8_t *>(buf) + work;
+  uint8_t *at = static_cast<uint8_t *>(M->gp_buf) + work;
   for (const Job &j : jobs) {
     if (int rc = gp_tile(*j.src, j.np, at, j.dst, M->stream)) return rc;
     at += gp_tiled_bytes(j.src->rows, j.src->cols, j.np);
   }
   MLLM_HIP(hipStreamSynchronize(M->stream));
   P.layers = M->gp_layer.data();
-  gp_carve(P, buf, tc);
+  gp_carve(P, M->gp_buf, tc);
+  return 0;
+}
+
+// Prompts of a kind-generic model through the token steps from here on; the
+// batched path's memory goes back.
+int generic_prompt_off(mllm_model *M) {
+  if (!M->gp_buf) return 0;
+  MLLM_HIP(hipStreamSynchronize(M->stream));
+  M->gp.tc = 0;
+  void *buf = M->gp_buf;
+  M->gp_buf = nullptr;
+  M->device_bytes -= M->gp_bytes;
+  MLLM_HIP(hipFree(buf));
   return 0;
 }
 
@@ -3941,6 +3956,7 @@ extern "C" int mllm_model_destroy(mllm_model *M) {
   for (hipGraphExec_t &ge : M->g_graph)
     if (ge) hipGraphExecDestroy(ge);
   if (M->h_out) hipHostFree(M->h_out);
+  if (M->gp_buf) hipFree(M->gp_buf);
   for (void *p : M->allocs) hipFree(p);
   for (hipEvent_t e : M->prof_ev) (void)hipEventDestroy(e);
   if (M->ev0) hipEventDestroy(M->ev0);
@@ -4064,6 +4080,7 @@ extern "C" int mllm_set_prefill(mllm_model *M, int min_tokens, int chunk_tokens)
   if (min_tokens > 0 && !M->pf_tc_max) return set_error(MLLM_ERR_UNSUPPORTED, "batched prompts unsupported for this model");
   MLLM_CHECK(chunk_tokens >= 0 && chunk_tokens <= M->pf_tc_max, "prefill chunk %d (at most %d)", chunk_tokens,
              M->pf_tc_max);
+  if (M->generic) return generic_prompt_off(M);
   M->pf_min = min_tokens;
   M->pf.tc = chunk_tokens ? chunk_tokens : M->pf_tc_max;
   return 0;

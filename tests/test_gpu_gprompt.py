@@ -83,3 +83,29 @@ def test_prompt_options_vs_oracle(oracle_lib, case):
         assert worst(oracle_lib, build(seed=46, kind="f32", n_layers=1), 60, kv_fp16=True) <= TOL_F16KV
     else:  # Q4 group-32 beyond the fused step's limits
         assert worst(oracle_lib, build(seed=47, kind="q4", d_ff=4160, n_layers=1), 45) <= TOL
+
+
+@gpu
+@pytest.mark.parametrize("n", [1, 3, 40])
+@pytest.mark.parametrize("kind", ["f16", "q4"])
+def test_set_prefill_0_gives_the_token_steps(kind, n):
+    """Batches switched off: the token steps' bits, the bytes of the bf16 copy
+    given back, and thresholds refused as before."""
+    bundle = build(seed=48, kind=kind, group=64)
+    ids = [int(v) for v in np.random.default_rng(n).integers(0, 512, n + 1)]
+    print(f"set_prefill 0 {kind} n={n}", flush=True)
+    g = mllm.PetitGPT(bundle)
+    steps = g.forwardPrompt(ids[:1]).copy()
+    for t in ids[1:n]:
+        steps = g.forwardDecode(t).copy()
+    before = g.bytesAllocated
+    for _ in range(2):  # a second time changes nothing
+        g.set_prefill(0)
+        c = bundle.cfg
+        weights = c.n_layers * c.d_model * (2 * c.d_model + 2 * 64 * c.n_kv_heads + 3 * c.d_ff)
+        assert before - g.bytesAllocated >= weights * (4 if kind == "f16" else 6)
+        got = g.forwardPrompt(ids[:n]).copy()
+        assert g.cacheLen == n and np.array_equal(got.view(np.uint32), steps.view(np.uint32))
+        with pytest.raises(mllm.abi.MllmError, match="UNSUPPORTED"):
+            g.set_prefill(3)
+    g.destroy()
