@@ -323,13 +323,14 @@ __global__ __launch_bounds__(AMT) void k_argmax_tiles(const unsigned char *__res
 // y[t][r] = W x[t] for many tokens, every row with the bits of k_gemv_q4.
 //
 // The GEMV's integers are three signed bytes, xi = 65536 h + 256 m + l
-// (|xi| <= Q6MAX < 2^23), so a group's exact dot is three
+// (|xi| <= Q6MAX < 2^23; of the integers that saturate where the scale
+// overflows, groups below 2.3e-32, the low 24 bits, as there), so a group's
+// exact dot is three
 // v_mfma_i32_32x32x32_i8 -- K = 32 is one group -- combined modulo 2^32 by two
 // shift-adds; then the GEMV's own ((float)dot * sx) * w_scale, one add a group,
 // and its order of additions: lane partial l of L sums groups l, l + L, ...,
 // and the segment tree is formed depth first, so one partial per tree level is
-// live instead of L of them.  (A group whose values are all below 2.3e-32, past
-// the GEMV's range, may saturate differently.)
+// live instead of L of them.
 //
 // Wave: 32 weight rows (lane j of a half: row j) x 32 tokens (value v: token
 // 8 (v / 4) + 4 hh + v % 4).  A workgroup's waves share its 32 tokens, whose
@@ -443,7 +444,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_q4(const uint8_t *__restrict__
         // byte p of xi + 0x808080, its top bit flipped, is the signed byte p of xi
         uint32_t b[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) b[k] = (uint32_t)(min(max((int)__builtin_rintf(e[k] * inv), -8388608), 8355711) + 0x808080);
+        for (int k = 0; k < 4; ++k) b[k] = (uint32_t)(int)__builtin_rintf(e[k] * inv) + 0x808080u;
         const uint32_t own0 = odd ? b[1] : b[0], own1 = odd ? b[3] : b[2];
         const uint32_t got0 = (uint32_t)dpp_i<0xB1>((int)(odd ? b[0] : b[1]));
         const uint32_t got1 = (uint32_t)dpp_i<0xB1>((int)(odd ? b[2] : b[3]));

@@ -71,6 +71,20 @@ def test_values_over_the_range():
 
 
 @gpu
+def test_gemm_groups_below_the_scaled_range():
+    """Groups whose largest value is below 2.3e-32, where the GEMV's scale
+    overflows and its integers wrap: still the GEMV's bits."""
+    rng = np.random.default_rng(3)
+    t, n = 40, 320
+    x = rng.standard_normal((t, n)).astype(np.float32)
+    x[::2, 32:64] *= np.float32(1e-33)
+    x[1::2, 64:128] *= np.float32(1e-38)
+    x[3] *= np.float32(1e-36)
+    print("gemm tiny groups", flush=True)
+    check(t, 100, n, x)
+
+
+@gpu
 @pytest.mark.parametrize("m,n", [(1, 32), (3, 96), (127, 160), (33, 4096), (2049, 4096)])
 @pytest.mark.parametrize("skip", [0, 1, 2])
 def test_dequant_every_alignment(m, n, skip):
