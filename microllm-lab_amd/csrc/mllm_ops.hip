@@ -681,12 +681,22 @@ __global__ __launch_bounds__(WGT) void k_gemv_q8i_batched(const int8_t *const *_
 // ---------------------------------------------------------------- f32 GEMV
 typedef float v4fl __attribute__((ext_vector_type(4)));
 // R rows per wavefront, lanes over float4s, fixed-pattern wave reduction (a
-// row's sum does not depend on R).  Bound by the matrix read: one row per wave
-// and ordinary loads took 22.6 us for 49152 x 576 (5.0 TB/s), loads past the
-// caches 21.3, four rows per wave (their loads in flight together) 18.0 (6.3
-// TB/s).  Matrices of fewer rows keep the ordinary loads: the caches hold them
-// between calls.
-template <int R>
+// row's sum does not depend on R or STREAM).  Bound by the matrix read.  Two
+// choices where the launch still has four waves per SIMD (16384 rows), us a call
+// on a matrix read again / on one not seen lately:
+//   R       rows per wave, whose loads are in flight together: more for shorter
+//           rows.  One / two / four rows: 49152 x 320 12.8 / 10.5 / 10.5, 32000 x
+//           1024 19.0 / 19.0 / 23.9, 16384 x 2048 19.4 / 21.3 / 21.4.
+//   STREAM  loads past the caches from 42 MB on, where the L2s no longer hold
+//           much of the matrix for the next call.  Ordinary and streamed, 16384 x
+//           512 (34 MB) 3.6 / 7.3 and 6.5 / 7.3, 16384 x 640 (42) 7.2 / 9.0 and
+//           7.7 / 8.5, 20000 x 576 (46) 8.0 / 9.7 and 8.2 / 9.2, 49152 x 576 (113)
+//           17.1 / 20.2 and 17.5 / 18.6, 49152 x 1792 (352) 57.7 / 57.5 and 50.6 /
+//           51.5.
+// Matrices of fewer rows have one row per wave and ordinary loads: 8192 x 8192
+// takes 38.9 / 48.3 that way, 43.7 / 45.7 streamed, 40.9 / 48.8 with two rows.
+constexpr size_t kF32Stream = 42u << 20;
+template <int R, bool STREAM>
 __global__ __launch_bounds__(WG) void k_gemv_f32(const float *__restrict__ w, const float *__restrict__ x,
                                                   float *__restrict__ y, int rows, int cols) {
   const int lane = threadIdx.x & 63;
@@ -706,7 +716,7 @@ __global__ __launch_bounds__(WG) void k_gemv_f32(const float *__restrict__ w, co
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const v4fl *p = reinterpret_cast<const v4fl *>(wr[r] + k);
-        a[r] = R > 1 ? __builtin_nontemporal_load(p) : *p;
+        a[r] = STREAM ? __builtin_nontemporal_load(p) : *p;
       }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
@@ -1250,10 +1260,12 @@ extern "C" int mllm_gemv_f32(int m, int n, const float *w, const float *x, float
   MLLM_CHECK(m > 0 && n > 0, "invalid shape m=%d n=%d", m, n);
   MLLM_CHECK(w && x && y, "null pointer");
   MLLM_CHECK((n & 3) != 0 || (((uintptr_t)w | (uintptr_t)x) & 15) == 0, "w and x must be 16-byte aligned");
-  // four rows per wave where that still leaves four waves per SIMD
-  const int R = m >= 4 * 16 * (device_wg_cap() / 8) ? 4 : 1, per_wg = R * (WG / 64);
-  hipLaunchKernelGGL(R == 4 ? k_gemv_f32<4> : k_gemv_f32<1>, dim3((m + per_wg - 1) / per_wg), dim3(WG), 0,
-                     as_stream(stream), w, x, y, m, n);
+  const bool many = m >= 4 * 16 * (device_wg_cap() / 8), stream_loads = many && 4 * (size_t)m * n > kF32Stream;
+  const int R = !many || n > 1024 ? 1 : n > 576 ? 2 : 4, per_wg = R * (WG / 64);
+  const auto kern = R == 4   ? (stream_loads ? k_gemv_f32<4, true> : k_gemv_f32<4, false>)
+                    : R == 2 ? (stream_loads ? k_gemv_f32<2, true> : k_gemv_f32<2, false>)
+                             : (stream_loads ? k_gemv_f32<1, true> : k_gemv_f32<1, false>);
+  hipLaunchKernelGGL(kern, dim3((m + per_wg - 1) / per_wg), dim3(WG), 0, as_stream(stream), w, x, y, m, n);
   MLLM_HIP(hipGetLastError());
   return 0;
 }

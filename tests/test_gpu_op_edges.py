@@ -128,6 +128,25 @@ def test_gemv_f32_rows_per_wave(n):
 
 
 @gpu
+@pytest.mark.parametrize("m,n", [(19999, 576), (16387, 580), (16387, 673), (16387, 1024), (16386, 1025), (16387, 1028)])
+def test_gemv_f32_rows_and_streams(m, n):
+    """Four, two and one row per wave past 16384 rows, with ordinary and with
+    streamed loads: the bits of a short call on the last rows (one row per wave,
+    ordinary loads)."""
+    rng = np.random.default_rng(m + n)
+    w, x = torch.from_numpy(rng.random((m, n), np.float32) - 0.5).cuda(), torch.from_numpy(rng.random(n, np.float32)).cuda()
+    y = torch.full((m + 1,), 7.0, dtype=torch.float32, device="cuda")
+    k = 1000 + (m & 3)  # the tail starts on a 16-byte boundary
+    y1 = torch.empty(k, dtype=torch.float32, device="cuda")
+    print(f"gemv f32 {m}x{n}", flush=True)
+    abi.call("mllm_gemv_f32", m, n, ptr(w), ptr(x), ptr(y), None)
+    abi.call("mllm_gemv_f32", k, n, ptr(w[m - k:]), ptr(x), ptr(y1), None)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert got[m] == 7.0 and np.array_equal(got[m - k:m].view(np.uint32), y1.cpu().numpy().view(np.uint32))
+
+
+@gpu
 @pytest.mark.parametrize("rows", [57216, 57344, 57345])
 @pytest.mark.parametrize("kind", ["first of ties", "nan0", "nan rows", "all nan"])
 def test_argmax_on_both_sides_of_two_launches(rows, kind):
