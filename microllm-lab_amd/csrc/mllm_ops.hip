@@ -1037,11 +1037,15 @@ int amx_scratch_for(int dev, size_t need, unsigned char **out) {
 }
 
 // Tokens from which a GEMM takes the matrix cores.  Up to a few hundred tokens
-// that launch's time is one workgroup's own (16 us at 576 columns, 26 at 960, 60
-// at 2560), and the GEMV kernel needs 8, 7.6 and 15 us per eight tokens: 24
-// tokens 29 / 23 / 46 us against 16 / 26 / 60, 32 tokens 38 / 31 / 61 against
-// 16 / 26 / 60.
-constexpr int kGemmTok = 32;
+// that launch's time is one workgroup's own, in proportion to the columns (16 us
+// at 576, 26 at 960, 58 at 2560, 92 at 4096), and the GEMV kernel needs 8, 7.6, 15
+// and 24 us per eight tokens: 24 tokens 29 / 23 / 46 us against 16 / 26 / 58, 32
+// tokens 38 / 31 / 61 / 98 against 16 / 26 / 58 / 92.  Past 4096 columns (rows on
+// more than 16 lanes) the GEMV's time per column falls, and again where its
+// workgroups have 512 threads: at 41 tokens and 1000 rows 110, 201 and 264 us at
+// 4128, 8192 and 12288 columns against 108, 187 and 287, at 4096 rows and 4128
+// columns 94 against 110.
+constexpr int gemm_tokens(int lanes) { return lanes <= 16 ? 32 : 48; }
 
 int gemm_q4_tiles(const Q4SegPlan &pl, int t, int m, int n, const uint8_t *packed, const float *scale, const float *x,
                   float *y, hipStream_t st) {
@@ -1069,7 +1073,7 @@ int q4_gemm(int t, int m, int n, const uint8_t *packed, const float *scale, cons
   MLLM_CHECK((size_t)m * n / 2 < (1ull << 31), "matrix of %zu bytes exceeds 2 GiB", (size_t)m * n / 2);
   const int ng = n / 32;
   const Q4SegPlan pl = q4_seg_plan(n, m, 1);
-  if (t >= kGemmTok) return gemm_q4_tiles(pl, t, m, n, packed, scale, x, y, st);
+  if (t >= gemm_tokens(pl.L)) return gemm_q4_tiles(pl, t, m, n, packed, scale, x, y, st);
   const int P = q4_seg_pick_p(pl, m, 1);
   const int ntiles = (m + pl.rpp * P - 1) / (pl.rpp * P);
   for (int t0 = 0; t0 < t;) {

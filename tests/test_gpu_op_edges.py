@@ -44,6 +44,15 @@ def test_rows_bit_identical_to_gemv(t, m, n):
 
 
 @gpu
+@pytest.mark.parametrize("t", [47, 48, 49])
+@pytest.mark.parametrize("m,n", [(33, 4096), (40, 4128), (33, 8192), (33, 12288)])
+def test_tokens_where_the_matrix_cores_take_over(t, m, n):
+    """Rows on more than 16 lanes change over at 48 tokens."""
+    print(f"gemm t={t} m={m} n={n}", flush=True)
+    check(t, m, n, np.random.default_rng(t + n).standard_normal((t, n)).astype(np.float32))
+
+
+@gpu
 @pytest.mark.parametrize("t,m,n", [(1000, 2300, 960), (1030, 2050, 2560), (520, 4100, 544), (530, 4100, 4096)])
 def test_large_launches(t, m, n):
     """A workgroup of eight waves per CU: fewer groups fit the LDS at a time."""
