@@ -3482,12 +3482,13 @@ int generic_create(mllm_model *M) {
   const mllm_config &c = M->cfg;
   const int D = c.d_model, FF = c.d_ff, NH = c.n_heads, NKV = c.n_kv_heads, V = c.vocab_size, L = c.n_layers;
   const int kvd = NKV * HD;
-  // the staged input row (k_g_gemv), the attention weights (k_g_attn) and
-  // the history lists (k_g_argmax) live in LDS
+  // The largest rows and contexts taken.  Of what the kernels hold in LDS, the
+  // merged attention row (4 D bytes, the O GEMV) and the history lists (4 (34 +
+  // max_seq_len) bytes, k_g_argmax) fit 64 KiB with them; d_ff is bounded as D.
   if (std::max(D, FF) > 15000)
-    return set_error(MLLM_ERR_UNSUPPORTED, "rows of %d columns exceed the staged row", std::max(D, FF));
-  if ((size_t)(HD + c.max_seq_len + 4 + 256 + 4) * sizeof(float) > 64 * 1024)
-    return set_error(MLLM_ERR_UNSUPPORTED, "max_seq_len %d exceeds the attention workgroup's LDS", c.max_seq_len);
+    return set_error(MLLM_ERR_UNSUPPORTED, "rows of %d columns exceed 15000", std::max(D, FF));
+  if (c.max_seq_len > 16056)
+    return set_error(MLLM_ERR_UNSUPPORTED, "max_seq_len %d exceeds 16056", c.max_seq_len);
   GArgs &A = M->g;
   A.arch = c.arch;
   A.L = L;

@@ -67,8 +67,8 @@ __device__ __forceinline__ bool stopped(const GCursor *c) {
 // on its way at once.  These launches are bound by that one latency (a layer's
 // matrices are 0.2 to 3 MB), where the former form (inputs staged in LDS, two
 // to three block reductions, then the weights) paid it two to three times:
-// per-row Q8 at the 135M shape, us a launch, QKV 5.1 -> 4.4, O 5.1 -> 4.0 (it
-// merges the attention's splits, too), gate/up 6.3 -> 4.7, down 5.1 -> 3.8,
+// per-row Q8 at the 135M shape, us a launch, QKV 5.1 -> 4.4, O 5.1 -> 4.1 (it
+// merges the attention's splits, too), gate/up 6.3 -> 4.7, down 5.1 -> 3.4,
 // lm_head 21 -> 12.5.
 constexpr int G_MIXED = -1;  // W and W3 of different storages
 template <int KIND>
@@ -483,7 +483,7 @@ __device__ __forceinline__ float rope_at(const GArgs &A, const float *hd, int d,
 // attp, and the O GEMV merges the splits while it reads its input.  The
 // former form -- a workgroup per head, a row per thread, then P.V down four
 // position slices -- was bound by one workgroup's load rate: 32.2 us at 700
-// positions of the 135M shape, 7.3 now (8.3 with 64 positions a wave: twice
+// positions of the 135M shape, 7.6 now (8.3 with 64 positions a wave: twice
 // the code, which runs once from a cold instruction cache).
 // The new position's k and v are taken from LDS (as the cache holds them:
 // f16-rounded for an f16 cache), so a group's heads do not wait for the one
@@ -797,7 +797,7 @@ bool g_kind_supported(int kind, int group) {
 int g_gemv(const GMat &W, const float *x, float *y, hipStream_t s) {
   MLLM_CHECK(g_kind_supported(W.kind, W.group) && W.cols % 8 == 0 && (W.kind != MLLM_Q4 || W.cols % W.group == 0),
              "matrix storage %d (group %d, %d columns) unsupported", W.kind, W.group, W.cols);
-  MLLM_CHECK(W.cols <= 16000, "%d columns exceed the staged row", W.cols);
+  MLLM_CHECK(W.cols <= 16000, "%d columns exceed 16000", W.cols);
   launch_gemv<G_STORE, GN_NONE>(gemv_args(W, x, nullptr, 0.f, nullptr, y, nullptr), s);
   MLLM_HIP(hipGetLastError());
   return 0;

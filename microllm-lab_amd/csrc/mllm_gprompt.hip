@@ -6,10 +6,14 @@
 //
 // GEMMs on the bf16 matrix cores at float32 accuracy: the activations are
 // three bf16 planes (mllm_planes.h, exact), the weights one, two or three
-// (gp_planes), and the products above 2^-26 of the largest are formed:
-// x0 w0, x1 w0, x2 w0 (1 plane), + x0 w1, x1 w1 (2), + x0 w2 (3).  x0 w0 has an
-// accumulator of its own, the corrections share another, added at the end, so
-// the roundings of the large sum are one per 16 columns.
+// (gp_planes), and these products are formed: x0 w0, x1 w0, x2 w0 (1 plane),
+// + x0 w1, x1 w1 (2), + x0 w2 (3).  What one plane leaves of a value is at most
+// 2^-8 of it, two planes 2^-17, so each product left out (x2 w1, with 3 planes
+// x1 w2 too) is at most 2^-25 of x w: half a float32 rounding.  Q8 group-32 and Q4 weights are
+// the de-quantised values rounded to float32 (the token steps multiply the
+// integers and scale the sums).  x0 w0 has an accumulator of its own, the
+// corrections share another, added at the end, so the roundings of the large
+// sum are one per 16 columns.
 //
 // No kernel needs a whole row except the norms' statistics, so nothing but the
 // GEMMs and the attention is launched for a llama layer:

@@ -1,7 +1,7 @@
 """Batched prompts of the kind-generic models (mllm_gprompt.hip; forwardPrompt,
 infer.js:553-577) against the oracle, which accumulates in float64: every
-storage at lengths around the 32-token tile, the workgroup order by XCD (a
-tile count that divides by eight), a chunk boundary, partial rotary, four
+storage at lengths around the 32-token tile, the workgroup order by XCD (one to
+eight token groups of XCDs), a chunk boundary, partial rotary, four
 query heads per KV head, gate and up rows in different storages.
 
 Bar: the last-token logits, and those of decode steps that read the cache,
@@ -51,10 +51,23 @@ def test_kind_prompt_vs_oracle(oracle_lib, arch, kind, group, n):
     assert worst(oracle_lib, bundle, n) <= TOL
 
 
+def token_groups(n, rows, planes):
+    """The token groups of XCDs that a GEMM of n tokens takes: the split whose
+    XCDs fetch least, in bytes per column."""
+    w, x = rows * 2 * planes, (n + 31) // 32 * 32 * 6
+    return min((1, 2, 4, 8), key=lambda t: t * w + 8 // t * x)
+
+
+def test_tile_placement_reaches_every_split():
+    rows = (256 + 2 * 64, 256, 512)  # QKV, O and down, gate/up
+    assert {token_groups(n, r, 1) for n in (20, 100, 300, 512) for r in rows} == {1, 2, 4, 8}
+
+
 @gpu
-@pytest.mark.parametrize("n", [255, 256, 300, 512])
+@pytest.mark.parametrize("n", [20, 100, 255, 256, 300, 512])
 def test_tile_placement_vs_oracle(oracle_lib, n):
-    """8 and 16 tiles (each tile's workgroups on one XCD), 10 (plain order)."""
+    """XCDs in one to eight token groups, and tile counts that do and do not
+    divide among them."""
     bundle = build(seed=42, kind="bf16", d_model=256, n_heads=4, n_kv_heads=1, max_seq_len=640)
     print(f"placement n={n}", flush=True)
     assert worst(oracle_lib, bundle, n) <= TOL
