@@ -498,6 +498,7 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
   const int h = blockIdx.x, kvh = h / rep, lane = tid() & 63, wv = tid() >> 6;
   const int s0 = (int)blockIdx.y * GSPLIT;
   if (s0 >= n) return;
+  constexpr int ES = F16 ? 2 : 4;  // bytes of a cache element
   const size_t kb = g_kv_index(A, li, 0, kvh, 0), vb = g_kv_index(A, li, 1, kvh, 0);
   const int k0 = s0 + GAK * wv;  // this wave's positions k0 .. k0 + GAK - 1
   const bool on = k0 < n;       // uniform in the wave
@@ -508,22 +509,25 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
   float kv = rope_at(A, kq, lane, pos), vv = kq[A.NKV * GHD + lane];
   const int grp = lane >> 4, d4 = 4 * (lane & 15);
   uint4 kr[GAK / 4], vr[GAK / 4];
-  if (on && pos == 0) {  // no cached row: row 0 is an earlier call's, or being written
-#pragma unroll
-    for (int i = 0; i < GAK / 4; ++i) kr[i] = vr[i] = make_uint4(0u, 0u, 0u, 0u);
-  } else if (on) {
+  if (on) {
+    // resources of the rows before the new one (none at position 0): the row at
+    // it, which another head may be writing, and those past it, left by earlier
+    // calls, are read as 0 -- their weight is 0, and 0 times an infinity is NaN
+    uint8_t *cache = static_cast<uint8_t *>(A.kv);
+    const __amdgpu_buffer_rsrc_t kres = __builtin_amdgcn_make_buffer_rsrc(cache + kb * ES, (short)0, pos * GHD * ES, 0x00020000);
+    const __amdgpu_buffer_rsrc_t vres = __builtin_amdgcn_make_buffer_rsrc(cache + vb * ES, (short)0, pos * GHD * ES, 0x00020000);
+    const int at = ((k0 + grp) * GHD + d4) * ES;
 #pragma unroll
     for (int i = 0; i < GAK / 4; ++i) {
-      // rows at and past the new one are not used: a valid row in their place
-      const size_t off = (size_t)min(k0 + 4 * i + grp, pos - 1) * GHD + d4;
+      const int off = at + 4 * i * GHD * ES;
       if (F16) {
-        const uint2 a = *reinterpret_cast<const uint2 *>(reinterpret_cast<const __half *>(A.kv) + kb + off);
-        const uint2 b = *reinterpret_cast<const uint2 *>(reinterpret_cast<const __half *>(A.kv) + vb + off);
+        const uint2 a = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(kres, off, 0, 0));
+        const uint2 b = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(vres, off, 0, 0));
         kr[i] = make_uint4(a.x, a.y, 0u, 0u);
         vr[i] = make_uint4(b.x, b.y, 0u, 0u);
       } else {
-        kr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(A.kv) + kb + off);
-        vr[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const float *>(A.kv) + vb + off);
+        kr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kres, off, 0, 0));
+        vr[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vres, off, 0, 0));
       }
     }
   }
@@ -571,10 +575,7 @@ __global__ __launch_bounds__(GAW * 64) void k_g_attn(GArgs A, int li) {
 #pragma unroll
     for (int i = 0; i < GAK / 4; ++i) {
       const float p = expf(sc[i] - ref);
-      // a position past the new one has weight 0 and a value of 0: 0 times the
-      // row loaded in its place is NaN where that row holds an infinity
-      const int key = k0 + 4 * i + grp;
-      const float4 v = key < pos ? row(vr[i]) : key == pos ? vl : make_float4(0.f, 0.f, 0.f, 0.f);
+      const float4 v = k0 + 4 * i + grp == pos ? vl : row(vr[i]);
       sum += p;
       o.x = __builtin_fmaf(p, v.x, o.x);
       o.y = __builtin_fmaf(p, v.y, o.y);
