@@ -215,18 +215,25 @@ __global__ __launch_bounds__(64 * GPW) void k_gp_gemm(GpArgs A, GpGemm G) {
       gp_half<NP>(ring[i].x, ring[i].w[1], h1, l1);
       if (h + i + RD < he) ring[i] = load(h + i + RD);
     }
+  // an infinity or NaN among the operands is in hi as it is, in lo as NaN
+  float big = 0.f;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) big = __builtin_elementwise_maximum(__builtin_elementwise_maximum(big, fabsf(l0[v])), fabsf(l1[v]));
+  if (__any(!(big < INFINITY))) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      l0[v] = fabsf(h0[v]) < INFINITY ? l0[v] : 0.f;
+      l1[v] = fabsf(h1[v]) < INFINITY ? l1[v] : 0.f;
+    }
+  }
   // value v of lane (j, hh): token j, row 8 (v / 4) + 4 hh + v % 4
   float *mine = buf + ks * GPT + j * 68 + 4 * hh;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
-    float y[8];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      y[e] = plane_sum(h0[4 * q + e], l0[4 * q + e]);
-      y[4 + e] = plane_sum(h1[4 * q + e], l1[4 * q + e]);
-    }
-    *reinterpret_cast<float4 *>(mine + 8 * q) = make_float4(y[0], y[1], y[2], y[3]);
-    *reinterpret_cast<float4 *>(mine + 32 + 8 * q) = make_float4(y[4], y[5], y[6], y[7]);
+    *reinterpret_cast<float4 *>(mine + 8 * q) = make_float4(h0[4 * q] + l0[4 * q], h0[4 * q + 1] + l0[4 * q + 1],
+                                                            h0[4 * q + 2] + l0[4 * q + 2], h0[4 * q + 3] + l0[4 * q + 3]);
+    *reinterpret_cast<float4 *>(mine + 32 + 8 * q) = make_float4(h1[4 * q] + l1[4 * q], h1[4 * q + 1] + l1[4 * q + 1],
+                                                                 h1[4 * q + 2] + l1[4 * q + 2], h1[4 * q + 3] + l1[4 * q + 3]);
   }
   __syncthreads();
   if (KS > 1) {

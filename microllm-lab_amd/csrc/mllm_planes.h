@@ -29,13 +29,10 @@ typedef float v2fl __attribute__((ext_vector_type(2)));
 // plane of a finite value is taken from the value cut to bf16's largest, so that
 // one past it keeps finite planes.  An infinity or NaN is itself in the first
 // plane and NaN in the others: a sum of first-plane products that is not finite
-// is the result, without the other planes' products (plane_sum).
+// is the result, without the other planes' products.
 __device__ __forceinline__ float bf16_cut(float v) {
   constexpr float M = 3.3895313892515355e38f;
   return fabsf(v) < INFINITY ? __builtin_amdgcn_fmed3f(v, -M, M) : v;
-}
-__device__ __forceinline__ float plane_sum(float first, float rest) {
-  return fabsf(first) < INFINITY ? first + rest : first;
 }
 __device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2fl){a, b}, v2bf));  // nearest even
