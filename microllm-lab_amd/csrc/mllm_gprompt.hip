@@ -422,8 +422,10 @@ __global__ __launch_bounds__(WG) void k_gp_ln(GpArgs A, const float *g, int t0, 
 // 72 us a launch (64 TFLOP/s over the unmasked half): 116 with a clamp and a
 // 64-bit address per load, instead of resources that end after the last row, and
 // the heads of a tile apart in the grid.  The f16-pair kernel, whose units have
-// sixteen times the rate: prompts of 200 tokens 1.83 ms (now 1.67), 1000 3.85
-// (3.19), 2000 6.42 (5.61); with an f16 cache 1.69 (1.68) and 2000 4.82 (5.68).
+// sixteen times the rate, took 16.0 us at 200 tokens (now 9.4), at 28 and 77 of
+// 11 heads with an f16 cache 7.1 and 7.3 (6.4 and 6.8), at 196 of 7 heads with an
+// f16 cache 9.4 (10.1); prompts of 1000 tokens 3.85 ms (3.18), 2000 6.41 (5.55)
+// and with an f16 cache 4.81 (5.66).
 constexpr int GAS = 8;
 
 // Cache elements as loaded, four components of a key (k) and one of a value
@@ -468,11 +470,13 @@ __device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
 // weigh 0; with the maximum itself they would weigh exp(-inf + inf) = NaN).
 __device__ __forceinline__ float score_ref(float mx) { return mx == -INFINITY ? 0.f : mx; }
 
-template <bool F16>
+// ND: halves of the output's 64 dimensions that a workgroup forms (blockIdx.z:
+// which, if one).
+template <bool F16, int ND>
 __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, int pos0, int tt0) {
   extern __shared__ __attribute__((aligned(16))) float buf[];  // [GAS][GPT] outputs, [GAS][2][32] (max, sum)
   const int T0 = (tt0 + (int)(gridDim.y - 1 - blockIdx.y)) * 32;  // the longest tiles first
-  const int hq = blockIdx.x, kvh = hq / (A.NH / A.NKV);
+  const int hq = blockIdx.x, kvh = hq / (A.NH / A.NKV), d0 = ND == 1 ? 32 * (int)blockIdx.z : 0;
   const int wv = __builtin_amdgcn_readfirstlane(tid() >> 6), lane = tid() & 63, j = lane & 31, hh = lane >> 5;
   const int qpos = pos0 + T0 + j, qlast = pos0 + min(T0 + 32, n) - 1;  // last key any query of the tile sees
   const int nb = (qlast >> 5) + 1, used = min(nb, GAS);
@@ -485,19 +489,18 @@ __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, i
       __builtin_amdgcn_make_buffer_rsrc(kp + A.NKV * hb, (short)0, (qlast + 1) * ROW, 0x00020000);
   float4 q[8];
   typename KvRaw<F16>::K kr[8];
-  typename KvRaw<F16>::V vr[2][16];
+  typename KvRaw<F16>::V vr[ND][16];
   auto load_k = [&](int b) {
     const int at = (32 * b + j) * ROW + 4 * hh * ES;
 #pragma unroll
     for (int c = 0; c < 8; ++c) kr[c] = KvRaw<F16>::k(kres, at + 8 * c * ES);
   };
   auto load_v = [&](int b) {
-    const int at = (32 * b + 4 * hh) * ROW + j * ES;
+    const int at = (32 * b + 4 * hh) * ROW + (d0 + j) * ES;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      vr[0][v] = KvRaw<F16>::v(vres, at + (8 * (v >> 2) + (v & 3)) * ROW);
-      vr[1][v] = KvRaw<F16>::v(vres, at + (8 * (v >> 2) + (v & 3)) * ROW + 32 * ES);
-    }
+    for (int v = 0; v < 16; ++v)
+#pragma unroll
+      for (int d = 0; d < ND; ++d) vr[d][v] = KvRaw<F16>::v(vres, at + (8 * (v >> 2) + (v & 3)) * ROW + 32 * d * ES);
   };
   {
     const float *qr = A.q + (size_t)min(T0 + j, n - 1) * A.D + hq * GPHD + 4 * hh;
@@ -509,9 +512,11 @@ __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, i
     load_v(wv);
   }
   float m = -INFINITY, l = 0.f;
-  v16f o[2];
+  v16f o[ND];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) o[0][v] = o[1][v] = 0.f;
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[d][v] = 0.f;
   for (int b = wv; b < nb; b += GAS) {
     v16f s;
 #pragma unroll
@@ -544,45 +549,42 @@ __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, i
     l = l * alpha + (ps + __shfl_xor(ps, 32));
     if (__any(mx != m)) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        o[0][v] *= alpha;
-        o[1][v] *= alpha;
-      }
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
     }
     m = mx;
     bool whole = true;
     if (masked) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) whole &= finite(KvRaw<F16>::f(vr[0][v])) && finite(KvRaw<F16>::f(vr[1][v]));
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) whole &= finite(KvRaw<F16>::f(vr[d][v]));
     }
     if (__all(whole)) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        o[0] = mfma_f32(KvRaw<F16>::f(vr[0][v]), s[v], o[0]);
-        o[1] = mfma_f32(KvRaw<F16>::f(vr[1][v]), s[v], o[1]);
-      }
+      for (int v = 0; v < 16; ++v)
+#pragma unroll
+        for (int d = 0; d < ND; ++d) o[d] = mfma_f32(KvRaw<F16>::f(vr[d][v]), s[v], o[d]);
     } else {
       // An infinity or NaN among the values of a block with masked keys: their
       // weight is 0 and 0 times it NaN, in the rows of queries that do not see
       // it.  It is left out of the products, and counted for the queries that
       // do: those are NaN.
-      for (int d = 0; d < 2; ++d) {
-        v16f hit, sum = o[d];
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        v16f hit;
 #pragma unroll
         for (int v = 0; v < 16; ++v) hit[v] = 0.f;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          const float val = KvRaw<F16>::f(d == 0 ? vr[0][v] : vr[1][v]);
+          const float val = KvRaw<F16>::f(vr[d][v]);
           const bool sees = 32 * b + 8 * (v >> 2) + 4 * hh + (v & 3) <= qpos;
-          sum = mfma_f32(finite(val) ? val : 0.f, s[v], sum);
+          o[d] = mfma_f32(finite(val) ? val : 0.f, s[v], o[d]);
           hit = mfma_f32(finite(val) ? 0.f : 1.f, sees ? 1.f : 0.f, hit);
         }
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const float r = hit[v] > 0.f ? NAN : sum[v];
-          if (d == 0) o[0][v] = r;
-          else o[1][v] = r;
-        }
+        for (int v = 0; v < 16; ++v) o[d][v] = hit[v] > 0.f ? NAN : o[d][v];
       }
     }
     if (b + GAS < nb) load_v(b + GAS);
@@ -592,7 +594,7 @@ __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, i
   if (wv < used) {
     float *mine = buf + wv * GPT + j * 68 + 4 * hh;
 #pragma unroll
-    for (int d = 0; d < 2; ++d)
+    for (int d = 0; d < ND; ++d)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         *reinterpret_cast<float4 *>(mine + 32 * d + 8 * g) =
@@ -600,8 +602,8 @@ __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, i
     ml[wv * 64 + 32 * hh + j] = hh ? l : m;
   }
   __syncthreads();
-  const int jt = tid() >> 4, c = tid() & 15;
-  if (T0 + jt >= n) return;
+  const int jt = (int)tid() / (8 * ND), c = (int)tid() % (8 * ND);
+  if (jt >= 32 || T0 + jt >= n) return;
   float M = -INFINITY;
   for (int w = 0; w < used; ++w) M = fmaxf(M, ml[w * 64 + jt]);
   M = score_ref(M);
@@ -615,7 +617,7 @@ __global__ __launch_bounds__(64 * GAS) void k_gp_attn(GpArgs A, int li, int n, i
   }
 #pragma unroll
   for (int e = 0; e < 4; ++e) r[e] = r[e] / L;
-  planes_store4(A.pxo + ((size_t)(T0 >> 5) * (A.D >> 5) + 2 * hq) * BPX, jt, c, r);
+  planes_store4(A.pxo + ((size_t)(T0 >> 5) * (A.D >> 5) + 2 * hq) * BPX, jt, (d0 >> 2) + c, r);
 }
 
 // Thread = one lane's 16 bytes of every plane: eight columns of one row.
@@ -646,6 +648,13 @@ const GpKernel kGpKernels[4][3] = {
     {k_gp_gemm<GP_SWIGLU, 1>, k_gp_gemm<GP_SWIGLU, 2>, k_gp_gemm<GP_SWIGLU, 3>},
     {k_gp_gemm<GP_GELU, 1>, k_gp_gemm<GP_GELU, 2>, k_gp_gemm<GP_GELU, 3>},
 };
+void (*const kGpAttn[2][2])(GpArgs, int, int, int, int) = {{k_gp_attn<false, 1>, k_gp_attn<false, 2>},
+                                                           {k_gp_attn<true, 1>, k_gp_attn<true, 2>}};
+// Workgroups (32-token tiles times heads) up to which the output's halves are
+// apart: while both fit the 256 CUs, a block's 64 MFMAs become 48 for each (the
+// scores are formed twice).  9 heads, 200 tokens: 10.9 -> 9.4 us a launch; 7
+// heads, 196 tokens 11.5 -> 10.1.
+constexpr int kAttnHalves = 128;
 size_t gp_lds(int ks) { return sizeof(float) * ((size_t)ks * GPT + 32); }
 
 // Column slices per tile: doubled while the launch has fewer than 1024 waves
@@ -736,8 +745,9 @@ int gp_init() {
     for (GpKernel k : row)
       MLLM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)gp_lds(GPW)));
-  for (const void *k : {reinterpret_cast<const void *>(k_gp_attn<false>), reinterpret_cast<const void *>(k_gp_attn<true>)})
-    MLLM_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kAttnLds));
+  for (const auto &row : kGpAttn)
+    for (const auto k : row)
+      MLLM_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kAttnLds));
   return 0;
 }
 
@@ -764,8 +774,9 @@ int gp_layers(const GpArgs &A, const int32_t *ids, int n, int pos0, bool last, c
     if (final_layer && !last) break;
     // the prompt's last token needs its own tile of the last layer only
     const int tt0 = final_layer ? ntt - 1 : 0;
-    hipLaunchKernelGGL(A.kv_fp16 ? k_gp_attn<true> : k_gp_attn<false>, dim3(A.NH, ntt - tt0), dim3(64 * GAS), kAttnLds, s,
-                       A, li, n, pos0, tt0);
+    const int nd = A.NH * (ntt - tt0) <= kAttnHalves ? 1 : 2;
+    hipLaunchKernelGGL(kGpAttn[A.kv_fp16 ? 1 : 0][nd - 1], dim3(A.NH, ntt - tt0, 2 / nd), dim3(64 * GAS), kAttnLds, s, A, li,
+                       n, pos0, tt0);
     GpGemm O = gemm_of(W.proj, n, tt0, A.pxo);
     O.bias = gpt2 ? W.proj_b : nullptr;
     O.gain = gpt2 ? nullptr : W.n2;

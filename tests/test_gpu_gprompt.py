@@ -74,6 +74,17 @@ def test_tile_placement_vs_oracle(oracle_lib, n):
 
 
 @gpu
+@pytest.mark.parametrize("kv_fp16", [False, True])
+@pytest.mark.parametrize("n", [33, 448, 449])
+def test_attention_halves_vs_oracle(oracle_lib, n, kv_fp16):
+    """Nine heads: 18, 126 and 135 (tile, head) workgroups, the output's halves
+    apart up to 128; up to 15 key blocks on eight waves."""
+    bundle = build(seed=49, kind="bf16", n_layers=1, d_model=576, n_heads=9, n_kv_heads=3, max_seq_len=512)
+    print(f"halves n={n} fp16={kv_fp16}", flush=True)
+    assert worst(oracle_lib, bundle, n, kv_fp16) <= (TOL_F16KV if kv_fp16 else TOL)
+
+
+@gpu
 @pytest.mark.parametrize("n", [2048, 2049, 2085])
 def test_chunk_boundary_vs_oracle(oracle_lib, n):
     """More tokens than a chunk holds: the second chunk reads the first's keys."""
