@@ -300,6 +300,12 @@ __device__ __forceinline__ float wave_max(float v) {
   return fmaxf(fmaxf(readlane_f(v, 0), readlane_f(v, 16)), fmaxf(readlane_f(v, 32), readlane_f(v, 48)));
 }
 
+// What a part of the keys subtracts from its scores: their maximum, or 0 where
+// all of them are -inf, so that these keys weigh exp(-inf) = 0 and not
+// exp(-inf + inf) = NaN.  (All keys of a row so: 0 / 0 at the end, as
+// infer.js:227-238 gives it.)
+__device__ __forceinline__ float score_ref(float mx) { return mx == -INFINITY ? 0.f : mx; }
+
 // Four floats at any 4-byte boundary (the f32 tensors of a payload).
 typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 ld4u(const float *p) {

@@ -67,9 +67,9 @@ __device__ __forceinline__ bool stopped(const GCursor *c) {
 // on its way at once.  These launches are bound by that one latency (a layer's
 // matrices are 0.2 to 3 MB), where the former form (inputs staged in LDS, two
 // to three block reductions, then the weights) paid it two to three times:
-// per-row Q8 at the 135M shape, us a launch, QKV 5.1 -> 4.4, O 5.1 -> 4.1 (it
-// merges the attention's splits, too), gate/up 6.3 -> 4.7, down 5.1 -> 3.4,
-// lm_head 21 -> 12.5.
+// per-row Q8 at the 135M shape, us a launch, QKV 5.1 -> 4.2, O 5.1 -> 4.1 (it
+// merges the attention's splits, too), gate/up 6.3 -> 4.9, down 5.1 -> 3.8,
+// lm_head 21 -> 12.3.
 constexpr int G_MIXED = -1;  // W and W3 of different storages
 template <int KIND>
 __host__ __device__ constexpr int g_cb() {
@@ -145,12 +145,6 @@ struct GemvArgs {
   int nsplit_max;      // GN_SPLITS: partials per head in x
   int m, xs;           // tokens of the pass and the stride of their inputs (outputs: W.rows)
 };
-
-// What a part of the keys subtracts from its scores: their maximum, or 0 where
-// all of them are -inf, so that these keys weigh exp(-inf) = 0 and not
-// exp(-inf + inf) = NaN.  (All keys of a row so: 0 / 0 at the end, as
-// infer.js:227-238 gives it.)
-__device__ __forceinline__ float score_ref(float mx) { return mx == -INFINITY ? 0.f : mx; }
 
 // The attention's output row from its splits' partials (infer.js:466-495) into
 // LDS: a thread per four components, its splits' loads four at a time.
@@ -483,7 +477,7 @@ __device__ __forceinline__ float rope_at(const GArgs &A, const float *hd, int d,
 // attp, and the O GEMV merges the splits while it reads its input.  The
 // former form -- a workgroup per head, a row per thread, then P.V down four
 // position slices -- was bound by one workgroup's load rate: 32.2 us at 700
-// positions of the 135M shape, 7.6 now (8.3 with 64 positions a wave: twice
+// positions of the 135M shape, 7.2 now (8.3 with 64 positions a wave: twice
 // the code, which runs once from a cold instruction cache).
 // The new position's k and v are taken from LDS (as the cache holds them:
 // f16-rounded for an f16 cache), so a group's heads do not wait for the one

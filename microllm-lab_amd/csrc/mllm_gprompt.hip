@@ -466,9 +466,6 @@ __device__ __forceinline__ v16f mfma_f32(float a, float b, v16f c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 __device__ __forceinline__ bool finite(float v) { return fabsf(v) < INFINITY; }
-// What a part of the keys subtracts from its scores: 0 where all are -inf (they
-// weigh 0; with the maximum itself they would weigh exp(-inf + inf) = NaN).
-__device__ __forceinline__ float score_ref(float mx) { return mx == -INFINITY ? 0.f : mx; }
 
 // ND: halves of the output's 64 dimensions that a workgroup forms (blockIdx.z:
 // which, if one).

@@ -617,9 +617,10 @@ __global__ __launch_bounds__(gemm_threads(KS)) void k_pf_gemm(PfArgs A, PfGemm G
 // so every lane holds one query's scores and output column, and the online
 // softmax (running max and sum, per-block rescaling) needs one exchange with
 // the lane 32 apart.  f32 accuracy from f16 operands: the scaled query and
-// the weights are split as hi + lo halves (v = hi + lo to ~2^-22), and so are
-// f32 keys and values (an f16 cache is exact as is); the dropped lo x lo
-// terms are below 2^-40 relative.  The scores are formed in the log2 domain
+// the weights are split as hi + lo halves (v = hi + lo to 2^-22 of it where lo is
+// a normal f16, |v| of about 1/8 and more, below that to 2^-25; past 65504 hi is
+// infinite), and so are f32 keys and values (an f16 cache is exact as is); the
+// dropped lo x lo terms are below 2^-22 of the product.  The scores are formed in the log2 domain
 // (the query scaled by attn_scale * log2 e) for v_exp_f32.
 constexpr int QTL = 32;   // queries per wave
 constexpr int KROW = 72;  // halves per staged key row (64 + pad)
